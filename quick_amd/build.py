@@ -2,8 +2,8 @@
 
     python -m quick_amd.build        (or __graft_entry__.build())
 
-Steps: regenerate the per-class VRR/HRR device code (csrc/gen_eri.py) and the
-gradient tables (csrc/gen_grad.py), compile every translation unit with hipcc
+Steps: regenerate the per-class VRR/HRR device code (csrc/gen_eri.py), the
+gradient tables (csrc/gen_grad.py) and its straight-line code (csrc/gen_gradw.py), compile every translation unit with hipcc
 (in parallel, into _build/), and link the shared library next to this file.
 """
 from __future__ import annotations
@@ -37,7 +37,7 @@ OBJ = HERE / "_build"
 def _compile(src: Path, verbose: bool) -> Path:
     obj = OBJ / (src.stem + ".o")
     deps = [src, CSRC / "qk_kernels.h", CSRC / "qk_internal.h", CSRC / "eri_generated.inc",
-            CSRC / "qk_team.h", CSRC / "team_tables.inc", CSRC / "grad_tables.inc", CSRC / "grad_light.inc",
+            CSRC / "qk_team.h", CSRC / "team_tables.inc", CSRC / "grad_tables.inc", CSRC / "grad_fold.inc",
             CSRC / "qk_grad_light.h", CSRC / "xc_b3lyp.inc", CSRC / "lebedev.inc",
             HERE.parent / "include" / "quick_mi355x.h", Path(__file__)]
     if obj.exists() and all(obj.stat().st_mtime >= d.stat().st_mtime for d in deps if d.exists()):
@@ -56,6 +56,8 @@ def build(verbose: bool = True, jobs: int = 8) -> Path:
     subprocess.run([sys.executable, str(CSRC / "gen_eri.py"), str(CSRC / "eri_generated.inc"),
                     str(CSRC / "gen")], check=True, stdout=subprocess.DEVNULL)
     subprocess.run([sys.executable, str(CSRC / "gen_grad.py"), str(CSRC / "grad_tables.inc")], check=True,
+                   stdout=subprocess.DEVNULL)
+    subprocess.run([sys.executable, str(CSRC / "gen_gradw.py"), str(CSRC / "grad_fold.inc")], check=True,
                    stdout=subprocess.DEVNULL)
     subprocess.run([sys.executable, str(CSRC / "gen_xc.py"), str(CSRC / "xc_b3lyp.inc"), str(CSRC / "lebedev.inc")],
                    check=True, stdout=subprocess.DEVNULL)

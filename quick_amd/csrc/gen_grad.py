@@ -258,7 +258,9 @@ def write(path):
 
 
 # ---------------------------------------------------------------------------
-# Straight-line gradient code for the light classes (one quartet per lane):
+# Straight-line gradient code from the same four contracted sets, for the light
+# classes: a second form of the table programs, which the tests hold against
+# them (the device runs the density-folded form of gen_gradw.py):
 #   vrg_<tag>: the raised VRR, accumulating the four contracted sets
 #              (acc0, accA, accB, accC with weights 1, wA, wB, wC);
 #   gcon_<tag>: the six derivative terms' bra/ket HRR and their contraction
@@ -518,32 +520,9 @@ def write_light(path):
         open(path, "w").write(new)
 
 
-def write_light_units(outdir):
-    """One translation unit per light gradient class."""
-    os.makedirs(outdir, exist_ok=True)
-    for cls in LIGHT_CLASSES:
-        t = tag(cls)
-        body = ["// Generated by quick_amd/csrc/gen_grad.py -- do not edit.", '#include "../qk_grad_light.h"',
-                "namespace qk {",
-                f"void launch_grad_light_{t}(const GradArgs& a, const ClassWork& w, int grid, size_t lds, hipStream_t s) {{",
-                f"    static const long long cap = scratch_grid_cap(kernel_scratch(reinterpret_cast<const void*>(&grad_light_kernel<{cls[0]}, {cls[1]}, {cls[2]}, {cls[3]}, double>)), 4);",
-                f"    hipLaunchKernelGGL((grad_light_kernel<{cls[0]}, {cls[1]}, {cls[2]}, {cls[3]}, double>), dim3((int)std::min<long long>(grid, cap)), dim3(256), lds, s, a, w);",
-                "}",
-                f"void launch_grad_light_f32_{t}(const GradArgs& a, const ClassWork& w, int grid, size_t lds, hipStream_t s) {{",
-                f"    static const long long cap = scratch_grid_cap(kernel_scratch(reinterpret_cast<const void*>(&grad_light_kernel<{cls[0]}, {cls[1]}, {cls[2]}, {cls[3]}, float>)), 4);",
-                f"    hipLaunchKernelGGL((grad_light_kernel<{cls[0]}, {cls[1]}, {cls[2]}, {cls[3]}, float>), dim3((int)std::min<long long>(grid, cap)), dim3(256), lds, s, a, w);",
-                "}", "}  // namespace qk"]
-        fn = os.path.join(outdir, f"grad_{t}.hip")
-        new = "\n".join(body) + "\n"
-        if not os.path.exists(fn) or open(fn).read() != new:
-            open(fn, "w").write(new)
-
-
 if __name__ == "__main__":
     if len(sys.argv) > 1:
         write(sys.argv[1])
-        write_light(os.path.join(os.path.dirname(sys.argv[1]), "grad_light.inc"))
-        write_light_units(os.path.join(os.path.dirname(sys.argv[1]), "gen"))
     else:
         for cls in quartet_classes():
             _, info = class_blob(cls)

@@ -64,18 +64,16 @@ __device__ __forceinline__ void gx_add(unsigned long long* G, long long idx, dou
     if (iv != 0) atomicAdd(G + idx, (unsigned long long)iv);
 }
 
-// kGradTeam threads (one or four wavefronts) work on one quartet.  R = double:
-// QUICK's Boys fit; R = float (mixed precision, weak quartets): the tabulated
-// FP32 Boys expansion, FP32 LDS buffers and arithmetic, the nine sums promoted
-// to FP64 before the wavefront reduction.
-// At least three wavefronts per SIMD in FP64, five in FP32: the FP64 form then
-// fits 168 VGPRs (76 bytes of spills) instead of 205 at two, the FP32 form 96
-// (no spills) instead of 100 at four.  Measured on (H2O)32: FP64 gradient
-// 174.5 -> 172.4 ms (dpdp 14.3 -> 11.0 ms); the mixed gradient's FP32 classes
-// gain 0.3-0.9 ms each at five (dpdp 6.7 -> 5.7 ms), except dppp (16.0 ms at
-// five), which runs a form built for four (kMinWaves 4).
-template <int kGradTeam, typename R, int kMinWaves = (sizeof(R) == 4 ? 5 : 3)>
-__global__ void __launch_bounds__(kGradTeam, kMinWaves) grad_kernel(const GradArgs a, const ClassWork w, const int* __restrict__ tab) {
+// kGradTeam threads work on one quartet: (dd|dd) alone, whose straight-line
+// code (45,600 operations a primitive quartet) no lane could hold; every other
+// class runs one quartet per lane (qk_grad_light.h).  R = double: QUICK's Boys
+// fit; R = float (mixed precision, weak quartets): the tabulated FP32 Boys
+// expansion, FP32 LDS buffers and arithmetic, the nine sums promoted to FP64
+// before the wavefront reduction.  At least three wavefronts per SIMD in FP64
+// (168 VGPRs), five in FP32 (96 VGPRs, no spills).
+constexpr int kGradTeam = 256;
+template <typename R>
+__global__ void __launch_bounds__(kGradTeam, (sizeof(R) == 4 ? 5 : 3)) grad_kernel(const GradArgs a, const ClassWork w, const int* __restrict__ tab) {
     constexpr bool f64 = sizeof(R) == 8;
     extern __shared__ double lds[];
     const int lane = threadIdx.x;          // thread of the block (kGradTeam threads share one quartet)
@@ -364,11 +362,6 @@ __global__ void grad_finalize(const unsigned long long* __restrict__ G, double* 
     grad[k] += (double)s * 0x1p-44;
 }
 
-// four wavefronts per quartet for the classes with the largest node programs
-// (dpdp, dddp, dddd); measured on (H2O)32, ddds and ddpp run as fast or faster
-// with one (ddds FP64 9.4 -> 7.5 ms) and dppp-sized classes twice as fast
-static int grad_team_of(const int* hdr) { return hdr[kGhSlots] >= 1800 ? 256 : 64; }
-
 // dynamic LDS of grad_kernel: the FP64 partial sums (9 x 4), then the VRR /
 // stage buffers, sets, density factors, powers, Boys values and the VRR factors in the
 // kernel's precision
@@ -378,50 +371,47 @@ size_t grad_lds_bytes(const int* hdr, bool fp32) {
     return sizeof(double) * 36 + (fp32 ? sizeof(float) : sizeof(double)) * (size_t)(RV + nS + hdr[kGhNOut] + 128 + 16 + 16);
 }
 
-template <int TEAM, typename R, int W = (sizeof(R) == 4 ? 5 : 3)>
+template <typename R>
 static int launch_team(const GradArgs& a, const ClassWork& w, const int* dtab, size_t lds, int grid, hipStream_t s) {
     if (lds > 64 * 1024 &&
-        hipFuncSetAttribute(reinterpret_cast<const void*>(&grad_kernel<TEAM, R, W>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
+        hipFuncSetAttribute(reinterpret_cast<const void*>(&grad_kernel<R>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                            (int)lds) != hipSuccess)
         return -1;
     static const long long cap =
-        scratch_grid_cap(kernel_scratch(reinterpret_cast<const void*>(&grad_kernel<TEAM, R, W>)), TEAM / 64);
-    hipLaunchKernelGGL((grad_kernel<TEAM, R, W>), dim3((int)std::min<long long>(grid, cap)), dim3(TEAM), lds, s, a, w,
-                       dtab);
+        scratch_grid_cap(kernel_scratch(reinterpret_cast<const void*>(&grad_kernel<R>)), kGradTeam / 64);
+    hipLaunchKernelGGL((grad_kernel<R>), dim3((int)std::min<long long>(grid, cap)), dim3(kGradTeam), lds, s, a, w, dtab);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-// hdr: the class's table header (host copy); dtab: the same table on the device
-// four_waves (FP32, one-wavefront teams): the form built for four wavefronts
-// per SIMD (100 VGPRs) instead of five (96), for a class that runs slower at five
-int launch_grad_class(const GradArgs& a, const ClassWork& w, const int* hdr, const int* dtab, size_t lds, int grid,
-                      bool fp32, bool four_waves, hipStream_t s) {
-    if (fp32 && four_waves && grad_team_of(hdr) == 64) return launch_team<64, float, 4>(a, w, dtab, lds, grid, s);
-    if (fp32)
-        return grad_team_of(hdr) == 256 ? launch_team<256, float>(a, w, dtab, lds, grid, s)
-                                        : launch_team<64, float>(a, w, dtab, lds, grid, s);
-    return grad_team_of(hdr) == 256 ? launch_team<256, double>(a, w, dtab, lds, grid, s)
-                                    : launch_team<64, double>(a, w, dtab, lds, grid, s);
+// dtab: the class's table on the device
+int launch_grad_class(const GradArgs& a, const ClassWork& w, const int* dtab, size_t lds, int grid, bool fp32,
+                      hipStream_t s) {
+    return fp32 ? launch_team<float>(a, w, dtab, lds, grid, s) : launch_team<double>(a, w, dtab, lds, grid, s);
 }
 
 #define QK_DECL(T)                                                                                 \
     void launch_grad_light_##T(const GradArgs&, const ClassWork&, int, size_t, hipStream_t);      \
     void launch_grad_light_f32_##T(const GradArgs&, const ClassWork&, int, size_t, hipStream_t);
 QK_DECL(ssss) QK_DECL(psss) QK_DECL(psps) QK_DECL(ppss) QK_DECL(dsss) QK_DECL(ppps) QK_DECL(dsps)
-QK_DECL(dpss) QK_DECL(pppp) QK_DECL(dspp) QK_DECL(dsds) QK_DECL(dpps) QK_DECL(ddss)
+QK_DECL(dpss) QK_DECL(pppp) QK_DECL(dspp) QK_DECL(dsds) QK_DECL(dpps) QK_DECL(ddss) QK_DECL(dppp)
+QK_DECL(dpds) QK_DECL(dpdp) QK_DECL(ddps) QK_DECL(ddpp) QK_DECL(ddds) QK_DECL(dddp)
 #undef QK_DECL
 using GradLightLauncher = void (*)(const GradArgs&, const ClassWork&, int, size_t, hipStream_t);
 // classes with a one-quartet-per-lane kernel (order of gen_eri.quartet_classes())
 static const GradLightLauncher kGradLight[kNumQuartetClasses] = {
     launch_grad_light_ssss, launch_grad_light_psss, launch_grad_light_psps, launch_grad_light_ppss,
     launch_grad_light_ppps, launch_grad_light_pppp, launch_grad_light_dsss, launch_grad_light_dsps,
-    launch_grad_light_dspp, launch_grad_light_dsds, launch_grad_light_dpss, launch_grad_light_dpps, nullptr, nullptr,
-    nullptr, launch_grad_light_ddss, nullptr, nullptr, nullptr, nullptr, nullptr};
+    launch_grad_light_dspp, launch_grad_light_dsds, launch_grad_light_dpss, launch_grad_light_dpps,
+    launch_grad_light_dppp, launch_grad_light_dpds, launch_grad_light_dpdp, launch_grad_light_ddss,
+    launch_grad_light_ddps, launch_grad_light_ddpp, launch_grad_light_ddds, launch_grad_light_dddp, nullptr};
 static const GradLightLauncher kGradLightF32[kNumQuartetClasses] = {
-    launch_grad_light_f32_ssss, launch_grad_light_f32_psss, launch_grad_light_f32_psps, launch_grad_light_f32_ppss,
-    launch_grad_light_f32_ppps, launch_grad_light_f32_pppp, launch_grad_light_f32_dsss, launch_grad_light_f32_dsps,
-    launch_grad_light_f32_dspp, launch_grad_light_f32_dsds, launch_grad_light_f32_dpss, launch_grad_light_f32_dpps,
-    nullptr, nullptr, nullptr, launch_grad_light_f32_ddss, nullptr, nullptr, nullptr, nullptr, nullptr};
+    launch_grad_light_f32_ssss, launch_grad_light_f32_psss, launch_grad_light_f32_psps,
+    launch_grad_light_f32_ppss, launch_grad_light_f32_ppps, launch_grad_light_f32_pppp,
+    launch_grad_light_f32_dsss, launch_grad_light_f32_dsps, launch_grad_light_f32_dspp,
+    launch_grad_light_f32_dsds, launch_grad_light_f32_dpss, launch_grad_light_f32_dpps,
+    launch_grad_light_f32_dppp, launch_grad_light_f32_dpds, launch_grad_light_f32_dpdp,
+    launch_grad_light_f32_ddss, launch_grad_light_f32_ddps, launch_grad_light_f32_ddpp,
+    launch_grad_light_f32_ddds, launch_grad_light_f32_dddp, nullptr};
 bool grad_class_is_light(int k) { return kGradLight[k] != nullptr; }
 int launch_grad_light(int k, const GradArgs& a, const ClassWork& w, int grid, bool fp32, hipStream_t s) {
     const size_t lds = a.lds_grad ? sizeof(unsigned long long) * 3 * (size_t)a.natom : 0;

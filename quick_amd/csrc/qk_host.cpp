@@ -35,8 +35,8 @@ void launch_team_class(int k, const FockArgs& a, const ClassWork& w, int grid, h
 void launch_team_f32_class(int k, const FockArgs& a, const ClassWork& w, int grid, hipStream_t s);
 void launch_scale_density(const double* D, const double* cons, double* Dp, float* Dpf, int n, hipStream_t s);
 size_t grad_lds_bytes(const int* hdr, bool fp32);
-int launch_grad_class(const GradArgs& a, const ClassWork& w, const int* hdr, const int* dtab, size_t lds, int grid,
-                      bool fp32, bool four_waves, hipStream_t s);
+int launch_grad_class(const GradArgs& a, const ClassWork& w, const int* dtab, size_t lds, int grid, bool fp32,
+                      hipStream_t s);
 void launch_grad_finalize(const unsigned long long* G, double* grad, int m, unsigned long long* flag, hipStream_t s);
 bool grad_class_is_light(int k);
 int launch_grad_light(int k, const GradArgs& a, const ClassWork& w, int grid, bool fp32, hipStream_t s);
@@ -1510,15 +1510,15 @@ static int grad_prepare(qk_ctx* c, const qk_opts* o) {
         return 0;
     (void)hipSetDevice(c->device);
     for (int k = 0; k < kNumQuartetClasses; ++k)
-        if (!c->d_gtab[k].p) {
+        if (!grad_class_is_light(k) && !c->d_gtab[k].p) {
             std::vector<int> blob(kGradBlobs[k], kGradBlobs[k] + kGradBlobLen[k]);
             if (c->d_gtab[k].upload(blob)) return -1;
         }
     // the work lists on the device: (bra group, ket group, bra) order, so that
     // neighbouring wavefronts read the same kets (measured faster than
     // bra-major order for the gradient); light classes one quartet per lane in
-    // tiles of up to 64 kets, the table-driven kernel one quartet at a time per
-    // wavefront in tiles of 16, 4 or 1
+    // tiles of up to 64 kets, the table-driven kernel ((dd|dd)) one quartet per
+    // block
     std::vector<ListEntry> E;
     std::vector<KetGroup> KG;
     std::vector<ListClass> LC(kNumQuartetClasses);
@@ -1529,9 +1529,8 @@ static int grad_prepare(qk_ctx* c, const qk_opts* o) {
         cls_item[k] = nitem;
         const int cb = pair_class_of(kClassL[k][0], kClassL[k][1]);
         const int ck = pair_class_of(kClassL[k][2], kClassL[k][3]);
-        const int LT = kClassL[k][0] + kClassL[k][1] + kClassL[k][2] + kClassL[k][3];
         const bool light = grad_class_is_light(k);
-        const int chunk = light ? 64 : (LT <= 3 ? 16 : (LT <= 5 ? 4 : 1));
+        const int chunk = light ? 64 : 1;
         LC[k] = ListClass{chunk, INT_MAX, INT_MAX, mixed ? 1 : 0, light ? 1 : 0, 1, 0, 0};
         for (size_t gb = 0; gb < ng; ++gb) {
             if (c->grp_cls[gb] != cb) continue;
@@ -1730,13 +1729,8 @@ static int grad_enqueue(qk_ctx* c, const double* dD, const double* dcutmat_or_nu
                 }
             } else {
                 const size_t lds = grad_lds_bytes(kGradBlobs[k], fp32);
-                // at most 16 blocks per CU (with one-wavefront blocks: four
-                // wavefronts per SIMD), 20 for the FP32 form (five), except for
-                // dppp, measured slower at five (12.4 ms at four, 16.0 at five on
-                // (H2O)32): it runs the FP32 form built for four
-                const bool dppp = kClassL[k][0] == 2 && kClassL[k][1] == 1 && kClassL[k][2] == 1 && kClassL[k][3] == 1;
-                const int grid = (int)std::min<long long>(nt, 256LL * (fp32 && !dppp ? 20 : 16));
-                if (launch_grad_class(a, w, kGradBlobs[k], c->d_gtab[k].p, lds, grid, fp32, dppp, ls)) {
+                const int grid = (int)std::min<long long>(nt, 256LL * (fp32 ? 20 : 16));
+                if (launch_grad_class(a, w, c->d_gtab[k].p, lds, grid, fp32, ls)) {
                     set_err("gradient kernel launch failed for class %d (%zu bytes LDS)", k, lds);
                     return -1;
                 }
