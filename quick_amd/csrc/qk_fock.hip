@@ -21,6 +21,7 @@
 // classes use the wavefront-cooperative kernel (qk_team.h) instead.
 #include "qk_kernels.h"
 
+#include <atomic>
 #include <mutex>
 
 namespace qk {
@@ -31,16 +32,14 @@ namespace qk {
 // Density screen of the candidate quartets, compacted: one wavefront per
 // segment (a bra pair and a ket range of one group) tests its candidate kets
 // 64 at a time and appends the survivors in order (ballot + prefix count) at
-// list[segs[s].w ...]; counts[s] gets their number.  The class kernels then
-// fill all 64 lanes with surviving quartets.  The test is the class kernels'
-// own, same operation order: Fock Y_p Y_q DNmax > tau; gradient (one-centre
-// quartets skipped) Y_p Y_q > tau and Y_p Y_q DNmax > tau.  With a.steps set,
-// the survivors are also cut into steps of 64, written to the slots of the
-// segment's tiles (same order as the tiles; the gradient's light kernels
-// stride over them).
+// list[segs[s].w ...].  The class kernels then fill their lanes with surviving
+// quartets.  The test is the class kernels' own, same operation order: Fock
+// Y_p Y_q DNmax > tau; gradient (one-centre quartets skipped) Y_p Y_q > tau and
+// Y_p Y_q DNmax > tau.  The survivors are cut into steps of a.chunk, written to
+// the slots of the segment's tiles (same order as the tiles; the class kernels
+// take them in the tiles' place).
 __global__ void __launch_bounds__(256) compact_kernel(const CompactArgs a, const int4* __restrict__ segs,
-                                                      long long nsegs, int* __restrict__ list, int* __restrict__ counts,
-                                                      int stage_rows) {
+                                                      long long nsegs, int* __restrict__ list, int stage_rows) {
     extern __shared__ double s_cmrows[];
     const long long s = ((long long)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
     const int lane = threadIdx.x & 63;
@@ -92,13 +91,10 @@ __global__ void __launch_bounds__(256) compact_kernel(const CompactArgs a, const
         if (keep) list[sg.w + cnt + __popcll(bal & ((1ull << lane) - 1ull))] = q;
         cnt += __popcll(bal);
     }
-    if (lane == 0) counts[s] = cnt;
-    if (a.steps != nullptr) {
-        // this segment's slots: its steps of 64 survivors, then empty ones
-        const int nslot = (sg.z - sg.y + 63) >> 6, base = a.slot0[s];
-        for (int j = lane; j < nslot; j += 64)
-            a.steps[base + j] = Tile{sg.x, sg.w + 64 * j, max(0, min(64, cnt - 64 * j)), 0};
-    }
+    // this segment's slots: its steps of `chunk` survivors, then empty ones
+    const int ch = a.chunk, nslot = (sg.z - sg.y + ch - 1) / ch, base = a.slot0[s], st = a.pstride[sg.y];
+    for (int j = lane; j < nslot; j += 64)
+        a.steps[base + j] = Tile{sg.x, sg.w + ch * j, max(0, min(ch, cnt - ch * j)), st};
 }
 
 // Dp = diag(cons) D diag(cons): folds QUICK's per-function cons factors
@@ -172,19 +168,14 @@ __global__ void jpair_scatter(const unsigned long long* __restrict__ J, const in
 // ---------------------------------------------------------------------------
 // launchers
 
-using FockLauncher = void (*)(const FockArgs&, const ClassWork&, int, size_t, hipStream_t);
 using TeamLauncher = void (*)(const FockArgs&, const ClassWork&, int, hipStream_t);
 using SchwarzLauncher = void (*)(const int*, int, const int*, const int*, const int*, const int*, const DevQshells&,
                                  const DevPrims&, const double*, const double*, double*, double*, hipStream_t);
-#define QK_DECL(T) void launch_fock_##T(const FockArgs&, const ClassWork&, int, size_t, hipStream_t);
-QK_DECL(ssss) QK_DECL(psss) QK_DECL(psps) QK_DECL(ppss) QK_DECL(ppps) QK_DECL(pppp) QK_DECL(dsss)
-QK_DECL(dsps) QK_DECL(dspp) QK_DECL(dsds) QK_DECL(dpss) QK_DECL(dpps) QK_DECL(dppp) QK_DECL(dpds)
-QK_DECL(dpdp) QK_DECL(ddss) QK_DECL(ddps) QK_DECL(ddpp) QK_DECL(ddds) QK_DECL(dddp) QK_DECL(dddd)
-#undef QK_DECL
-#define QK_DECL(T) size_t fock_scratch_##T();
-QK_DECL(ssss) QK_DECL(psss) QK_DECL(psps) QK_DECL(ppss) QK_DECL(ppps) QK_DECL(pppp) QK_DECL(dsss)
-QK_DECL(dsps) QK_DECL(dspp) QK_DECL(dsds) QK_DECL(dpss) QK_DECL(dpps) QK_DECL(dppp) QK_DECL(dpds)
-QK_DECL(dpdp) QK_DECL(ddss) QK_DECL(ddps) QK_DECL(ddpp) QK_DECL(ddds) QK_DECL(dddp) QK_DECL(dddd)
+// the thread-per-quartet kernel of a class in the given form (FockMode)
+using FockFn = const void* (*)(int);
+#define QK_DECL(T) const void* fock_fn_##T(int); const void* fock_f32_fn_##T(int);
+QK_DECL(ssss) QK_DECL(psss) QK_DECL(psps) QK_DECL(ppss) QK_DECL(ppps) QK_DECL(pppp) QK_DECL(dsss) QK_DECL(dsps)
+QK_DECL(dspp) QK_DECL(dsds) QK_DECL(dpss) QK_DECL(dpps) QK_DECL(dppp) QK_DECL(dpds) QK_DECL(ddss) QK_DECL(ddps)
 #undef QK_DECL
 #define QK_DECL(T)                                                                                              \
     void launch_schwarz_##T(const int*, int, const int*, const int*, const int*, const int*, const DevQshells&, \
@@ -193,11 +184,15 @@ QK_DECL(ss) QK_DECL(ps) QK_DECL(pp) QK_DECL(ds) QK_DECL(dp) QK_DECL(dd)
 #undef QK_DECL
 
 // order matches gen_eri.quartet_classes()
-static const FockLauncher kFockLaunchers[kNumQuartetClasses] = {
-    launch_fock_ssss, launch_fock_psss, launch_fock_psps, launch_fock_ppss, launch_fock_ppps, launch_fock_pppp,
-    launch_fock_dsss, launch_fock_dsps, launch_fock_dspp, launch_fock_dsds, launch_fock_dpss, launch_fock_dpps,
-    launch_fock_dppp, launch_fock_dpds, launch_fock_dpdp, launch_fock_ddss, launch_fock_ddps, launch_fock_ddpp,
-    launch_fock_ddds, launch_fock_dddp, launch_fock_dddd};
+static const FockFn kFockFn[kNumQuartetClasses] = {
+    fock_fn_ssss, fock_fn_psss, fock_fn_psps, fock_fn_ppss, fock_fn_ppps, fock_fn_pppp, fock_fn_dsss,
+    fock_fn_dsps, fock_fn_dspp, fock_fn_dsds, fock_fn_dpss, fock_fn_dpps, fock_fn_dppp, fock_fn_dpds, nullptr,
+    fock_fn_ddss, fock_fn_ddps, nullptr, nullptr, nullptr, nullptr};
+static const FockFn kFockF32Fn[kNumQuartetClasses] = {
+    fock_f32_fn_ssss, fock_f32_fn_psss, fock_f32_fn_psps, fock_f32_fn_ppss, fock_f32_fn_ppps, fock_f32_fn_pppp,
+    fock_f32_fn_dsss, fock_f32_fn_dsps, fock_f32_fn_dspp, fock_f32_fn_dsds, fock_f32_fn_dpss, fock_f32_fn_dpps,
+    fock_f32_fn_dppp, fock_f32_fn_dpds, nullptr, fock_f32_fn_ddss, fock_f32_fn_ddps, nullptr, nullptr, nullptr,
+    nullptr};
 static const SchwarzLauncher kSchwarzLaunchers[kNumPairClasses] = {
     launch_schwarz_ss, launch_schwarz_ps, launch_schwarz_pp, launch_schwarz_ds, launch_schwarz_dp, launch_schwarz_dd};
 
@@ -223,55 +218,40 @@ void launch_team_f32_class(int k, const FockArgs& a, const ClassWork& w, int gri
     kTeamF32Launchers[k](a, w, grid, s);
 }
 
-#define QK_DECL(T) int fock_blocks_##T(size_t, bool);
-QK_DECL(ssss) QK_DECL(psss) QK_DECL(psps) QK_DECL(ppss) QK_DECL(ppps) QK_DECL(pppp) QK_DECL(dsss)
-QK_DECL(dsps) QK_DECL(dspp) QK_DECL(dsds) QK_DECL(dpss) QK_DECL(dpps) QK_DECL(dppp) QK_DECL(dpds)
-QK_DECL(dpdp) QK_DECL(ddss) QK_DECL(ddps) QK_DECL(ddpp) QK_DECL(ddds) QK_DECL(dddp) QK_DECL(dddd)
-#undef QK_DECL
-using BlocksQuery = int (*)(size_t, bool);
-static const BlocksQuery kFockBlocks[kNumQuartetClasses] = {
-    fock_blocks_ssss, fock_blocks_psss, fock_blocks_psps, fock_blocks_ppss, fock_blocks_ppps, fock_blocks_pppp,
-    fock_blocks_dsss, fock_blocks_dsps, fock_blocks_dspp, fock_blocks_dsds, fock_blocks_dpss, fock_blocks_dpps,
-    fock_blocks_dppp, fock_blocks_dpds, fock_blocks_dpdp, fock_blocks_ddss, fock_blocks_ddps, fock_blocks_ddpp,
-    fock_blocks_ddds, fock_blocks_dddp, fock_blocks_dddd};
-// resident blocks of 256 threads per CU of the FP64 thread-per-quartet kernel
-// of class k (its staged form if staged) with lds bytes of dynamic LDS
-// (registers, LDS and wave limits)
-int fock_class_blocks(int k, size_t lds, bool staged) { return kFockBlocks[k](lds, staged); }
+bool fock_class_has_f32(int k) { return kFockF32Fn[k] != nullptr || kTeamF32Launchers[k] != nullptr; }
 
-using ScratchQuery = size_t (*)();
-static const ScratchQuery kFockScratch[kNumQuartetClasses] = {
-    fock_scratch_ssss, fock_scratch_psss, fock_scratch_psps, fock_scratch_ppss, fock_scratch_ppps, fock_scratch_pppp,
-    fock_scratch_dsss, fock_scratch_dsps, fock_scratch_dspp, fock_scratch_dsds, fock_scratch_dpss, fock_scratch_dpps,
-    fock_scratch_dppp, fock_scratch_dpds, fock_scratch_dpdp, fock_scratch_ddss, fock_scratch_ddps, fock_scratch_ddpp,
-    fock_scratch_ddds, fock_scratch_dddp, fock_scratch_dddd};
+// the thread-per-quartet kernel of class k in form `mode` (FockMode)
+static const void* fock_fn(int k, bool fp32, int mode) { return (fp32 ? kFockF32Fn : kFockFn)[k](mode); }
 
-#define QK_DECL(T) void launch_fock_f32_##T(const FockArgs&, const ClassWork&, int, size_t, hipStream_t); size_t fock_scratch_f32_##T();
-QK_DECL(ssss) QK_DECL(psss) QK_DECL(psps) QK_DECL(ppss) QK_DECL(ppps) QK_DECL(pppp) QK_DECL(dsss)
-QK_DECL(dsps) QK_DECL(dspp) QK_DECL(dsds) QK_DECL(dpss) QK_DECL(dpps) QK_DECL(dppp) QK_DECL(dpds)
-QK_DECL(ddss) QK_DECL(ddps)
-#undef QK_DECL
-// FP32 kernels of the mixed-precision mode; the cooperative classes stay FP64
-static const FockLauncher kFockF32Launchers[kNumQuartetClasses] = {
-    launch_fock_f32_ssss, launch_fock_f32_psss, launch_fock_f32_psps, launch_fock_f32_ppss, launch_fock_f32_ppps,
-    launch_fock_f32_pppp, launch_fock_f32_dsss, launch_fock_f32_dsps, launch_fock_f32_dspp, launch_fock_f32_dsds,
-    launch_fock_f32_dpss, launch_fock_f32_dpps, launch_fock_f32_dppp, launch_fock_f32_dpds, nullptr,
-    launch_fock_f32_ddss, launch_fock_f32_ddps, nullptr, nullptr, nullptr, nullptr};
-static const ScratchQuery kFockF32Scratch[kNumQuartetClasses] = {
-    fock_scratch_f32_ssss, fock_scratch_f32_psss, fock_scratch_f32_psps, fock_scratch_f32_ppss, fock_scratch_f32_ppps,
-    fock_scratch_f32_pppp, fock_scratch_f32_dsss, fock_scratch_f32_dsps, fock_scratch_f32_dspp, fock_scratch_f32_dsds,
-    fock_scratch_f32_dpss, fock_scratch_f32_dpps, fock_scratch_f32_dppp, fock_scratch_f32_dpds, nullptr,
-    fock_scratch_f32_ddss, fock_scratch_f32_ddps, nullptr, nullptr, nullptr, nullptr};
-bool fock_class_has_f32(int k) { return kFockF32Launchers[k] != nullptr || kTeamF32Launchers[k] != nullptr; }
-void launch_fock_f32_class(int k, const FockArgs& a, const ClassWork& w, int grid, size_t lds, hipStream_t s) {
-    kFockF32Launchers[k](a, w, grid, lds, s);
+// scratch of that kernel per lane; a property of the code, asked for once
+long long fock_class_scratch(int k, bool fp32, int mode) {
+    static std::atomic<long long> known[2][kNumQuartetClasses][4];   // value + 1
+    std::atomic<long long>& v = known[fp32 ? 1 : 0][k][mode];
+    long long x = v.load(std::memory_order_relaxed);
+    if (x == 0) {
+        x = kernel_scratch(fock_fn(k, fp32, mode)) + 1;
+        v.store(x, std::memory_order_relaxed);
+    }
+    return x - 1;
 }
-size_t fock_class_scratch_f32(int k) { return kFockF32Scratch[k] ? kFockF32Scratch[k]() : 0; }
 
-void launch_fock_class(int k, const FockArgs& a, const ClassWork& w, int grid, size_t lds, hipStream_t s) {
-    kFockLaunchers[k](a, w, grid, lds, s);
+// resident blocks of 256 threads per CU of that kernel with lds bytes of
+// dynamic LDS (registers, LDS and wave limits)
+int fock_class_blocks(int k, bool fp32, int mode, size_t lds) {
+    int nb = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, fock_fn(k, fp32, mode), 256, lds) != hipSuccess) return 0;
+    return nb;
 }
-size_t fock_class_scratch(int k) { return kFockScratch[k](); }
+
+void launch_fock_class(int k, bool fp32, int mode, const FockArgs& a, const ClassWork& w, int grid, size_t lds,
+                       hipStream_t s) {
+    const void* f = fock_fn(k, fp32, mode);
+    if (lds > 64 * 1024) (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    FockArgs aa = a;
+    ClassWork ww = w;
+    void* args[] = {&aa, &ww};
+    (void)hipLaunchKernel(f, dim3(grid), dim3(256), args, lds, s);
+}
 void launch_schwarz(int pair_class, const int* pairs, int np, const int* qa, const int* qb, const int* prim0,
                     const int* nprim, const DevQshells& qs, const DevPrims& pp, const double* xyz, const double* cons,
                     double* ymax, double* pmax, hipStream_t s) {
@@ -288,14 +268,14 @@ void launch_density_cutoff(const double* D, const int* sh_f0, const int* sh_nf, 
     hipLaunchKernelGGL(density_cutoff, dim3(blocks_for((long long)ns * ns, 256)), dim3(256), 0, s, D, sh_f0, sh_nf,
                        cm, n, ns);
 }
-void launch_compact(const CompactArgs& a, const int4* segs, long long nsegs, int* list, int* counts, hipStream_t s) {
+void launch_compact(const CompactArgs& a, const int4* segs, long long nsegs, int* list, hipStream_t s) {
     if (nsegs <= 0) return;
     // rows staged while the block's four wavefronts need at most 64 KB
     // (nshell <= 1024)
     const size_t rows = sizeof(double) * 2 * 4 * (size_t)a.nshell;
     const int stage = rows <= 64 * 1024 ? 1 : 0;
     hipLaunchKernelGGL(compact_kernel, dim3((unsigned)((nsegs + 3) / 4)), dim3(256), stage ? rows : 0, s, a, segs,
-                       nsegs, list, counts, stage);
+                       nsegs, list, stage);
 }
 void launch_fill_u64(unsigned long long* p, long long count, hipStream_t s) {
     if (count > 0) hipLaunchKernelGGL(fill_u64, dim3(blocks_for(count, 256)), dim3(256), 0, s, p, count);

@@ -24,13 +24,12 @@
 #include "grad_tables.inc"
 
 namespace qk {
-void launch_fock_class(int k, const FockArgs& a, const ClassWork& w, int grid, size_t lds, hipStream_t s);
-size_t fock_class_scratch(int k);
-int fock_class_blocks(int k, size_t lds, bool staged);
+void launch_fock_class(int k, bool fp32, int mode, const FockArgs& a, const ClassWork& w, int grid, size_t lds,
+                       hipStream_t s);
+long long fock_class_scratch(int k, bool fp32, int mode);
+int fock_class_blocks(int k, bool fp32, int mode, size_t lds);
 bool fock_class_is_team(int k);
 bool fock_class_has_f32(int k);
-void launch_fock_f32_class(int k, const FockArgs& a, const ClassWork& w, int grid, size_t lds, hipStream_t s);
-size_t fock_class_scratch_f32(int k);
 void launch_team_class(int k, const FockArgs& a, const ClassWork& w, int grid, hipStream_t s);
 void launch_team_f32_class(int k, const FockArgs& a, const ClassWork& w, int grid, hipStream_t s);
 void launch_scale_density(const double* D, const double* cons, double* Dp, float* Dpf, int n, hipStream_t s);
@@ -43,7 +42,7 @@ int launch_grad_light(int k, const GradArgs& a, const ClassWork& w, int grid, bo
 void launch_density_cutoff(const double* D, const int* sh_f0, const int* sh_nf, double* cm, int n, int ns,
                            hipStream_t s);
 void launch_fill_u64(unsigned long long* p, long long count, hipStream_t s);
-void launch_compact(const CompactArgs& a, const int4* segs, long long nsegs, int* list, int* counts, hipStream_t s);
+void launch_compact(const CompactArgs& a, const int4* segs, long long nsegs, int* list, hipStream_t s);
 void launch_oneint(const OneFuncs& f, const OneSys& sys, const int2* const* pairs, const long long* npairs, double* S,
                    double* H, hipStream_t s);
 void launch_oneint_grad(const OneFuncs& f, const OneSys& sys, const int2* const* pairs, const long long* npairs,
@@ -193,12 +192,14 @@ struct ClassHost {
     DBuf<Tile> d_tiles, d_tiles32;
     DBuf<int2> d_runs, d_runs32;
     // the same candidates as segments {bra pair, first ket, end ket, offset}
-    // (one bra pair and one ket group each), for the per-build density
-    // compaction; segruns: [first, end) segment of each bra pair
-    long long nsegs = 0, nsegs32 = 0, nsegruns = 0, nsegruns32 = 0;
+    // (one bra pair and one ket group each) with the first tile of each, for
+    // the per-build density compaction, and the steps and kets it writes
+    long long nsegs = 0, nsegs32 = 0;
     DBuf<int4> d_segs, d_segs32;
-    DBuf<int2> d_segruns, d_segruns32;
-    DBuf<int> d_list, d_list32, d_counts, d_counts32;
+    DBuf<int> d_slot0, d_slot032;
+    DBuf<Tile> d_steps, d_steps32;
+    DBuf<int> d_list, d_list32;
+    int lsplit = 0, lsplit32 = 0;   // wavefronts per tile, log2 (share_tiles)
     // compaction pays where segments span several 64-ket steps (with short
     // segments every step is already the whole segment)
     bool compact = false, compact32 = false;
@@ -275,7 +276,7 @@ struct qk_ctx {
     DBuf<int4> d_gsegs[2][kNumQuartetClasses];
     DBuf<Tile> d_gsteps[2][kNumQuartetClasses];
     DBuf<int> d_gslot0[2][kNumQuartetClasses];
-    DBuf<int> d_glist[2][kNumQuartetClasses], d_gcounts[2][kNumQuartetClasses];
+    DBuf<int> d_glist[2][kNumQuartetClasses];
     double grad_prep_cutoff = -1, grad_prep_thr = -1;
     int grad_prep_precision = -1;
     bool grad_prepared = false;
@@ -288,6 +289,7 @@ struct qk_ctx {
     DBuf<double> d_xyz, d_cons;
     DBuf<int> dq_atom, dq_f0, dq_shell, dq_qf, dq_nc;
     DBuf<int> dp_qa, dp_qb, dp_prim0, dp_nprim;
+    DBuf<PairRec> dp_rec;
     DBuf<int> dp_sh, dp_at;   // per pair: shells and atoms of its two Qshells, 16 bits each (< 2^15)
     DBuf<double> dp_Y;
     DBuf<double> dpp_zeta, dpp_oo2z, dpp_Px, dpp_Py, dpp_Pz, dpp_K, dpp_cut, dpp_ea, dpp_eb;
@@ -629,6 +631,21 @@ extern "C" int qk_set_schwarz(qk_ctx* c, const double* Ycutoff, const double* cu
 
 using ListSumsFn = std::function<int(const std::vector<long long>&, std::vector<ListDst>&)>;
 
+// Wavefronts per tile, log2, of a class with `tiles` tiles whose quartets hold at
+// most `prims` primitive quartets.  A lane works through its quartet's primitives
+// one after another (up to 1,296 of them, 0.4 us each in FP64), so where a class
+// has too few tiles to fill the GPU the longest chain is the kernel's time; there
+// each tile's primitives are split over wavefronts that would be idle (one water:
+// Fock build 2.39 -> 0.54 ms).  2,048 wavefronts (two
+// per SIMD) are taken as full: above that a share only repeats the quartet's
+// screening and digestion.
+constexpr long long kSplitTiles = 2048;
+static int share_tiles(long long tiles, int prims) {
+    int l = 0;
+    while (l < 6 && tiles > 0 && (tiles << l) < kSplitTiles && (2 << l) <= prims) ++l;
+    return l;
+}
+
 // The work lists of the entries E (qk_lists.hip): per-item counts and their
 // scans on the device, the per-class sums to the host, where dst_f allocates
 // the lists and says where they go; then the lists are written.  With runs_f
@@ -681,6 +698,44 @@ static int build_lists(qk_ctx* c, const std::vector<ListEntry>& E, const std::ve
     }
     HIPCHK(hipStreamSynchronize(nullptr));
     return 0;
+}
+
+// the most primitive quartets of any quartet of each class, from the pair groups
+static std::vector<int> most_primitives(const qk_ctx* c) {
+    int np[kNumPairClasses] = {};
+    for (size_t k = 0; k < c->ap_cls.size(); ++k) np[c->ap_cls[k]] = std::max(np[c->ap_cls[k]], c->ap_nprim[k]);
+    std::vector<int> out(kNumQuartetClasses);
+    for (int k = 0; k < kNumQuartetClasses; ++k)
+        out[k] = np[pair_class_of(kClassL[k][0], kClassL[k][1])] * np[pair_class_of(kClassL[k][2], kClassL[k][3])];
+    return out;
+}
+
+// LDS for one bra's exchange rows.  gfx950 gives a block up to 160 KB of
+// dynamic LDS (152 KB leave room for the bra slab and the kernels' static
+// LDS, <= 6 KB), but rows beyond 64 KB hold a CU to one or two blocks and
+// every run zeroes and flushes them: measured on (H2O)64 (1,600 functions)
+// against direct atomics into X, run mode with large rows pays for the FP64
+// classes up to a d-p bra (ppps 16.5 -> 10.7 ms, dpps 17.4 -> 9.5 ms, FP64
+// build 235 -> 202 ms) and for the FP32 classes with a p or p-p ket (ppps
+// 10.3 -> 7.6 ms), and costs the FP32 classes with an s-s ket (dsss 6.6 ->
+// 9.1 ms) and every d-d bra (on (H2O)32, ddps 1.04 -> 1.77 ms)
+constexpr size_t kRowsLdsMax = 152 * 1024, kRowsLdsSmall = 64 * 1024;
+static int bra_rows(int k) { return ncart_of(kClassL[k][0]) + ncart_of(kClassL[k][1]); }
+// whether class k takes one bra pair per block with its exchange rows in LDS
+static bool fock_uses_runs(int k, int n, bool fp32) {
+    const size_t rows = sizeof(unsigned long long) * (size_t)bra_rows(k) * n;
+    const bool big_ok = bra_rows(k) <= 9 && rows <= kRowsLdsMax;
+    const int nket = ncart_of(kClassL[k][2]) * ncart_of(kClassL[k][3]);
+    return !fock_class_is_team(k) && (rows <= kRowsLdsSmall || (big_ok && (!fp32 || nket >= 3)));
+}
+
+// sets the wavefronts per tile of a run-mode launch and the blocks per run that
+// give each of them work; returns the blocks
+static long long share_runs(ClassWork& w, int lsplit) {
+    w.lsplit = lsplit;
+    w.lblocks = 0;
+    while (lsplit && (w.nruns * 4 << w.lblocks) < (w.ntiles << lsplit)) ++w.lblocks;
+    return w.nruns << w.lblocks;
 }
 
 static int prepare(qk_ctx* c, const qk_opts* o) {
@@ -769,6 +824,7 @@ static int prepare(qk_ctx* c, const qk_opts* o) {
         psh[k] = c->q_shell[qa[k]] | (c->q_shell[qb[k]] << 16);
         pat[k] = c->q_atom[qa[k]] | (c->q_atom[qb[k]] << 16);
     }
+    std::vector<PairRec> rec(std::max(npair, 1), PairRec{});
     // primitive-major layout per group: entry (pair k, primitive j) at
     // base(group) + j * count(group) + (k - start(group)); the copy itself runs
     // on the device (gather_prims_kernel)
@@ -791,8 +847,14 @@ static int prepare(qk_ctx* c, const qk_opts* o) {
         jsize += (long long)ne * g.count;
         if (jsize > INT32_MAX) { set_err("pair Coulomb buffer beyond 2^31 entries"); return -1; }
     }
+    for (int k = 0; k < npair; ++k)
+        rec[k] = PairRec{Yp[k], prim0[k], jofs[k],
+                         (unsigned)c->q_f0[qa[k]] | ((unsigned)c->q_f0[qb[k]] << 16), (unsigned)psh[k],
+                         (unsigned)pat[k],
+                         (unsigned)(c->q_qf[qa[k]] + c->q_qf[qb[k]]) | (qa[k] == qb[k] ? 16u : 0u) |
+                             ((unsigned)nprim[k] << 8)};
     (void)hipSetDevice(c->device);
-    if (c->dp_qa.upload(qa) || c->dp_qb.upload(qb) || c->dp_prim0.upload(prim0) || c->dp_pstride.upload(pstride) ||
+    if (c->dp_rec.upload(rec) || c->dp_qa.upload(qa) || c->dp_qb.upload(qb) || c->dp_prim0.upload(prim0) || c->dp_pstride.upload(pstride) ||
         c->dp_nprim.upload(nprim) || c->dp_Y.upload(Yp) || c->dp_sh.upload(psh) || c->dp_at.upload(pat) ||
         c->dp_jofs.upload(jofs) || c->d_sel.upload(sel) || c->d_J.alloc((size_t)std::max(jsize, 1LL)))
         return -1;
@@ -850,7 +912,7 @@ static int prepare(qk_ctx* c, const qk_opts* o) {
         const bool team = fock_class_is_team(k);
         const bool cap_ss = kClassL[k][0] + kClassL[k][1] == 0;
         LC[k] = ListClass{team ? 2 : 64, cap_ss || mixed ? 2048 : INT_MAX, cap_ss ? 2048 : INT_MAX,
-                          mixed && fock_class_has_f32(k) ? 1 : 0, team ? 0 : 1, 0, team ? 0 : 1, 0};
+                          mixed && fock_class_has_f32(k) ? 1 : 0, team ? 0 : 1, team ? 0 : 1};
         for (size_t gb = 0; gb < groups.size(); ++gb) {
             if (groups[gb].cls != cb) continue;
             const int kg0 = (int)KG.size();
@@ -868,6 +930,7 @@ static int prepare(qk_ctx* c, const qk_opts* o) {
     cls_item[kNumQuartetClasses] = nitem;
     cls_bra[kNumQuartetClasses] = nbra;
     if (c->classes.size() != (size_t)kNumQuartetClasses) c->classes.resize(kNumQuartetClasses);
+    const std::vector<int> most = most_primitives(c);
     const ListSumsFn fock_dst = [&](const std::vector<long long>& sm, std::vector<ListDst>& dst) -> int {
         for (int k = 0; k < kNumQuartetClasses; ++k) {
             ClassHost& CH = c->classes[k];
@@ -879,30 +942,36 @@ static int prepare(qk_ctx* c, const qk_opts* o) {
             CH.ntiles = v[0]; CH.ntiles32 = v[1]; CH.nsegs = v[2]; CH.nsegs32 = v[3];
             CH.total = v[4] + v[5];
             CH.total32 = v[5];
+            CH.lsplit = fock_uses_runs(k, c->nbasis, false) ? share_tiles(v[0], most[k]) : 0;
+            CH.lsplit32 = fock_uses_runs(k, c->nbasis, true) ? share_tiles(v[1], most[k]) : 0;
         }
         // every class's lists in one allocation
         Arena& A = c->fock_arena;
         A.reset();
-        std::vector<int> slot((size_t)kNumQuartetClasses * 8);
+        std::vector<int> slot((size_t)kNumQuartetClasses * 10);
         for (int k = 0; k < kNumQuartetClasses; ++k) {
             const long long* v = &sm[(size_t)k * kListCounts];
-            int* sl = &slot[(size_t)k * 8];
-            sl[0] = A.reserve<Tile>(v[0]); sl[1] = A.reserve<Tile>(v[1]);
-            sl[2] = A.reserve<int4>(v[2]); sl[3] = A.reserve<int4>(v[3]);
-            sl[4] = A.reserve<int>(v[4]); sl[5] = A.reserve<int>(v[5]);
-            sl[6] = A.reserve<int>(v[2]); sl[7] = A.reserve<int>(v[3]);
+            int* sl = &slot[(size_t)k * 10];
+            for (int f = 0; f < 2; ++f) {
+                sl[f] = A.reserve<Tile>(v[f]);
+                sl[2 + f] = A.reserve<int4>(v[2 + f]);
+                sl[4 + f] = A.reserve<int>(v[4 + f]);
+                sl[6 + f] = A.reserve<int>(v[2 + f]);
+                sl[8 + f] = A.reserve<Tile>(v[2 + f] ? v[f] : 0);
+            }
         }
         if (A.commit()) return -1;
         for (int k = 0; k < kNumQuartetClasses; ++k) {
             ClassHost& CH = c->classes[k];
             const long long* v = &sm[(size_t)k * kListCounts];
-            const int* sl = &slot[(size_t)k * 8];
+            const int* sl = &slot[(size_t)k * 10];
             A.place(CH.d_tiles, sl[0], v[0]); A.place(CH.d_tiles32, sl[1], v[1]);
             A.place(CH.d_segs, sl[2], v[2]); A.place(CH.d_segs32, sl[3], v[3]);
             A.place(CH.d_list, sl[4], v[4]); A.place(CH.d_list32, sl[5], v[5]);
-            A.place(CH.d_counts, sl[6], v[2]); A.place(CH.d_counts32, sl[7], v[3]);
-            dst[k] = ListDst{CH.d_tiles.p, CH.d_tiles32.p, CH.d_segs.p, CH.d_segs32.p, nullptr, nullptr,
-                             nullptr, nullptr, nullptr, nullptr};
+            A.place(CH.d_slot0, sl[6], v[2]); A.place(CH.d_slot032, sl[7], v[3]);
+            A.place(CH.d_steps, sl[8], v[2] ? v[0] : 0); A.place(CH.d_steps32, sl[9], v[3] ? v[1] : 0);
+            dst[k] = ListDst{CH.d_tiles.p, CH.d_tiles32.p, CH.d_segs.p, CH.d_segs32.p, CH.d_slot0.p, CH.d_slot032.p,
+                             nullptr, nullptr};
         }
         return 0;
     };
@@ -910,7 +979,7 @@ static int prepare(qk_ctx* c, const qk_opts* o) {
         for (int k = 0; k < kNumQuartetClasses; ++k) {
             ClassHost& CH = c->classes[k];
             const long long* v = &rs[(size_t)k * kRunCounts];
-            CH.nruns = v[0]; CH.nruns32 = v[1]; CH.nsegruns = v[2]; CH.nsegruns32 = v[3];
+            CH.nruns = v[0]; CH.nruns32 = v[1];
         }
         Arena& A = c->fock_run_arena;
         A.reset();
@@ -922,9 +991,7 @@ static int prepare(qk_ctx* c, const qk_opts* o) {
             const long long* v = &rs[(size_t)k * kRunCounts];
             const int s0 = k * kRunCounts;
             A.place(CH.d_runs, s0, v[0]); A.place(CH.d_runs32, s0 + 1, v[1]);
-            A.place(CH.d_segruns, s0 + 2, v[2]); A.place(CH.d_segruns32, s0 + 3, v[3]);
             dst[k].r64 = CH.d_runs.p; dst[k].r32 = CH.d_runs32.p;
-            dst[k].sr64 = CH.d_segruns.p; dst[k].sr32 = CH.d_segruns32.p;
         }
         return 0;
     };
@@ -937,8 +1004,8 @@ static int prepare(qk_ctx* c, const qk_opts* o) {
         ClassHost& CH = c->classes[k];
         const int LT = kClassL[k][0] + kClassL[k][1] + kClassL[k][2] + kClassL[k][3];
         const bool small = kClassL[k][1] == 0 && kClassL[k][3] == 0 && LT <= 2 && kClassL[k][0] <= 1;
-        CH.compact = CH.nsegs > 0 && LT >= 1;
-        CH.compact32 = CH.nsegs32 > 0 && !small;
+        CH.compact = CH.nsegs > 0 && LT >= 1 && CH.lsplit == 0;   // split: lanes to spare, one launch less
+        CH.compact32 = CH.nsegs32 > 0 && !small && CH.lsplit32 == 0;
     }
     if (mixed && !c->d_boys_tab.p) {
         std::vector<float> tab;
@@ -987,6 +1054,7 @@ static FockArgs make_args(qk_ctx* c, const qk_opts* o, const FockBufs& fb) {
     a.ppf = {c->dkf_zeta.p, c->dkf_oo2z.p, c->dkf_Px.p, c->dkf_Py.p, c->dkf_Pz.p, c->dkf_K.p, c->dkf_cut.p};
     a.Dpf = fb.Dpf;
     a.boys_tab = c->d_boys_tab.p;
+    a.rec = c->dp_rec.p;
     a.xyz = c->d_xyz.p;
     a.Dp = fb.Dp;
     a.cutmat = fb.cm;
@@ -1001,7 +1069,6 @@ static FockArgs make_args(qk_ctx* c, const qk_opts* o, const FockBufs& fb) {
     a.prim_limit = o->prim_limit;
     a.hybrid = o->hybrid;
     a.boys_qshell_order = o->boys_order == QK_BOYS_ORDER_QSHELL ? 1 : 0;
-    a.stage_d = 0;
     return a;
 }
 
@@ -1015,8 +1082,10 @@ static CompactArgs compact_args(const qk_ctx* c, const FockArgs& a, int grad, do
     ca.nshell = a.nshell;
     ca.tau = tau;
     ca.grad = grad;
+    ca.pstride = a.pr.pstride;
     ca.steps = nullptr;
     ca.slot0 = nullptr;
+    ca.chunk = 64;
     return ca;
 }
 
@@ -1078,16 +1147,6 @@ static int fock_enqueue(qk_ctx* c, const double* dD, const double* dcutmat_or_nu
     // are in flight.  Kernels that spill get a grid small enough
     // that their private-segment backing stays under kScratchBudget
     // (scratch_grid_cap); the grid-stride loop over tiles covers the rest.
-    // LDS for one bra's exchange rows.  gfx950 gives a block up to 160 KB of
-    // dynamic LDS (152 KB leave room for the bra slab and the kernels' static
-    // LDS, <= 6 KB), but rows beyond 64 KB hold a CU to one or two blocks and
-    // every run zeroes and flushes them: measured on (H2O)64 (1,600 functions)
-    // against direct atomics into X, run mode with large rows pays for the FP64
-    // classes up to a d-p bra (ppps 16.5 -> 10.7 ms, dpps 17.4 -> 9.5 ms, FP64
-    // build 235 -> 202 ms) and for the FP32 classes with a p or p-p ket (ppps
-    // 10.3 -> 7.6 ms), and costs the FP32 classes with an s-s ket (dsss 6.6 ->
-    // 9.1 ms) and every d-d bra (on (H2O)32, ddps 1.04 -> 1.77 ms)
-    constexpr size_t kRowsLdsMax = 152 * 1024, kRowsLdsSmall = 64 * 1024;
     constexpr size_t kStageLds = 64 * 1024;
     // With light FP64 lists (under a tenth of the tiles) the second stream
     // ends first, so the FP32 lists of (dd|dp) and (dd|dd) follow the FP64
@@ -1107,12 +1166,9 @@ static int fock_enqueue(qk_ctx* c, const double* dD, const double* dcutmat_or_nu
         // the stream of this class's FP64 list
         const hipStream_t l64 = !mixed && (pos & 1) ? s : s64;
         // one bra pair per block with its exchange rows in LDS, when they fit
-        const int nrow = ncart_of(kClassL[k][0]) + ncart_of(kClassL[k][1]);
+        const int nrow = bra_rows(k);
         const size_t rows_lds = sizeof(unsigned long long) * (size_t)nrow * n;
-        const bool big_ok = nrow <= 9 && rows_lds <= kRowsLdsMax;
-        const int nket = ncart_of(kClassL[k][2]) * ncart_of(kClassL[k][3]);
-        const bool use_runs = !fock_class_is_team(k) && (rows_lds <= kRowsLdsSmall || big_ok);
-        const bool use_runs32 = !fock_class_is_team(k) && (rows_lds <= kRowsLdsSmall || (big_ok && nket >= 3));
+        const bool use_runs = fock_uses_runs(k, n, false), use_runs32 = fock_uses_runs(k, n, true);
         // dynamic LDS of the thread-per-quartet kernels: the exchange rows and
         // one bra slab (run mode), or four bra slabs (7 x 64 values each)
         const size_t slab64 = 7 * 64 * sizeof(double), slab32 = 7 * 64 * sizeof(float);
@@ -1128,7 +1184,10 @@ static int fock_enqueue(qk_ctx* c, const double* dD, const double* dcutmat_or_nu
         }
         if (use_runs && c->stage_ok[k] < 0) {
             const size_t plain = rows_lds + slab64, staged = plain + drows64;
-            c->stage_ok[k] = staged <= kStageLds && fock_class_blocks(k, staged, true) >= fock_class_blocks(k, plain, false) ? 1 : 0;
+            c->stage_ok[k] = staged <= kStageLds && fock_class_blocks(k, false, kStaged, staged) >=
+                                                        fock_class_blocks(k, false, kRuns, plain)
+                                 ? 1
+                                 : 0;
         }
         const bool stage64 = use_runs && c->stage_ok[k] == 1;
         const size_t lds64 = use_runs ? rows_lds + slab64 + (stage64 ? drows64 : 0) : 4 * slab64;
@@ -1136,28 +1195,31 @@ static int fock_enqueue(qk_ctx* c, const double* dD, const double* dcutmat_or_nu
         if (CH.ntiles) {
             if (c->timing) HIPCHK(hipEventRecord(c->ev_t0[k], l64));
             a.counters = fb->counters + 2 * k;
-            a.stage_d = stage64 ? 1 : 0;
             if (fock_class_is_team(k)) {
                 ClassWork w{CH.d_tiles.p, CH.ntiles, nullptr, 0};
                 // one 64-lane block per tile; up to 16 resident per CU
                 const int grid = (int)std::min<long long>(CH.ntiles, 256LL * 16);
                 launch_team_class(k, a, w, grid, l64);
             } else {
-                const long long cap = std::min(256LL * 16, scratch_grid_cap((long long)fock_class_scratch(k), 4));
-                if (use_runs && CH.compact && fb->compact) {
-                    // density screen first: every lane of the class kernel then has a quartet
-                    launch_compact(ca, CH.d_segs.p, CH.nsegs, CH.d_list.p, CH.d_counts.p, l64);
-                    ClassWork w{CH.d_tiles.p, CH.ntiles, CH.d_segruns.p, CH.nsegruns, CH.d_segs.p, CH.d_list.p,
-                                CH.d_counts.p};
-                    launch_fock_class(k, a, w, (int)std::min<long long>(CH.nsegruns, cap), lds64, l64);
-                } else if (use_runs) {
-                    ClassWork w{CH.d_tiles.p, CH.ntiles, CH.d_runs.p, CH.nruns};
-                    launch_fock_class(k, a, w, (int)std::min<long long>(CH.nruns, cap), lds64, l64);
-                } else {
-                    ClassWork w{CH.d_tiles.p, CH.ntiles, nullptr, 0};
-                    const long long want = (CH.ntiles + 3) / 4;   // 4 wavefronts per block
-                    launch_fock_class(k, a, w, (int)std::min<long long>(want, cap), lds64, l64);
+                const int mode = !use_runs ? kNoRuns : (stage64 ? kStaged : kRuns);
+                const long long cap = std::min(256LL * 16, scratch_grid_cap(fock_class_scratch(k, false, mode), 4));
+                ClassWork w{CH.d_tiles.p, CH.ntiles};
+                long long grid = (CH.ntiles + 3) / 4;   // 4 wavefronts per block
+                if (use_runs) {
+                    w.runs = CH.d_runs.p;
+                    w.nruns = CH.nruns;
+                    grid = share_runs(w, CH.lsplit);
+                    if (CH.compact && fb->compact) {
+                        // density screen first: every lane of the class kernel then has a quartet
+                        CompactArgs cq = ca;
+                        cq.steps = CH.d_steps.p;
+                        cq.slot0 = CH.d_slot0.p;
+                        launch_compact(cq, CH.d_segs.p, CH.nsegs, CH.d_list.p, l64);
+                        w.list = CH.d_list.p;
+                        w.steps = CH.d_steps.p;
+                    }
                 }
+                launch_fock_class(k, false, mode, a, w, (int)std::min(grid, cap), lds64, l64);
             }
             HIPCHK(hipGetLastError());
             if (c->timing) HIPCHK(hipEventRecord(c->ev_t1[k], l64));
@@ -1166,32 +1228,31 @@ static int fock_enqueue(qk_ctx* c, const double* dD, const double* dcutmat_or_nu
         if (mixed && CH.ntiles32) {
             const hipStream_t ls = light64 && (k == 19 || k == 20) ? s64 : s;
             a.counters = fb->counters + 2 * kNumQuartetClasses + 2 * k;
-            a.stage_d = 0;
-            const long long cap = std::min(256LL * 16, scratch_grid_cap((long long)fock_class_scratch_f32(k), 4));
-            const int slot = kNumQuartetClasses + k;
+                    const int slot = kNumQuartetClasses + k;
             if (c->timing) HIPCHK(hipEventRecord(c->ev_t0[slot], ls));
-            ClassWork w{CH.d_tiles32.p, CH.ntiles32, nullptr, 0};
-            int grid = (int)std::min<long long>((CH.ntiles32 + 3) / 4, cap);
-            size_t lds = lds32;
-            // one 64-lane block per tile; up to 20 resident per CU (five wavefronts per SIMD)
-            if (fock_class_is_team(k)) grid = (int)std::min<long long>(CH.ntiles32, 256LL * 20);
-            if (use_runs32 && CH.compact32 && fb->compact) {
-                launch_compact(ca, CH.d_segs32.p, CH.nsegs32, CH.d_list32.p, CH.d_counts32.p, ls);
-                w.runs = CH.d_segruns32.p;
-                w.nruns = CH.nsegruns32;
-                w.segs = CH.d_segs32.p;
-                w.list = CH.d_list32.p;
-                w.counts = CH.d_counts32.p;
-                grid = (int)std::min<long long>(w.nruns, cap);
-                lds = lds32;
-            } else if (use_runs32) {
-                w.runs = CH.d_runs32.p;
-                w.nruns = CH.nruns32;
-                grid = (int)std::min<long long>(w.nruns, cap);
-                lds = lds32;
+            ClassWork w{CH.d_tiles32.p, CH.ntiles32};
+            if (fock_class_is_team(k)) {
+                // one 64-lane block per tile; up to 20 resident per CU (five wavefronts per SIMD)
+                launch_team_f32_class(k, a, w, (int)std::min<long long>(CH.ntiles32, 256LL * 20), ls);
+            } else {
+                const int mode = use_runs32 ? kRuns : kNoRuns;
+                const long long cap = std::min(256LL * 16, scratch_grid_cap(fock_class_scratch(k, true, mode), 4));
+                long long grid = (CH.ntiles32 + 3) / 4;
+                if (use_runs32) {
+                    w.runs = CH.d_runs32.p;
+                    w.nruns = CH.nruns32;
+                    grid = share_runs(w, CH.lsplit32);
+                    if (CH.compact32 && fb->compact) {
+                        CompactArgs cq = ca;
+                        cq.steps = CH.d_steps32.p;
+                        cq.slot0 = CH.d_slot032.p;
+                        launch_compact(cq, CH.d_segs32.p, CH.nsegs32, CH.d_list32.p, ls);
+                        w.list = CH.d_list32.p;
+                        w.steps = CH.d_steps32.p;
+                    }
+                }
+                launch_fock_class(k, true, mode, a, w, (int)std::min(grid, cap), lds32, ls);
             }
-            if (fock_class_is_team(k)) launch_team_f32_class(k, a, w, grid, ls);
-            else launch_fock_f32_class(k, a, w, grid, lds, ls);
             HIPCHK(hipGetLastError());
             if (c->timing) HIPCHK(hipEventRecord(c->ev_t1[slot], ls));
             c->cls_timed[slot] = c->timing;
@@ -1531,7 +1592,7 @@ static int grad_prepare(qk_ctx* c, const qk_opts* o) {
         const int ck = pair_class_of(kClassL[k][2], kClassL[k][3]);
         const bool light = grad_class_is_light(k);
         const int chunk = light ? 64 : 1;
-        LC[k] = ListClass{chunk, INT_MAX, INT_MAX, mixed ? 1 : 0, light ? 1 : 0, 1, 0, 0};
+        LC[k] = ListClass{chunk, INT_MAX, INT_MAX, mixed ? 1 : 0, light ? 1 : 0, 0};
         for (size_t gb = 0; gb < ng; ++gb) {
             if (c->grp_cls[gb] != cb) continue;
             for (size_t gk = 0; gk < ng; ++gk) {
@@ -1558,39 +1619,37 @@ static int grad_prepare(qk_ctx* c, const qk_opts* o) {
         // every class's lists in one allocation
         Arena& A = c->grad_arena;
         A.reset();
-        std::vector<int> slot((size_t)kNumQuartetClasses * 12);
+        std::vector<int> slot((size_t)kNumQuartetClasses * 10);
         for (int k = 0; k < kNumQuartetClasses; ++k) {
             const long long* v = &sm[(size_t)k * kListCounts];
             const bool light = grad_class_is_light(k);
-            int* sl = &slot[(size_t)k * 12];
+            int* sl = &slot[(size_t)k * 10];
             sl[0] = A.reserve<Tile>(v[0]);
             sl[1] = A.reserve<Tile>(v[1]);
             for (int f = 0; f < 2; ++f) {
                 const long long nslot = light ? v[f] : 0;   // a light class's segment owns the slots of its tiles
-                sl[2 + 5 * f] = A.reserve<int4>(v[2 + f]);
-                sl[3 + 5 * f] = A.reserve<int>(v[2 + f]);
-                sl[4 + 5 * f] = A.reserve<Tile>(std::max<long long>(nslot, 1));
-                sl[5 + 5 * f] = A.reserve<int>(std::max<long long>(v[4 + f], 1));
-                sl[6 + 5 * f] = A.reserve<int>(std::max<long long>(v[2 + f], 1));
+                sl[2 + 4 * f] = A.reserve<int4>(v[2 + f]);
+                sl[3 + 4 * f] = A.reserve<int>(v[2 + f]);
+                sl[4 + 4 * f] = A.reserve<Tile>(std::max<long long>(nslot, 1));
+                sl[5 + 4 * f] = A.reserve<int>(std::max<long long>(v[4 + f], 1));
             }
         }
         if (A.commit()) return -1;
         for (int k = 0; k < kNumQuartetClasses; ++k) {
             const long long* v = &sm[(size_t)k * kListCounts];
             const bool light = grad_class_is_light(k);
-            const int* sl = &slot[(size_t)k * 12];
+            const int* sl = &slot[(size_t)k * 10];
             A.place(c->d_gtiles[k], sl[0], v[0]);
             A.place(c->d_gtiles32[k], sl[1], v[1]);
             for (int f = 0; f < 2; ++f) {
                 const long long nslot = light ? v[f] : 0;
-                A.place(c->d_gsegs[f][k], sl[2 + 5 * f], v[2 + f]);
-                A.place(c->d_gslot0[f][k], sl[3 + 5 * f], v[2 + f]);
-                A.place(c->d_gsteps[f][k], sl[4 + 5 * f], std::max<long long>(nslot, 1));
-                A.place(c->d_glist[f][k], sl[5 + 5 * f], std::max<long long>(v[4 + f], 1));
-                A.place(c->d_gcounts[f][k], sl[6 + 5 * f], std::max<long long>(v[2 + f], 1));
+                A.place(c->d_gsegs[f][k], sl[2 + 4 * f], v[2 + f]);
+                A.place(c->d_gslot0[f][k], sl[3 + 4 * f], v[2 + f]);
+                A.place(c->d_gsteps[f][k], sl[4 + 4 * f], std::max<long long>(nslot, 1));
+                A.place(c->d_glist[f][k], sl[5 + 4 * f], std::max<long long>(v[4 + f], 1));
             }
             dst[k] = ListDst{c->d_gtiles[k].p, c->d_gtiles32[k].p, c->d_gsegs[0][k].p, c->d_gsegs[1][k].p,
-                             c->d_gslot0[0][k].p, c->d_gslot0[1][k].p, nullptr, nullptr, nullptr, nullptr};
+                             c->d_gslot0[0][k].p, c->d_gslot0[1][k].p, nullptr, nullptr};
         }
         return 0;
     };
@@ -1668,8 +1727,10 @@ static int grad_enqueue(qk_ctx* c, const double* dD, const double* dcutmat_or_nu
     ca.nshell = ns;
     ca.tau = o->tau;
     ca.grad = 1;
+    ca.pstride = a.pr.pstride;
     ca.steps = nullptr;
     ca.slot0 = nullptr;
+    ca.chunk = 64;
     // Two streams, forked from the caller's and joined with events.  A mixed
     // gradient's FP64 list holds the few strongest pairs: its kernels have
     // little parallelism and long per-quartet chains, so they run on the second
@@ -1712,8 +1773,7 @@ static int grad_enqueue(qk_ctx* c, const double* dD, const double* dcutmat_or_nu
                 CompactArgs cq = ca;
                 cq.steps = c->d_gsteps[f][k].p;
                 cq.slot0 = c->d_gslot0[f][k].p;
-                launch_compact(cq, c->d_gsegs[f][k].p, c->ngsegs[f][k], c->d_glist[f][k].p,
-                               c->d_gcounts[f][k].p, ls);
+                launch_compact(cq, c->d_gsegs[f][k].p, c->ngsegs[f][k], c->d_glist[f][k].p, ls);
                 w.list = c->d_glist[f][k].p;
                 w.steps = cq.steps;
                 const int grid = (int)std::min<long long>((nt + 3) / 4, 256LL * 8);

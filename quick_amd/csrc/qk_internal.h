@@ -96,6 +96,18 @@ struct DevPairs {
     double* Y;     // Schwarz bound of the parent shell pair
 };
 
+// A significant pair's data in one 32-byte record, so that a lane has its ket
+// after one round trip to memory.
+struct alignas(16) PairRec {
+    double Y;            // Schwarz bound of the parent shell pair
+    int prim0;           // first primitive pair
+    int jofs;            // its block in the pair Coulomb buffer
+    unsigned f01;        // first basis functions of its two Qshells (16 bits each)
+    unsigned sh;         // parent shells
+    unsigned at;         // atoms
+    unsigned misc;       // Qfinal of both parent shells, summed (bits 0-3); same Qshell (4); primitive pairs (8-14)
+};
+
 // Per primitive pair.  In the kernels' copy the primitive pairs of a group of
 // pairs with equal primitive count are stored primitive-major: entry j of the
 // pairs q, q+1, ... of a group is contiguous, so the lanes of a wavefront (one
@@ -119,7 +131,7 @@ struct Tile {
     int p;
     int q0;
     int len;
-    int pad;
+    int pad;   // pairs in the ket group: the distance of its consecutive primitives
 };
 
 // Work-list construction on the device (qk_lists.hip).  An entry is a block of
@@ -138,23 +150,22 @@ struct KetGroup {
 };
 struct ListClass {
     int chunk;          // kets per tile
-    int cap64, cap32;   // candidates per run and per segment (FP64, FP32 lists)
+    int cap64, cap32;   // candidates per run and per segment (FP64, FP32 lists; multiples of chunk)
     int split;          // mixed precision: kets with Y_ij*Y_kl >= threshold stay FP64
     int segs;           // compaction segments are listed
-    int grad;           // gradient form: one segment per item, with its first tile
-    int runs;           // runs of tiles and segments per bra (Fock)
+    int runs;           // runs of tiles per bra (Fock)
     int pad;
 };
-// per class: where the lists go (FP64 / FP32 tiles, segments, the gradient's
-// first tile per segment, runs of tiles and of segments)
+// per class: where the lists go (FP64 / FP32 tiles, segments, the first tile
+// of each segment, runs of tiles)
 struct ListDst {
     Tile *t64, *t32;
     int4 *s64, *s32;
     int *slot64, *slot32;
-    int2 *r64, *r32, *sr64, *sr32;
+    int2 *r64, *r32;
 };
 constexpr int kListCounts = 6;   // per item: tiles, tiles32, segs, segs32, candidates, candidates32
-constexpr int kRunCounts = 4;    // per bra: runs, runs32, segment runs, segment runs32
+constexpr int kRunCounts = 2;    // per bra: runs, runs32
 // the primitive-pair fields copied primitive-major per group: zeta, 1/2zeta,
 // Px, Py, Pz, K, cut, and the two exponents
 constexpr int kPrimArrays = 9;
@@ -165,6 +176,9 @@ struct PrimArraysF {
     float* a[kPrimArrays];   // a[0] == nullptr: no FP32 copy
 };
 
+// forms of the thread-per-quartet Fock kernels (fock_quartets)
+enum FockMode { kNoRuns = 0, kRuns = 1, kStaged = 2 };
+
 struct ClassWork {
     const Tile* tiles = nullptr;
     long long ntiles = 0;
@@ -174,17 +188,13 @@ struct ClassWork {
     // them to X once per run
     const int2* runs = nullptr;
     long long nruns = 0;
-    // optional (with runs): the density-screened quartets compacted per
-    // segment (one bra pair, one ket group): segs[s] = {bra pair, first ket,
-    // end ket, offset}, the surviving kets of segment s at list[offset ..
-    // offset + counts[s]); runs then index segments
-    const int4* segs = nullptr;
+    // optional: the density-screened quartets, compacted: the steps written by
+    // compact_kernel, one per tile and in tile order: tiles whose kets are
+    // list[q0 .. q0 + len) (len 0: nothing survived there)
     const int* list = nullptr;
-    const int* counts = nullptr;
-    // optional (without runs): the steps written by compact_kernel, one per
-    // tile and in tile order: tiles whose kets are list[q0 .. q0 + len)
-    // (len 0: nothing survived there)
     const Tile* steps = nullptr;
+    // wavefronts sharing a tile and blocks sharing a run, log2
+    int lsplit = 0, lblocks = 0;
 };
 
 // Inputs of the per-build density compaction (compact_kernel): per pair its
@@ -197,11 +207,14 @@ struct CompactArgs {
     int nshell;
     double tau;
     int grad;   // 1: the gradient's test (one-centre skip, Y Y > tau and Y Y DNmax > tau)
-    // optional: work steps, each a bra pair and up to 64 surviving kets of one
-    // segment ({bra, list offset, count}); segment s owns the ceil(len / 64)
-    // slots from slot0[s] (the slots of its tiles), the unused ones get count 0
+    // work steps, each a bra pair and up to `chunk` surviving kets of one
+    // segment ({bra, list offset, count, distance of primitives}); segment s
+    // owns the ceil(len / chunk) slots from slot0[s] (the slots of its tiles),
+    // the unused ones get count 0
+    const int* pstride;
     Tile* steps;
     const int* slot0;
+    int chunk;
 };
 
 // FP32 copy of the kernels' primitive-pair data (same layout as DevPrims).
@@ -286,6 +299,7 @@ struct FockArgs {
     DevPrimsF ppf;  // FP32 copy for the mixed-precision kernels
     const float* Dpf;          // FP32 copy of the cons-scaled density
     const float* boys_tab;     // kBoysTabRows x kBoysTabM
+    const PairRec* rec;       // per significant pair
     const double* xyz;        // 3 x natom
     const double* Dp;         // cons-scaled density, n x n
     const double* cutmat;     // nshell x nshell, max |D| over shell blocks
@@ -304,10 +318,6 @@ struct FockArgs {
     double prim_limit;
     double hybrid;
     int boys_qshell_order;    // 1: Boys order = class L total (reference GPU)
-    // FP64 run mode: the density rows of the run's bra functions ((NA + NB) x n)
-    // staged in LDS after the bra slab, so the exchange contractions read them
-    // there instead of gathering them from memory
-    int stage_d;
 };
 
 }  // namespace qk

@@ -118,31 +118,63 @@ __device__ __forceinline__ double rsqrt_nr(double x) {
 }
 __device__ __forceinline__ float rsqrt_nr(float x) { return __builtin_amdgcn_rsqf(x); }
 
+// exp(-X), X >= 0: X = -k ln2 - r with |r| <= ln2 / 2 (ln2 in two parts, the
+// high one exact times k below 2^21), exp(r) by the degree-11 interpolant at the
+// Chebyshev nodes of the interval (largest relative error 1.7e-17), scaled by 2^k
+// (to zero beyond the range)
+__device__ __forceinline__ double exp_neg(double X) {
+    const double k = __builtin_rint(X * -1.4426950408889634);
+    const double r = fma(k, -1.9082149292705877e-10, fma(k, -0.6931471803691238, -X));
+    double p = 2.511003761756205e-08;
+    p = fma(p, r, 2.7632639654123758e-07);
+    p = fma(p, r, 2.7557240918547625e-06);
+    p = fma(p, r, 2.4801485482287731e-05);
+    p = fma(p, r, 0.00019841269890047143);
+    p = fma(p, r, 0.0013888888952314812);
+    p = fma(p, r, 0.0083333333333196011);
+    p = fma(p, r, 0.041666666666488092);
+    p = fma(p, r, 0.1666666666666668);
+    p = fma(p, r, 0.50000000000000189);
+    p = fma(p, r, 1.0);
+    p = fma(p, r, 1.0);
+    return __builtin_amdgcn_ldexp(p, int(k));
+}
+
+// QUICK's fit in two parts: the regions above T = 3e-5 (or 3e-7) without any
+// branch, so that several primitive quartets can be interleaved, and the few
+// lanes near T = 0 (centres that coincide) afterwards.
+template <int LT>
+__device__ __forceinline__ void boys_fit_main(double X, double E, const double* __restrict__ tab, double* F) {
+    const double RS = rsqrt_nr(X);           // 1/sqrt(X); 1/X as its square
+    const double XINV = RS * RS;
+    const int r = int(X > 1.0) + int(X > 3.0) + int(X > 5.0) + int(X > 10.0) + int(X > 15.0) + int(X > 33.0);
+    const double off = r == 0 ? 0.0 : (r == 1 ? 2.0 : 4.0);
+    const double z = r <= 2 ? X - off : XINV;
+    const double* c = tab + kBoysFitTerms * r;
+    double v = c[0];
+#pragma unroll
+    for (int k = 1; k < kBoysFitTerms; ++k) v = fma(v, z, c[k]);
+    const double s = 0.88622692545275801365 * RS;   // sqrt(PIE4 / X), sqrt(pi/4) = 0.886...
+    F[0] = r <= 2 ? fma(v, X + X, E) : fma(v, E, s);
+    const double h = 0.5 * XINV;
+#pragma unroll
+    for (int m = 1; m <= LT; ++m) F[m] = (double(2 * m - 1) * F[m - 1] - E) * h;
+}
+__device__ __forceinline__ bool boys_fit_up(double X, int Mb) { return (X > 3.0e-5) || (X > 3.0e-7 && Mb < 4); }
+template <int LT>
+__device__ __forceinline__ void boys_fit_near0(double X, double E, int Mb, double* F) {
+    double v = (1.0 - X) / double(2 * Mb + 1);
+    const double twot = X * 2.0;
+    for (int m = Mb - 1; m >= LT; --m) v = (twot * v + E) / double(m * 2 + 1);
+    F[LT] = v;
+#pragma unroll
+    for (int m = LT - 1; m >= 0; --m) F[m] = (twot * F[m + 1] + E) / double(m * 2 + 1);
+}
 template <int LT>
 __device__ __forceinline__ void boys_fit(double X, int Mb, const double* __restrict__ tab, double* F) {
-    const double E = exp(-X);
-    const bool up = (X > 3.0e-5) || (X > 3.0e-7 && Mb < 4);
-    if (up) {
-        const double RS = rsqrt_nr(X);           // 1/sqrt(X); 1/X as its square
-        const double XINV = RS * RS;
-        const int r = int(X > 1.0) + int(X > 3.0) + int(X > 5.0) + int(X > 10.0) + int(X > 15.0) + int(X > 33.0);
-        const double z = r == 0 ? X : (r == 1 ? X - 2.0 : (r == 2 ? X - 4.0 : XINV));
-        const double* c = tab + kBoysFitTerms * r;
-        double v = c[0];
-#pragma unroll
-        for (int k = 1; k < kBoysFitTerms; ++k) v = fma(v, z, c[k]);
-        const double s = 0.88622692545275801365 * RS;   // sqrt(PIE4 / X), sqrt(pi/4) = 0.886...
-        F[0] = r <= 2 ? fma(v, X + X, E) : fma(v, E, s);
-#pragma unroll
-        for (int m = 1; m <= LT; ++m) F[m] = (double(2 * m - 1) * F[m - 1] - E) * 0.5 * XINV;
-    } else {
-        double v = (1.0 - X) / double(2 * Mb + 1);
-        const double twot = X * 2.0;
-        for (int m = Mb - 1; m >= LT; --m) v = (twot * v + E) / double(m * 2 + 1);
-        F[LT] = v;
-#pragma unroll
-        for (int m = LT - 1; m >= 0; --m) F[m] = (twot * F[m + 1] + E) / double(m * 2 + 1);
-    }
+    const double E = exp_neg(X);
+    boys_fit_main<LT>(X, E, tab, F);
+    if (!boys_fit_up(X, Mb)) boys_fit_near0<LT>(X, E, Mb, F);
 }
 
 // Copies primitive pairs base, base + stride, ... (n <= 64 of them) into the
@@ -169,17 +201,6 @@ __device__ __forceinline__ void stage_bra(const PP& pp, int base, int stride, in
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Exchange contribution to X[row r of the bra][col]: into the block's LDS rows
-// (xr, n columns per bra function) when the block works on one bra at a time,
-// else straight into X.
-__device__ __forceinline__ void xk_add(unsigned long long* X, unsigned long long* xr, int r, int grow, int col,
-                                       int n, double v) {
-    const long long iv = __double2ll_rn(v * 0x1p48);
-    if (iv == 0) return;
-    if (xr) atomicAdd(xr + (long long)r * n + col, (unsigned long long)iv);
-    else atomicAdd(X + (long long)grow * n + col, (unsigned long long)iv);
-}
-
 __device__ __forceinline__ void fx_add(unsigned long long* X, long long idx, double v) {
     const long long iv = __double2ll_rn(v * 0x1p48);
     if (iv != 0) atomicAdd(X + idx, (unsigned long long)iv);
@@ -196,15 +217,6 @@ __device__ __forceinline__ long long fx_round_f(float v) {
     const unsigned lo = (unsigned)rintf(fabsf(a - h) * 4294967296.0f);
     const long long hi = (long long)(int)h * 4294967296LL;
     return a < 0.0f ? hi - (long long)lo : hi + (long long)lo;
-}
-
-// xk_add for an FP32 contribution
-__device__ __forceinline__ void xk_add_f(unsigned long long* X, unsigned long long* xr, int r, int grow, int col,
-                                         int n, float v) {
-    const long long iv = fx_round_f(v);
-    if (iv == 0) return;
-    if (xr) atomicAdd(xr + (long long)r * n + col, (unsigned long long)iv);
-    else atomicAdd(X + (long long)grow * n + col, (unsigned long long)iv);
 }
 
 __device__ __forceinline__ double dn_max(const double* cm, int ns, int A, int B, int C, int D) {
@@ -270,261 +282,334 @@ __device__ __forceinline__ long long wave_sum_i64(long long v) {
     return v;
 }
 
-// STAGE: run mode only (the host launches it with runs): the run's bra rows of
-// the density staged in LDS after the bra slab, the exchange contractions read
-// there; a separate instantiation, so the unstaged kernel carries no second path
-template <int LA, int LB, int LC, int LD, bool STAGE = false>
-__global__ void __launch_bounds__(256, (Occupancy<LA, LB, LC, LD>::value)) fock_kernel(const FockArgs a, const ClassWork w) {
+// ---------------------------------------------------------------------------
+// The thread-per-quartet Fock kernels: one body, in FP64 (fock_kernel) and in
+// FP32 with FP64-grade accumulation (fock_kernel_f32).
+
+// pieces that differ with the arithmetic type
+template <typename R>
+struct FockType;
+template <>
+struct FockType<double> {
+    static __device__ __forceinline__ const DevPrims& prims(const FockArgs& a) { return a.pp; }
+    static __device__ __forceinline__ const double* density(const FockArgs& a) { return a.Dp; }
+    static __device__ __forceinline__ long long fixed(double v) { return __double2ll_rn(v * 0x1p48); }
+};
+template <>
+struct FockType<float> {
+    static __device__ __forceinline__ const DevPrimsF& prims(const FockArgs& a) { return a.ppf; }
+    static __device__ __forceinline__ const float* density(const FockArgs& a) { return a.Dpf; }
+    static __device__ __forceinline__ long long fixed(float v) { return fx_round_f(v); }
+};
+
+// What a lane needs of a ket beyond its pair record, gathered ahead: the five
+// shell-block density maxima of its screen, the centre C, its first primitive
+template <typename R>
+struct KetGather {
+    double cd, ad, ac, bd, bc;
+    double Cx, Cy, Cz;
+    R z, o, x, y, zz, K, c;
+};
+
+// A wavefront takes tiles (a bra pair, up to 64 kets of one group, one per
+// lane) t0, t0 + step, ... < t1.  Two thirds of its cycles used to go to waiting
+// for memory: a tile's ket list, the kets' pair arrays, their Qshells' arrays,
+// the density maxima and centres, and the primitives were five dependent
+// round trips.  A pair's data now sits in one 32-byte record, and the next
+// tiles are fetched while one is evaluated: the tile after next, the next tile's
+// kets, and their records at the top; their screens, centres and first
+// primitives between the primitive loop and the digestion.  With that, and with
+// the density reads of a quartet's digestion issued together, the FP64 build of
+// (H2O)32 went from 31.8 to 27.0 ms, the mixed one at 1e-3 from 21.3 to 18.3 ms,
+// the B3LYP build of (H2O)64 from 142 to 114 ms.
+//
+// In run mode (kRuns) a block takes the tiles of one bra pair: the exchange
+// contributions to the bra's rows of X are summed in LDS (NA + NB rows of n)
+// and added to X once per run, the bra's primitives sit in one LDS slab, and
+// its Coulomb block is summed in registers (small blocks) over the run.
+// kStaged: run mode with the run's bra rows of the density in LDS after the slab,
+// the exchange contractions read there.
+// Where a class has too few tiles to fill the GPU, 2^w.lsplit wavefronts share a
+// tile in run mode, each taking a part of its primitive quartets, and 2^w.lblocks
+// blocks a run (share_tiles): everything after the primitive loop is linear in
+// the integrals, so each wavefront digests its own partial sums (one water: 2.39 ->
+// 0.54 ms for the build).
+template <int LA, int LB, int LC, int LD, typename R, int MODE, class Boys>
+__device__ __forceinline__ void fock_quartets(const FockArgs& a, const ClassWork& w, const Boys& boys) {
     constexpr int NE = nrange(LA, LA + LB), NF = nrange(LC, LC + LD);
     constexpr int NACC = NE * NF;
     constexpr int NA = ncart(LA), NB = ncart(LB), NC = ncart(LC), ND = ncart(LD);
     constexpr int NOUT = NA * NB * NC * ND;
     constexpr int LT = LA + LB + LC + LD;
-    const double X0 = 34.98683665524972;  // 2 pi^(5/2), quick_constants_module.f90:55
-    const int n = a.n;
+    constexpr bool RUNS = MODE != kNoRuns, STAGE = MODE == kStaged;
+    constexpr bool kKeepJ = RUNS && NA * NB <= 9;   // the run's Coulomb block in registers
+    constexpr bool kCentreC = LC + LD > 0;
+    using Ft = FockType<R>;
+    const R X0 = R(34.98683665524972);  // 2 pi^(5/2), quick_constants_module.f90:55
+    const int n = a.n, ns = a.nshell;
     const int lane = threadIdx.x & 63;
     unsigned long long* const Xc = a.X + (long long)(blockIdx.x % a.xcopies) * n * n;
-    const long long wave0 = __builtin_amdgcn_readfirstlane(((long long)blockIdx.x * blockDim.x + threadIdx.x) >> 6);
-    const long long nwaves = ((long long)gridDim.x * blockDim.x) >> 6;
-    unsigned long long nsurv = 0, nprimq = 0;
-    __shared__ double s_boys[kBoysFitRegions * kBoysFitTerms];
-    for (int k = threadIdx.x; k < kBoysFitRegions * kBoysFitTerms; k += blockDim.x) s_boys[k] = kBoysFit[k];
-    __syncthreads();
-    // one tile per wavefront and iteration: a bra pair shared by all lanes and
-    // one ket pair per lane; every lane reaches the reduction below
+    const int wib = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    unsigned nsurv = 0, nprimq = 0;
+    const auto& pp = Ft::prims(a);
+    const R* __restrict__ Dp = Ft::density(a);
+    const R plim = R(a.prim_limit);
+    const int lsplit = RUNS ? w.lsplit : 0;
+
     // dynamic LDS: in run mode the exchange rows of the run's bra, then that
     // bra's primitive pairs (at most 64; one slab for the block, staged once per
     // run); otherwise one slab per wavefront, staged per tile
     extern __shared__ unsigned long long s_xrows[];
-    const bool runs = w.runs != nullptr;
-    unsigned long long* const xr = runs ? s_xrows : nullptr;
-    const int wib = threadIdx.x >> 6;
-    double* const bra = runs ? reinterpret_cast<double*>(s_xrows + (NA + NB) * n)
-                             : reinterpret_cast<double*>(s_xrows) + wib * (7 * 64);
-    double* const sD = STAGE ? bra + 7 * 64 : nullptr;   // the run's bra rows of D
-    const bool compact = runs && w.segs != nullptr;
-    int c_seg = 0, c_end = 0, c_step = 0, c_nst = -1, c_gt = 0;   // compacted-run walk
-    long long run = blockIdx.x;
-    for (;;) {
+    R* const bra = RUNS ? reinterpret_cast<R*>(s_xrows + (NA + NB) * n)
+                        : reinterpret_cast<R*>(s_xrows) + wib * (7 * 64);
+    R* const sD = STAGE ? bra + 7 * 64 : nullptr;   // the run's bra rows of D
+    const Tile* const tiles = w.steps ? w.steps : w.tiles;
+    const bool listed = w.steps != nullptr;
+
+    for (long long run = blockIdx.x;; run += gridDim.x) {
     long long t0, t1, tstep;
-    int rp = 0;
-    if (runs) {
-        if (run >= w.nruns) break;
-        const int2 rg = w.runs[run];
-        t0 = rg.x + wib; t1 = rg.y; tstep = 4;
-        rp = compact ? w.segs[rg.x].x : w.tiles[rg.x].p;
-        c_seg = rg.x; c_end = rg.y; c_step = 0; c_nst = -1; c_gt = 0;
+    int p = 0;
+    if constexpr (RUNS) {
+        if ((run >> w.lblocks) >= w.nruns) break;
+        const int2 rg = w.runs[run >> w.lblocks];
+        tstep = 4ll << w.lblocks;
+        t0 = ((long long)rg.x << lsplit) + ((run * 4 + wib) & (tstep - 1)); t1 = (long long)rg.y << lsplit;
+        p = w.tiles[rg.x].p;
+    } else {
+        t0 = (long long)blockIdx.x * 4 + wib; t1 = w.ntiles; tstep = (long long)gridDim.x * 4;
+    }
+    auto tile_at = [&](long long t) { return t < t1 ? tiles[t >> lsplit] : Tile{0, 0, 0, 0}; };
+    auto ket_of = [&](const Tile& tl) { return lane < tl.len ? (listed ? w.list[tl.q0 + lane] : tl.q0 + lane) : 0; };
+    Tile T0 = tile_at(t0), T1 = tile_at(t0 + tstep), T2 = tile_at(t0 + 2 * tstep);
+    int q0 = ket_of(T0), q1 = ket_of(T1);
+    PairRec r0 = a.rec[q0];
+    if constexpr (RUNS) {
         for (int k = threadIdx.x; k < (NA + NB) * n; k += blockDim.x) s_xrows[k] = 0ull;
-        if (wib == 0) stage_bra(a.pp, a.pr.prim0[rp], a.pr.pstride[rp], a.pr.nprim[rp], lane, bra);
+        if (wib == 0) stage_bra(pp, a.pr.prim0[p], a.pr.pstride[p], a.pr.nprim[p], lane, bra);
         if constexpr (STAGE) {
-            const int fa0 = a.q.f0[a.pr.qa[rp]], fb0 = a.q.f0[a.pr.qb[rp]];
+            const unsigned f = a.rec[p].f01;
+            const int fa0 = f & 0xffff, fb0 = f >> 16;
             for (int k = threadIdx.x; k < (NA + NB) * n; k += blockDim.x) {
                 const int r = k / n, col = k - r * n;
-                sD[k] = a.Dp[(long long)(r < NA ? fa0 + r : fb0 + r - NA) * n + col];
+                sD[k] = Dp[(long long)(r < NA ? fa0 + r : fb0 + r - NA) * n + col];
             }
         }
         __syncthreads();
-    } else {
-        t0 = wave0; t1 = w.ntiles; tstep = nwaves;
     }
-    for (long long t = t0;; t += tstep) {
-        int p, q;
-        bool inrange;
-        if (compact) {
-            // the run's segments in steps of 64 surviving kets; step g of the
-            // run goes to wavefront g % 4 (all of this is wavefront-uniform)
-            bool found = false;
-            while (c_seg < c_end) {
-                if (c_nst < 0) c_nst = (w.counts[c_seg] + 63) >> 6;
-                if (c_step < c_nst) {
-                    const bool mine = (c_gt & 3) == wib;
-                    ++c_gt;
-                    if (mine) { found = true; break; }
-                    ++c_step;
-                    continue;
-                }
-                ++c_seg; c_step = 0; c_nst = -1;
+    // a wavefront's share of a tile: bra primitives si, si + 2^lsi, ..., ket
+    // primitives sj, sj + 2^(lsplit - lsi), ...; the bra's are split first
+    int lsi = 0;
+    if constexpr (RUNS)
+        while (lsi < lsplit && (1 << lsi) < int((a.rec[p].misc >> 8) & 0x7f)) ++lsi;
+    auto share_i = [&](long long t) { return int(t) & ((1 << lsi) - 1); };
+    auto share_j = [&](long long t) { return (int(t) & ((1 << lsplit) - 1)) >> lsi; };
+    // gathers of a ket's density maxima, centre and first primitive (of the share)
+    auto gather = [&](const Tile& tl, const PairRec& r, const unsigned shb, int first) {
+        KetGather<R> g;
+        const unsigned sC = r.sh & 0xffff, sD_ = r.sh >> 16;
+        const double* ca = a.cutmat + (long long)(shb & 0xffff) * ns;
+        const double* cb = a.cutmat + (long long)(shb >> 16) * ns;
+        g.cd = a.cutmat[(long long)sC * ns + sD_];
+        g.ad = ca[sD_]; g.ac = ca[sC]; g.bd = cb[sD_]; g.bc = cb[sC];
+        if constexpr (kCentreC) {
+            const int at = r.at & 0xffff;
+            g.Cx = a.xyz[3 * at]; g.Cy = a.xyz[3 * at + 1]; g.Cz = a.xyz[3 * at + 2];
+        }
+        // (a lane without a ket holds pair 0, whose primitives lie otherwise)
+        const int k = r.prim0 + (lane < tl.len && first < int((r.misc >> 8) & 0x7f) ? first * tl.pad : 0);
+        g.z = pp.zeta[k]; g.o = pp.oo2z[k]; g.x = pp.Px[k]; g.y = pp.Py[k]; g.zz = pp.Pz[k];
+        g.K = pp.K[k]; g.c = pp.cut[k];
+        return g;
+    };
+    KetGather<R> g0 = gather(T0, r0, a.rec[RUNS ? p : T0.p].sh, share_j(t0));
+    long long jac[NA * NB];
+#pragma unroll
+    for (int k = 0; k < NA * NB; ++k) jac[k] = 0;
+    // J on the bra block, in fixed point and so summed exactly across the
+    // wavefront (all lanes share the bra pair): one atomic per element
+    auto flush_j = [&](const PairRec& rb, int pb) {
+        const int fb = rb.f01 >> 16;
+#pragma unroll
+        for (int k = 0; k < NA * NB; ++k) {
+            const long long v = wave_sum_i64(jac[k]);
+            jac[k] = 0;
+            if (lane == 0 && v != 0) {
+                if constexpr (RUNS) atomicAdd(s_xrows + (k / NB) * n + fb + k % NB, (unsigned long long)v);
+                else atomicAdd(a.J + rb.jofs + (long long)k * a.pr.pstride[pb], (unsigned long long)v);
             }
-            if (!found) break;
-            const int4 sg = w.segs[c_seg];
-            const int idx = c_step * 64 + lane;
-            p = __builtin_amdgcn_readfirstlane(sg.x);
-            inrange = idx < w.counts[c_seg];
-            q = inrange ? w.list[sg.w + idx] : 0;
-            ++c_step;
-        } else {
-            if (t >= t1) break;
-            const Tile tl = w.tiles[t];
-            p = __builtin_amdgcn_readfirstlane(tl.p);
-            q = tl.q0 + lane;
-            inrange = lane < tl.len;
         }
-
-        const int qa = a.pr.qa[p], qb = a.pr.qb[p];
-        const int qc = inrange ? a.pr.qa[q] : 0, qd = inrange ? a.pr.qb[q] : 0;
-        bool active = false;
-        double dn = 0.0;
-        if (inrange) {
-            const int sA = a.q.shell[qa], sB = a.q.shell[qb], sC = a.q.shell[qc], sD = a.q.shell[qd];
-            dn = dn_max(a.cutmat, a.nshell, sA, sB, sC, sD);
-            active = a.pr.Y[q] * a.pr.Y[p] * dn > a.tau;
-        }
-        const int fa = a.q.f0[qa], fb = a.q.f0[qb];
-        const double* Dp = a.Dp;
-        double jab[NA * NB];
+    };
+    for (long long t = t0; t < t1; t += tstep) {
+        if constexpr (!RUNS) p = __builtin_amdgcn_readfirstlane(T0.p);
+        const PairRec rb = a.rec[p];
+        const PairRec r1 = a.rec[q1];
+        const int q2 = ket_of(T2);
+        const Tile T3 = tile_at(t + 3 * tstep);
+        const int fa = rb.f01 & 0xffff, fb = rb.f01 >> 16;
+        const int nbp = (rb.misc >> 8) & 0x7f;
+        if constexpr (!RUNS) stage_bra(pp, rb.prim0, a.pr.pstride[p], nbp, lane, bra);   // run mode: staged for the run
+        const double dn =
+            fmax(fmax(4.0 * a.cutmat[(long long)(rb.sh & 0xffff) * ns + (rb.sh >> 16)], 4.0 * g0.cd),
+                 fmax(fmax(g0.ad, g0.ac), fmax(g0.bc, g0.bd)));
+        const bool active = lane < T0.len && r0.Y * rb.Y * dn > a.tau;
+        R acc[NACC];
 #pragma unroll
-        for (int k = 0; k < NA * NB; ++k) jab[k] = 0.0;
-
-        const int pb0 = a.pr.prim0[p], pbs = a.pr.pstride[p], nbp = a.pr.nprim[p];
-        if (!runs) stage_bra(a.pp, pb0, pbs, nbp, lane, bra);   // run mode: p is the run's bra, staged
-
+        for (int k = 0; k < NACC; ++k) acc[k] = R(0);
+        const int pks = T0.pad;   // distance of the ket group's consecutive primitives
         if (active) {
-            ++nsurv;
-            const int Mb = a.boys_qshell_order ? LT : a.q.qfinal[qa] + a.q.qfinal[qb] + a.q.qfinal[qc] + a.q.qfinal[qd];
-            const int atA = a.q.atom[qa], atB = a.q.atom[qb], atC = a.q.atom[qc], atD = a.q.atom[qd];
-            const double Ax = a.xyz[3 * atA], Ay = a.xyz[3 * atA + 1], Az = a.xyz[3 * atA + 2];
-            const double Cx = a.xyz[3 * atC], Cy = a.xyz[3 * atC + 1], Cz = a.xyz[3 * atC + 2];
-
-            double acc[NACC];
+            nsurv += (t & ((1 << lsplit) - 1)) == 0;
+            const int Mb = a.boys_qshell_order ? LT : int(rb.misc & 15u) + int(r0.misc & 15u);
+            const int atA = rb.at & 0xffff;
+            const R Ax = R(a.xyz[3 * atA]), Ay = R(a.xyz[3 * atA + 1]), Az = R(a.xyz[3 * atA + 2]);
+            const R Cx = kCentreC ? R(g0.Cx) : R(0), Cy = kCentreC ? R(g0.Cy) : R(0), Cz = kCentreC ? R(g0.Cz) : R(0);
+            const R dnr = R(dn);
+            const int pk0 = r0.prim0, nkp = (r0.misc >> 8) & 0x7f;
+            // one primitive quartet: bra primitive i (from the slab) with the ket
+            // primitive's data
+            auto prims = [&](int i, R zcd, R oo2e, R Qx, R Qy, R Qz, R Kcd, R ccd, R QCx, R QCy, R QCz) {
+                if (!((dnr * bra[6 * 64 + i]) * ccd > plim)) return;
+                ++nprimq;
+                const R zab = bra[i], oo2z = bra[64 + i];
+                const R Px = bra[2 * 64 + i], Py = bra[3 * 64 + i], Pz = bra[4 * 64 + i];
+                const R rs = rsqrt_nr(zab + zcd);   // 1/sqrt(zeta+eta): reciprocal and root in one
+                const R inv = rs * rs;
+                const R ROU = zab * (zcd * inv);
+                const R Wx = (Px * zab + Qx * zcd) * inv;
+                const R Wy = (Py * zab + Qy * zcd) * inv;
+                const R Wz = (Pz * zab + Qz * zcd) * inv;
+                const R dx = Px - Qx, dy = Py - Qy, dz = Pz - Qz;
+                const R T = (dx * dx + dy * dy + dz * dz) * ROU;
+                R F[LT + 1];
+                const typename Boys::State bs = boys.main(T, F);
+                boys.rare(T, Mb, bs, F);
+                const R s = X0 * bra[5 * 64 + i] * Kcd * rs;
 #pragma unroll
-            for (int k = 0; k < NACC; ++k) acc[k] = 0.0;
-
+                for (int m = 0; m <= LT; ++m) F[m] *= s;
+                ClassOps<LA, LB, LC, LD>::template vrr<R>(F, Px - Ax, Py - Ay, Pz - Az, Wx - Px, Wy - Py, Wz - Pz, QCx,
+                                                          QCy, QCz, Wx - Qx, Wy - Qy, Wz - Qz, oo2z, oo2e, R(0.5) * inv,
+                                                          zcd * inv, zab * inv, acc);
+            };
             // kets outer (vector loads; the next ket primitive is fetched while the
             // current one runs), bra primitives inner, read from the bra slab in LDS
             // (the same address on every lane: broadcast reads)
-            const int pk0 = a.pr.prim0[q], pks = a.pr.pstride[q], nkp = a.pr.nprim[q];
-            {
-                const int ni = nbp;   // <= 64 primitive pairs per Qshell pair (checked on the host)
-                double nz = a.pp.zeta[pk0], no = a.pp.oo2z[pk0], nx = a.pp.Px[pk0], ny = a.pp.Py[pk0],
-                       nzz = a.pp.Pz[pk0], nK = a.pp.K[pk0], nc = a.pp.cut[pk0];
-                for (int j = 0; j < nkp; ++j) {
-                    const double zcd = nz, oo2e = no, Qx = nx, Qy = ny, Qz = nzz, Kcd = nK, ccd = nc;
-                    if (j + 1 < nkp) {
-                        const int kn = pk0 + (j + 1) * pks;
-                        nz = a.pp.zeta[kn]; no = a.pp.oo2z[kn]; nx = a.pp.Px[kn]; ny = a.pp.Py[kn];
-                        nzz = a.pp.Pz[kn]; nK = a.pp.K[kn]; nc = a.pp.cut[kn];
-                    }
-                    const double QCx = Qx - Cx, QCy = Qy - Cy, QCz = Qz - Cz;
-                    // two bra primitives interleaved where it measured faster
-                    // ((ss|ss): 4.24 -> 3.74 ms on (H2O)32; the five-unit classes ~5%)
-                    constexpr int kUnroll = (LT == 0 || LT == 5) ? 2 : 1;
-#pragma unroll kUnroll
-                    for (int i = 0; i < ni; ++i) {
-                        if (!((dn * bra[6 * 64 + i]) * ccd > a.prim_limit)) continue;
-                        ++nprimq;
-                        const double zab = bra[i], oo2z = bra[64 + i];
-                        const double Px = bra[2 * 64 + i], Py = bra[3 * 64 + i], Pz = bra[4 * 64 + i];
-                        const double rs = rsqrt_nr(zab + zcd);   // 1/sqrt(zeta+eta): reciprocal and root in one
-                        const double inv = rs * rs;
-                        const double roz = zcd * inv, roe = zab * inv;
-                        const double ROU = zab * roz;
-                        const double Wx = (Px * zab + Qx * zcd) * inv;
-                        const double Wy = (Py * zab + Qy * zcd) * inv;
-                        const double Wz = (Pz * zab + Qz * zcd) * inv;
-                        const double dx = Px - Qx, dy = Py - Qy, dz = Pz - Qz;
-                        const double T = (dx * dx + dy * dy + dz * dz) * ROU;
-                        double F[LT + 1];
-                        boys_fit<LT>(T, Mb, s_boys, F);
-                        const double s = X0 * bra[5 * 64 + i] * Kcd * rs;
-#pragma unroll
-                        for (int m = 0; m <= LT; ++m) F[m] *= s;
-                        ClassOps<LA, LB, LC, LD>::template vrr<double>(
-                            F, Px - Ax, Py - Ay, Pz - Az, Wx - Px, Wy - Py, Wz - Pz, QCx, QCy, QCz,
-                            Wx - Qx, Wy - Qy, Wz - Qz, oo2z, oo2e, 0.5 * inv, roz, roe, acc);
-                    }
+            R nz = g0.z, no = g0.o, nx = g0.x, ny = g0.y, nzz = g0.zz, nK = g0.K, nc = g0.c;
+            const int si = share_i(t), SI = 1 << lsi, SJ = 1 << (lsplit - lsi);
+            for (int j = share_j(t); j < nkp; j += SJ) {
+                const R zcd = nz, oo2e = no, Qx = nx, Qy = ny, Qz = nzz, Kcd = nK, ccd = nc;
+                if (j + SJ < nkp) {
+                    const int kn = pk0 + (j + SJ) * pks;
+                    nz = pp.zeta[kn]; no = pp.oo2z[kn]; nx = pp.Px[kn]; ny = pp.Py[kn];
+                    nzz = pp.Pz[kn]; nK = pp.K[kn]; nc = pp.cut[kn];
                 }
+                const R QCx = Qx - Cx, QCy = Qy - Cy, QCz = Qz - Cz;
+                for (int i = si; i < nbp; i += SI) prims(i, zcd, oo2e, Qx, Qy, Qz, Kcd, ccd, QCx, QCy, QCz);
             }
-
-            double out[NOUT];
+        }
+        const KetGather<R> g1 = gather(T1, r1, RUNS ? rb.sh : a.rec[T1.p].sh, share_j(t + tstep));
+        if (active) {
+            const int atA = rb.at & 0xffff, atB = rb.at >> 16, atD = r0.at >> 16;
+            R out[NOUT];
             {
-                const double Bx = a.xyz[3 * atB], By = a.xyz[3 * atB + 1], Bz = a.xyz[3 * atB + 2];
-                const double Dx = a.xyz[3 * atD], Dy = a.xyz[3 * atD + 1], Dz = a.xyz[3 * atD + 2];
-                ClassOps<LA, LB, LC, LD>::template hrr<double>(acc, Ax - Bx, Ay - By, Az - Bz, Cx - Dx, Cy - Dy,
-                                                               Cz - Dz, out);
+                const R Ax = R(a.xyz[3 * atA]), Ay = R(a.xyz[3 * atA + 1]), Az = R(a.xyz[3 * atA + 2]);
+                const R Bx = R(a.xyz[3 * atB]), By = R(a.xyz[3 * atB + 1]), Bz = R(a.xyz[3 * atB + 2]);
+                R CDx = R(0), CDy = R(0), CDz = R(0);
+                if constexpr (kCentreC) {
+                    CDx = R(g0.Cx) - R(a.xyz[3 * atD]);
+                    CDy = R(g0.Cy) - R(a.xyz[3 * atD + 1]);
+                    CDz = R(g0.Cz) - R(a.xyz[3 * atD + 2]);
+                }
+                ClassOps<LA, LB, LC, LD>::template hrr<R>(acc, Ax - Bx, Ay - By, Az - Bz, CDx, CDy, CDz, out);
             }
-
             // digestion: G = (X + X^T)/2 with X accumulating
             //   X[a][b] += 4w D[c][d] I,  X[c][d] += 4w D[a][b] I,
             //   X[a][c] -= h w D[b][d] I, X[a][d] -= h w D[b][c] I,
             //   X[b][c] -= h w D[a][d] I, X[b][d] -= h w D[a][c] I
             // w = 1/((1+[qa==qb])(1+[qc==qd])(1+[p==q])) is the share of the quartet's
             // 8-fold orbit this component set represents.
-            const int fc = a.q.f0[qc], fd = a.q.f0[qd];
-            double wgt = 1.0;
-            if (qa == qb) wgt *= 0.5;
-            if (qc == qd) wgt *= 0.5;
-            if (p == q) wgt *= 0.5;
-            const double jw = 4.0 * wgt, kw = -a.hybrid * wgt;
+            const int fc = r0.f01 & 0xffff, fd = r0.f01 >> 16;
+            R wgt = R(1);
+            if (rb.misc & 16u) wgt *= R(0.5);
+            if (r0.misc & 16u) wgt *= R(0.5);
+            if (p == q0) wgt *= R(0.5);
+            const R jw = R(4) * wgt, kw = -R(a.hybrid) * wgt;
+            // element (row, col) of the density; n <= 65535, so the index fits 32 bits
+            auto DG = [&](int row, int col) { return Dp[unsigned(row) * unsigned(n) + unsigned(col)]; };
 #define OUT(ia, ib, ic, id) out[(((ia)*NB + (ib)) * NC + (ic)) * ND + (id)]
+            if (a.hybrid != 0.0) {
+                // exchange: the bra rows of D from LDS (staged per run) or from memory,
+                // the sums into the block's LDS rows or straight into X.  No branch
+                // between them: the density reads of all of them go out together (a
+                // test for zero at each one made every sum wait for its own reads)
+                auto B = [&](int r, int grow, int col) {
+                    if constexpr (STAGE) return sD[r * n + col];
+                    else return DG(grow, col);
+                };
+                auto put = [&](int r, int grow, int col, R s) {
+                    const long long iv = Ft::fixed(kw * s);
+                    if constexpr (RUNS) atomicAdd(s_xrows + r * n + col, (unsigned long long)iv);
+                    else if (iv != 0) atomicAdd(Xc + (long long)grow * n + col, (unsigned long long)iv);
+                };
+                for (int ia = 0; ia < NA; ++ia)
+                    for (int ic = 0; ic < NC; ++ic) {
+                        R s = R(0);
+                        for (int ib = 0; ib < NB; ++ib)
+                            for (int id = 0; id < ND; ++id) s += B(NA + ib, fb + ib, fd + id) * OUT(ia, ib, ic, id);
+                        put(ia, fa + ia, fc + ic, s);
+                    }
+                for (int ia = 0; ia < NA; ++ia)
+                    for (int id = 0; id < ND; ++id) {
+                        R s = R(0);
+                        for (int ib = 0; ib < NB; ++ib)
+                            for (int ic = 0; ic < NC; ++ic) s += B(NA + ib, fb + ib, fc + ic) * OUT(ia, ib, ic, id);
+                        put(ia, fa + ia, fd + id, s);
+                    }
+                for (int ib = 0; ib < NB; ++ib)
+                    for (int ic = 0; ic < NC; ++ic) {
+                        R s = R(0);
+                        for (int ia = 0; ia < NA; ++ia)
+                            for (int id = 0; id < ND; ++id) s += B(ia, fa + ia, fd + id) * OUT(ia, ib, ic, id);
+                        put(NA + ib, fb + ib, fc + ic, s);
+                    }
+                for (int ib = 0; ib < NB; ++ib)
+                    for (int id = 0; id < ND; ++id) {
+                        R s = R(0);
+                        for (int ia = 0; ia < NA; ++ia)
+                            for (int ic = 0; ic < NC; ++ic) s += B(ia, fa + ia, fc + ic) * OUT(ia, ib, ic, id);
+                        put(NA + ib, fb + ib, fd + id, s);
+                    }
+            }
             for (int ia = 0; ia < NA; ++ia)
                 for (int ib = 0; ib < NB; ++ib) {
-                    double s = 0.0;
+                    R s = R(0);
                     for (int ic = 0; ic < NC; ++ic)
-                        for (int id = 0; id < ND; ++id) s += Dp[(long long)(fc + ic) * n + fd + id] * OUT(ia, ib, ic, id);
-                    jab[ia * NB + ib] = jw * s;
+                        for (int id = 0; id < ND; ++id) s += DG(fc + ic, fd + id) * OUT(ia, ib, ic, id);
+                    jac[ia * NB + ib] += Ft::fixed(jw * s);
                 }
+            long long vj[NC * ND];
             for (int ic = 0; ic < NC; ++ic)
                 for (int id = 0; id < ND; ++id) {
-                    double s = 0.0;
+                    R s = R(0);
                     for (int ia = 0; ia < NA; ++ia)
-                        for (int ib = 0; ib < NB; ++ib) s += Dp[(long long)(fa + ia) * n + fb + ib] * OUT(ia, ib, ic, id);
-                    fx_add(a.J, a.jofs[q] + (long long)(ic * ND + id) * pks, jw * s);
+                        for (int ib = 0; ib < NB; ++ib) s += DG(fa + ia, fb + ib) * OUT(ia, ib, ic, id);
+                    vj[ic * ND + id] = Ft::fixed(jw * s);
                 }
-            if (a.hybrid != 0.0) {
-                // exchange: the bra rows of D from LDS (staged per run) or from memory
-                auto exch = [&](auto DG) {
-                    for (int ia = 0; ia < NA; ++ia)
-                        for (int ic = 0; ic < NC; ++ic) {
-                            double s = 0.0;
-                            for (int ib = 0; ib < NB; ++ib)
-                                for (int id = 0; id < ND; ++id) s += DG(NA + ib, fb + ib, fd + id) * OUT(ia, ib, ic, id);
-                            xk_add(Xc, xr, ia, fa + ia, fc + ic, n, (kw * s));
-                        }
-                    for (int ia = 0; ia < NA; ++ia)
-                        for (int id = 0; id < ND; ++id) {
-                            double s = 0.0;
-                            for (int ib = 0; ib < NB; ++ib)
-                                for (int ic = 0; ic < NC; ++ic) s += DG(NA + ib, fb + ib, fc + ic) * OUT(ia, ib, ic, id);
-                            xk_add(Xc, xr, ia, fa + ia, fd + id, n, (kw * s));
-                        }
-                    for (int ib = 0; ib < NB; ++ib)
-                        for (int ic = 0; ic < NC; ++ic) {
-                            double s = 0.0;
-                            for (int ia = 0; ia < NA; ++ia)
-                                for (int id = 0; id < ND; ++id) s += DG(ia, fa + ia, fd + id) * OUT(ia, ib, ic, id);
-                            xk_add(Xc, xr, NA + ib, fb + ib, fc + ic, n, (kw * s));
-                        }
-                    for (int ib = 0; ib < NB; ++ib)
-                        for (int id = 0; id < ND; ++id) {
-                            double s = 0.0;
-                            for (int ia = 0; ia < NA; ++ia)
-                                for (int ic = 0; ic < NC; ++ic) s += DG(ia, fa + ia, fc + ic) * OUT(ia, ib, ic, id);
-                            xk_add(Xc, xr, NA + ib, fb + ib, fd + id, n, (kw * s));
-                        }
-                };
-                if constexpr (STAGE) exch([&](int r, int, int col) { return sD[r * n + col]; });
-                else exch([&](int, int grow, int col) { return Dp[(long long)grow * n + col]; });
-            }
+            for (int k = 0; k < NC * ND; ++k)
+                if (vj[k] != 0) atomicAdd(a.J + r0.jofs + (long long)k * pks, (unsigned long long)vj[k]);
 #undef OUT
         }
-
-        // J on the bra block: converted to fixed point per lane and summed across
-        // the wavefront (all lanes share the bra pair): one atomic per element
-        // instead of up to 64.
-#pragma unroll
-        for (int k = 0; k < NA * NB; ++k) {
-            const long long v = wave_sum_i64(__double2ll_rn(jab[k] * 0x1p48));
-            if (lane == 0 && v != 0) {
-                if (xr) atomicAdd(xr + (long long)(k / NB) * n + fb + k % NB, (unsigned long long)v);
-                else atomicAdd(a.J + a.jofs[p] + (long long)k * pbs, (unsigned long long)v);
-            }
-        }
+        if constexpr (!kKeepJ) flush_j(rb, p);
+        T0 = T1; T1 = T2; T2 = T3;
+        q0 = q1; q1 = q2;
+        r0 = r1;
+        g0 = g1;
     }
-    if (!runs) break;
+    if constexpr (!RUNS) break;
+    if constexpr (kKeepJ) flush_j(a.rec[p], p);
     // add the run's rows to X once
     __syncthreads();
     {
-        const int fa0 = a.q.f0[a.pr.qa[rp]], fb0 = a.q.f0[a.pr.qb[rp]];
+        const unsigned f = a.rec[p].f01;
+        const int fa0 = f & 0xffff, fb0 = f >> 16;
         for (int k = threadIdx.x; k < (NA + NB) * n; k += blockDim.x) {
             const unsigned long long v = s_xrows[k];
             if (v == 0ull) continue;
@@ -534,10 +619,32 @@ __global__ void __launch_bounds__(256, (Occupancy<LA, LB, LC, LD>::value)) fock_
         }
     }
     __syncthreads();
-    run += gridDim.x;
     }
-    if (nsurv) atomicAdd(a.counters + 0, nsurv);
-    if (nprimq) atomicAdd(a.counters + 1, nprimq);
+    if (nsurv) atomicAdd(a.counters + 0, (unsigned long long)nsurv);
+    if (nprimq) atomicAdd(a.counters + 1, (unsigned long long)nprimq);
+}
+
+// the two parts of QUICK's fit, with the coefficients in LDS (kernel below)
+template <int LT>
+struct BoysFit {
+    using State = double;   // exp(-T)
+    const double* tab;
+    __device__ __forceinline__ double main(double T, double* F) const {
+        const double E = exp_neg(T);
+        boys_fit_main<LT>(T, E, tab, F);
+        return E;
+    }
+    __device__ __forceinline__ void rare(double T, int Mb, double E, double* F) const {
+        if (!boys_fit_up(T, Mb)) boys_fit_near0<LT>(T, E, Mb, F);
+    }
+};
+
+template <int LA, int LB, int LC, int LD, int MODE>
+__global__ void __launch_bounds__(256, (Occupancy<LA, LB, LC, LD>::value)) fock_kernel(const FockArgs a, const ClassWork w) {
+    __shared__ double s_boys[kBoysFitRegions * kBoysFitTerms];
+    for (int k = threadIdx.x; k < kBoysFitRegions * kBoysFitTerms; k += blockDim.x) s_boys[k] = kBoysFit[k];
+    __syncthreads();
+    fock_quartets<LA, LB, LC, LD, double, MODE>(a, w, BoysFit<LA + LB + LC + LD>{s_boys});
 }
 
 // ---------------------------------------------------------------------------
@@ -568,25 +675,30 @@ __device__ __forceinline__ void stage_boys_f32(const float* __restrict__ tab, fl
 // grid point 0, rows kStride apart (the LDS slice: kBoysLdsCols; the table in
 // memory: a.boys_tab + LT and kBoysTabM)
 template <int LT, int kStride = kBoysLdsCols>
+__device__ __forceinline__ void boys_f32_main(float T, const float* tab, float* F) {
+    const int k = __float2int_rn(fminf(T, kBoysTabTmax) * float(kBoysTabPerUnit));
+    const float d = float(k) * (1.0f / float(kBoysTabPerUnit)) - T;
+    const float* r = tab + k * kStride;
+    // F_LT(T) = sum_j F_{LT+j}(T_k) d^j / j!,  d = T_k - T, |d| <= 1/16
+    F[LT] = (((r[4] * (d * 0.25f) + r[3]) * (d * (1.0f / 3.0f)) + r[2]) * (d * 0.5f) + r[1]) * d + r[0];
+    const float e = __expf(-T);
+    const float t2 = T + T;
+#pragma unroll
+    for (int m = LT - 1; m >= 0; --m) F[m] = (t2 * F[m + 1] + e) * (1.0f / float(2 * m + 1));
+}
+// T >= kBoysTabTmax: sqrt(pi / 4T) by the hardware reciprocal square root
+// (no denormal or zero operand here)
+template <int LT>
+__device__ __forceinline__ void boys_f32_far(float T, float* F) {
+    F[0] = 0.88622692545275801f * __builtin_amdgcn_rsqf(T);
+    const float h = 0.5f * __builtin_amdgcn_rcpf(T);
+#pragma unroll
+    for (int m = 1; m <= LT; ++m) F[m] = F[m - 1] * (float(2 * m - 1) * h);
+}
+template <int LT, int kStride = kBoysLdsCols>
 __device__ __forceinline__ void boys_f32(float T, const float* tab, float* F) {
-    if (T < kBoysTabTmax) {
-        const int k = __float2int_rn(T * float(kBoysTabPerUnit));
-        const float d = float(k) * (1.0f / float(kBoysTabPerUnit)) - T;
-        const float* r = tab + k * kStride;
-        // F_LT(T) = sum_j F_{LT+j}(T_k) d^j / j!,  d = T_k - T, |d| <= 1/16
-        F[LT] = (((r[4] * (d * 0.25f) + r[3]) * (d * (1.0f / 3.0f)) + r[2]) * (d * 0.5f) + r[1]) * d + r[0];
-        const float e = __expf(-T);
-        const float t2 = T + T;
-#pragma unroll
-        for (int m = LT - 1; m >= 0; --m) F[m] = (t2 * F[m + 1] + e) * (1.0f / float(2 * m + 1));
-    } else {
-        // T >= kBoysTabTmax: sqrt(pi / 4T) by the hardware reciprocal square root
-        // (no denormal or zero operand here)
-        F[0] = 0.88622692545275801f * __builtin_amdgcn_rsqf(T);
-        const float h = 0.5f * __builtin_amdgcn_rcpf(T);
-#pragma unroll
-        for (int m = 1; m <= LT; ++m) F[m] = F[m - 1] * (float(2 * m - 1) * h);
-    }
+    boys_f32_main<LT, kStride>(T, tab, F);
+    if (!(T < kBoysTabTmax)) boys_f32_far<LT>(T, F);
 }
 
 // the primitive-pair data, exponents and density in the kernel's precision
@@ -635,240 +747,31 @@ struct OccupancyF {
     static constexpr int value = nacc <= 36 ? (rows >= 6 ? 3 : 4) : 2;
 };
 
-template <int LA, int LB, int LC, int LD>
+// the tabulated expansion (kStride: the LDS slice or the table in memory)
+template <int LT, int kStride>
+struct BoysTab {
+    struct State {};
+    const float* tab;
+    __device__ __forceinline__ State main(float T, float* F) const {
+        boys_f32_main<LT, kStride>(T, tab, F);
+        return {};
+    }
+    __device__ __forceinline__ void rare(float T, int, State, float* F) const {
+        if (!(T < kBoysTabTmax)) boys_f32_far<LT>(T, F);
+    }
+};
+
+template <int LA, int LB, int LC, int LD, int MODE>
 __global__ void __launch_bounds__(256, (OccupancyF<LA, LB, LC, LD>::value)) fock_kernel_f32(const FockArgs a, const ClassWork w) {
-    constexpr int NE = nrange(LA, LA + LB), NF = nrange(LC, LC + LD);
-    constexpr int NACC = NE * NF;
-    constexpr int NA = ncart(LA), NB = ncart(LB), NC = ncart(LC), ND = ncart(LD);
-    constexpr int NOUT = NA * NB * NC * ND;
     constexpr int LT = LA + LB + LC + LD;
-    const float X0 = 34.98683665524972f;
-    const int n = a.n;
-    const int lane = threadIdx.x & 63;
-    unsigned long long* const Xc = a.X + (long long)(blockIdx.x % a.xcopies) * n * n;
-    const long long wave0 = __builtin_amdgcn_readfirstlane(((long long)blockIdx.x * blockDim.x + threadIdx.x) >> 6);
-    const long long nwaves = ((long long)gridDim.x * blockDim.x) >> 6;
-    unsigned long long nsurv = 0, nprimq = 0;
-    const float plim = float(a.prim_limit);
-    constexpr bool kBoysLds = NA + NB <= 4;   // two or four exchange rows
+    constexpr bool kBoysLds = ncart(LA) + ncart(LB) <= 4;   // two or four exchange rows
     __shared__ float s_btab[kBoysLds ? kBoysTabRows * kBoysLdsCols : 1];
     if constexpr (kBoysLds) {
         stage_boys_f32<LT>(a.boys_tab, s_btab);
         __syncthreads();
     }
-
-    // dynamic LDS: in run mode the exchange rows of the run's bra, then that
-    // bra's primitive pairs (one slab for the block, staged once per run);
-    // otherwise one slab per wavefront, staged per tile
-    extern __shared__ unsigned long long s_xrows[];
-    const bool runs = w.runs != nullptr;
-    unsigned long long* const xr = runs ? s_xrows : nullptr;
-    const int wib = threadIdx.x >> 6;
-    float* const bra = runs ? reinterpret_cast<float*>(s_xrows + (NA + NB) * n)
-                            : reinterpret_cast<float*>(s_xrows) + wib * (7 * 64);
-    const bool compact = runs && w.segs != nullptr;
-    int c_seg = 0, c_end = 0, c_step = 0, c_nst = -1, c_gt = 0;   // compacted-run walk
-    long long run = blockIdx.x;
-    for (;;) {
-    long long t0, t1, tstep;
-    int rp = 0;
-    if (runs) {
-        if (run >= w.nruns) break;
-        const int2 rg = w.runs[run];
-        t0 = rg.x + wib; t1 = rg.y; tstep = 4;
-        rp = compact ? w.segs[rg.x].x : w.tiles[rg.x].p;
-        c_seg = rg.x; c_end = rg.y; c_step = 0; c_nst = -1; c_gt = 0;
-        for (int k = threadIdx.x; k < (NA + NB) * n; k += blockDim.x) s_xrows[k] = 0ull;
-        if (wib == 0) stage_bra(a.ppf, a.pr.prim0[rp], a.pr.pstride[rp], a.pr.nprim[rp], lane, bra);
-        __syncthreads();
-    } else {
-        t0 = wave0; t1 = w.ntiles; tstep = nwaves;
-    }
-    for (long long t = t0;; t += tstep) {
-        int p, q;
-        bool inrange;
-        if (compact) {
-            // the run's segments in steps of 64 surviving kets; step g of the
-            // run goes to wavefront g % 4 (all of this is wavefront-uniform)
-            bool found = false;
-            while (c_seg < c_end) {
-                if (c_nst < 0) c_nst = (w.counts[c_seg] + 63) >> 6;
-                if (c_step < c_nst) {
-                    const bool mine = (c_gt & 3) == wib;
-                    ++c_gt;
-                    if (mine) { found = true; break; }
-                    ++c_step;
-                    continue;
-                }
-                ++c_seg; c_step = 0; c_nst = -1;
-            }
-            if (!found) break;
-            const int4 sg = w.segs[c_seg];
-            const int idx = c_step * 64 + lane;
-            p = __builtin_amdgcn_readfirstlane(sg.x);
-            inrange = idx < w.counts[c_seg];
-            q = inrange ? w.list[sg.w + idx] : 0;
-            ++c_step;
-        } else {
-            if (t >= t1) break;
-            const Tile tl = w.tiles[t];
-            p = __builtin_amdgcn_readfirstlane(tl.p);
-            q = tl.q0 + lane;
-            inrange = lane < tl.len;
-        }
-        const int qa = a.pr.qa[p], qb = a.pr.qb[p];
-        const int qc = inrange ? a.pr.qa[q] : 0, qd = inrange ? a.pr.qb[q] : 0;
-        bool active = false;
-        double dn = 0.0;
-        if (inrange) {
-            const int sA = a.q.shell[qa], sB = a.q.shell[qb], sC = a.q.shell[qc], sD = a.q.shell[qd];
-            dn = dn_max(a.cutmat, a.nshell, sA, sB, sC, sD);
-            active = a.pr.Y[q] * a.pr.Y[p] * dn > a.tau;
-        }
-        const int fa = a.q.f0[qa], fb = a.q.f0[qb];
-        const float* Dp = a.Dpf;
-        float jab[NA * NB];
-#pragma unroll
-        for (int k = 0; k < NA * NB; ++k) jab[k] = 0.0f;
-        const int pb0 = a.pr.prim0[p], pbs = a.pr.pstride[p], nbp = a.pr.nprim[p];
-        if (!runs) stage_bra(a.ppf, pb0, pbs, nbp, lane, bra);   // run mode: p is the run's bra, staged
-
-        if (active) {
-            ++nsurv;
-            const int atA = a.q.atom[qa], atB = a.q.atom[qb], atC = a.q.atom[qc], atD = a.q.atom[qd];
-            const float Ax = float(a.xyz[3 * atA]), Ay = float(a.xyz[3 * atA + 1]), Az = float(a.xyz[3 * atA + 2]);
-            const float Cx = float(a.xyz[3 * atC]), Cy = float(a.xyz[3 * atC + 1]), Cz = float(a.xyz[3 * atC + 2]);
-            float acc[NACC];
-#pragma unroll
-            for (int k = 0; k < NACC; ++k) acc[k] = 0.0f;
-            const int pk0 = a.pr.prim0[q], pks = a.pr.pstride[q], nkp = a.pr.nprim[q];
-            const float dnf = float(dn);
-            {
-                const int ni = nbp;   // <= 64 primitive pairs per Qshell pair (checked on the host)
-                float nz = a.ppf.zeta[pk0], no = a.ppf.oo2z[pk0], nx = a.ppf.Px[pk0], ny = a.ppf.Py[pk0],
-                      nzz = a.ppf.Pz[pk0], nK = a.ppf.K[pk0], nc = a.ppf.cut[pk0];
-                for (int j = 0; j < nkp; ++j) {
-                    const float zcd = nz, oo2e = no, Qx = nx, Qy = ny, Qz = nzz, Kcd = nK, ccd = nc;
-                    if (j + 1 < nkp) {
-                        const int kn = pk0 + (j + 1) * pks;
-                        nz = a.ppf.zeta[kn]; no = a.ppf.oo2z[kn]; nx = a.ppf.Px[kn]; ny = a.ppf.Py[kn];
-                        nzz = a.ppf.Pz[kn]; nK = a.ppf.K[kn]; nc = a.ppf.cut[kn];
-                    }
-                    const float QCx = Qx - Cx, QCy = Qy - Cy, QCz = Qz - Cz;
-                    for (int i = 0; i < ni; ++i) {
-                        if (!((dnf * bra[6 * 64 + i]) * ccd > plim)) continue;
-                        ++nprimq;
-                        const float zab = bra[i], oo2z = bra[64 + i];
-                        const float Px = bra[2 * 64 + i], Py = bra[3 * 64 + i], Pz = bra[4 * 64 + i];
-                        const float rs = rsqrt_nr(zab + zcd);
-                        const float inv = rs * rs;
-                        const float roz = zcd * inv, roe = zab * inv;
-                        const float ROU = zab * roz;
-                        const float Wx = (Px * zab + Qx * zcd) * inv;
-                        const float Wy = (Py * zab + Qy * zcd) * inv;
-                        const float Wz = (Pz * zab + Qz * zcd) * inv;
-                        const float dx = Px - Qx, dy = Py - Qy, dz = Pz - Qz;
-                        const float T = (dx * dx + dy * dy + dz * dz) * ROU;
-                        float F[LT + 1];
-                        if constexpr (kBoysLds) boys_f32<LT>(T, s_btab, F);
-                        else boys_f32<LT, kBoysTabM>(T, a.boys_tab + LT, F);
-                        const float s = X0 * bra[5 * 64 + i] * Kcd * rs;
-#pragma unroll
-                        for (int m = 0; m <= LT; ++m) F[m] *= s;
-                        ClassOps<LA, LB, LC, LD>::template vrr<float>(
-                            F, Px - Ax, Py - Ay, Pz - Az, Wx - Px, Wy - Py, Wz - Pz, QCx, QCy, QCz,
-                            Wx - Qx, Wy - Qy, Wz - Qz, oo2z, oo2e, 0.5f * inv, roz, roe, acc);
-                    }
-                }
-            }
-            float out[NOUT];
-            {
-                const float Bx = float(a.xyz[3 * atB]), By = float(a.xyz[3 * atB + 1]), Bz = float(a.xyz[3 * atB + 2]);
-                const float Dx = float(a.xyz[3 * atD]), Dy = float(a.xyz[3 * atD + 1]), Dz = float(a.xyz[3 * atD + 2]);
-                ClassOps<LA, LB, LC, LD>::template hrr<float>(acc, Ax - Bx, Ay - By, Az - Bz, Cx - Dx, Cy - Dy,
-                                                              Cz - Dz, out);
-            }
-            // digestion as in fock_kernel, in FP32, promoted to FP64 at the accumulate
-            const int fc = a.q.f0[qc], fd = a.q.f0[qd];
-            float wgt = 1.0f;
-            if (qa == qb) wgt *= 0.5f;
-            if (qc == qd) wgt *= 0.5f;
-            if (p == q) wgt *= 0.5f;
-            const float jw = 4.0f * wgt, kw = -float(a.hybrid) * wgt;
-#define OUT(ia, ib, ic, id) out[(((ia)*NB + (ib)) * NC + (ic)) * ND + (id)]
-            for (int ia = 0; ia < NA; ++ia)
-                for (int ib = 0; ib < NB; ++ib) {
-                    float s = 0.0f;
-                    for (int ic = 0; ic < NC; ++ic)
-                        for (int id = 0; id < ND; ++id) s += Dp[(long long)(fc + ic) * n + fd + id] * OUT(ia, ib, ic, id);
-                    jab[ia * NB + ib] = jw * s;
-                }
-            for (int ic = 0; ic < NC; ++ic)
-                for (int id = 0; id < ND; ++id) {
-                    float s = 0.0f;
-                    for (int ia = 0; ia < NA; ++ia)
-                        for (int ib = 0; ib < NB; ++ib) s += Dp[(long long)(fa + ia) * n + fb + ib] * OUT(ia, ib, ic, id);
-                    fx_add_f(a.J, a.jofs[q] + (long long)(ic * ND + id) * pks, jw * s);
-                }
-            if (a.hybrid != 0.0) {
-                for (int ia = 0; ia < NA; ++ia)
-                    for (int ic = 0; ic < NC; ++ic) {
-                        float s = 0.0f;
-                        for (int ib = 0; ib < NB; ++ib)
-                            for (int id = 0; id < ND; ++id) s += Dp[(long long)(fb + ib) * n + fd + id] * OUT(ia, ib, ic, id);
-                        xk_add_f(Xc, xr, ia, fa + ia, fc + ic, n, kw * s);
-                    }
-                for (int ia = 0; ia < NA; ++ia)
-                    for (int id = 0; id < ND; ++id) {
-                        float s = 0.0f;
-                        for (int ib = 0; ib < NB; ++ib)
-                            for (int ic = 0; ic < NC; ++ic) s += Dp[(long long)(fb + ib) * n + fc + ic] * OUT(ia, ib, ic, id);
-                        xk_add_f(Xc, xr, ia, fa + ia, fd + id, n, kw * s);
-                    }
-                for (int ib = 0; ib < NB; ++ib)
-                    for (int ic = 0; ic < NC; ++ic) {
-                        float s = 0.0f;
-                        for (int ia = 0; ia < NA; ++ia)
-                            for (int id = 0; id < ND; ++id) s += Dp[(long long)(fa + ia) * n + fd + id] * OUT(ia, ib, ic, id);
-                        xk_add_f(Xc, xr, NA + ib, fb + ib, fc + ic, n, kw * s);
-                    }
-                for (int ib = 0; ib < NB; ++ib)
-                    for (int id = 0; id < ND; ++id) {
-                        float s = 0.0f;
-                        for (int ia = 0; ia < NA; ++ia)
-                            for (int ic = 0; ic < NC; ++ic) s += Dp[(long long)(fa + ia) * n + fc + ic] * OUT(ia, ib, ic, id);
-                        xk_add_f(Xc, xr, NA + ib, fb + ib, fd + id, n, kw * s);
-                    }
-            }
-#undef OUT
-        }
-#pragma unroll
-        for (int k = 0; k < NA * NB; ++k) {
-            const long long v = wave_sum_i64(fx_round_f(jab[k]));
-            if (lane == 0 && v != 0) {
-                if (xr) atomicAdd(xr + (long long)(k / NB) * n + fb + k % NB, (unsigned long long)v);
-                else atomicAdd(a.J + a.jofs[p] + (long long)k * pbs, (unsigned long long)v);
-            }
-        }
-    }
-    if (!runs) break;
-    // add the run's rows to X once
-    __syncthreads();
-    {
-        const int fa0 = a.q.f0[a.pr.qa[rp]], fb0 = a.q.f0[a.pr.qb[rp]];
-        for (int k = threadIdx.x; k < (NA + NB) * n; k += blockDim.x) {
-            const unsigned long long v = s_xrows[k];
-            if (v == 0ull) continue;
-            const int r = k / n, col = k - r * n;
-            const int grow = r < NA ? fa0 + r : fb0 + (r - NA);
-            atomicAdd(Xc + (long long)grow * n + col, v);
-        }
-    }
-    __syncthreads();
-    run += gridDim.x;
-    }
-    if (nsurv) atomicAdd(a.counters + 0, nsurv);
-    if (nprimq) atomicAdd(a.counters + 1, nprimq);
+    constexpr int kStride = kBoysLds ? kBoysLdsCols : kBoysTabM;
+    fock_quartets<LA, LB, LC, LD, float, MODE>(a, w, BoysTab<LT, kStride>{kBoysLds ? s_btab : a.boys_tab + LT});
 }
 
 // ---------------------------------------------------------------------------

@@ -12,7 +12,7 @@
 // split at Y_ij * Y_kl >= fp32_threshold; exclusive scans over the items give
 // every item its place in the class's tile, segment and candidate lists; a
 // second pass writes them.  For the Fock build one thread per bra pair then
-// cuts the bra's tiles and segments into runs of at most `cap` candidate kets.
+// cuts the bra's tiles into runs of at most `cap` candidate kets.
 // The lists are those of a sequential walk over (bra group, bra, ket group)
 // (Fock) or (bra group, ket group, bra) (gradient), element for element.
 #include <hipcub/hipcub.hpp>
@@ -86,9 +86,8 @@ __global__ void list_count_kernel(const ListEntry* __restrict__ E, int ne, const
         long long v[kListCounts];
         v[0] = ceil_div(c64, C.chunk);
         v[1] = ceil_div(c32, C.chunk);
-        if (!C.segs) v[2] = v[3] = 0;
-        else if (C.grad) { v[2] = c64 > 0; v[3] = c32 > 0; }
-        else { v[2] = ceil_div(c64, C.cap64); v[3] = ceil_div(c32, C.cap32); }
+        v[2] = C.segs ? ceil_div(c64, C.cap64) : 0;
+        v[3] = C.segs ? ceil_div(c32, C.cap32) : 0;
         v[4] = c64;
         v[5] = c32;
         for (int a = 0; a < kListCounts; ++a) cnt[a * (N + 1) + it] = v[a];
@@ -115,7 +114,7 @@ __global__ void list_write_kernel(const ListEntry* __restrict__ E, int ne, const
         const ListClass C = LC[k];
         const long long r = it - E[e].item0;
         const int i = (int)(r / E[e].m), t = (int)(r - (long long)i * E[e].m);
-        const int p = E[e].s1 + i, s2 = KG[E[e].kg0 + t].s2;
+        const int p = E[e].s1 + i, s2 = KG[E[e].kg0 + t].s2, n2 = KG[E[e].kg0 + t].n2;
         const int4 x = items[it];
         const int qb = x.x, lo = x.y, lo64 = x.z;
         const long long c0 = cls_item[k];
@@ -123,43 +122,34 @@ __global__ void list_write_kernel(const ListEntry* __restrict__ E, int ne, const
         for (int a = 0; a < kListCounts; ++a) o[a] = off[a * (N + 1) + it] - off[a * (N + 1) + c0];
         const ListDst D = dst[k];
         long long j = o[0];
-        for (int q = qb; q < lo64; q += C.chunk) D.t64[j++] = Tile{p, s2 + q, min(C.chunk, lo64 - q), 0};
+        for (int q = qb; q < lo64; q += C.chunk) D.t64[j++] = Tile{p, s2 + q, min(C.chunk, lo64 - q), n2};
         j = o[1];
-        for (int q = lo64; q < lo; q += C.chunk) D.t32[j++] = Tile{p, s2 + q, min(C.chunk, lo - q), 0};
+        for (int q = lo64; q < lo; q += C.chunk) D.t32[j++] = Tile{p, s2 + q, min(C.chunk, lo - q), n2};
         if (!C.segs) continue;
-        if (C.grad) {
-            if (lo64 > qb) {
-                D.s64[o[2]] = make_int4(p, s2 + qb, s2 + lo64, (int)o[4]);
-                D.slot64[o[2]] = (int)o[0];
-            }
-            if (lo > lo64) {
-                D.s32[o[3]] = make_int4(p, s2 + lo64, s2 + lo, (int)o[5]);
-                D.slot32[o[3]] = (int)o[1];
-            }
-        } else {
-            j = o[2];
-            long long c = o[4];
-            for (int q = qb; q < lo64;) {
-                const int en = lo64 - q > C.cap64 ? q + C.cap64 : lo64;
-                D.s64[j++] = make_int4(p, s2 + q, s2 + en, (int)c);
-                c += en - q;
-                q = en;
-            }
-            j = o[3];
-            c = o[5];
-            for (int q = lo64; q < lo;) {
-                const int en = lo - q > C.cap32 ? q + C.cap32 : lo;
-                D.s32[j++] = make_int4(p, s2 + q, s2 + en, (int)c);
-                c += en - q;
-                q = en;
-            }
+        j = o[2];
+        long long c = o[4];
+        for (int q = qb; q < lo64;) {
+            const int en = lo64 - q > C.cap64 ? q + C.cap64 : lo64;
+            D.s64[j] = make_int4(p, s2 + q, s2 + en, (int)c);
+            D.slot64[j++] = (int)o[0] + (q - qb) / C.chunk;   // caps are multiples of chunk
+            c += en - q;
+            q = en;
+        }
+        j = o[3];
+        c = o[5];
+        for (int q = lo64; q < lo;) {
+            const int en = lo - q > C.cap32 ? q + C.cap32 : lo;
+            D.s32[j] = make_int4(p, s2 + q, s2 + en, (int)c);
+            D.slot32[j++] = (int)o[1] + (q - lo64) / C.chunk;
+            c += en - q;
+            q = en;
         }
     }
 }
 
-// Greedy runs over one bra's pieces (tiles of `chunk` kets, or segments of
-// `cap` kets) in list order: a run ends before a piece that would take its
-// candidates past cap.  emit(first, end) gets piece indices relative to `base`.
+// Greedy runs over one bra's tiles (`piece` kets each) in list order: a run
+// ends before a tile that would take its candidates past cap.  emit(first, end)
+// gets tile indices relative to the bra's first.
 template <class Emit>
 __device__ __forceinline__ long long bra_runs(const ListEntry& E, const int4* items, int i, bool fp32, int piece,
                                               int cap, Emit&& emit) {
@@ -185,7 +175,7 @@ __device__ __forceinline__ long long bra_runs(const ListEntry& E, const int4* it
     return nrun;
 }
 
-// per bra pair of the Fock lists: runs of FP64 / FP32 tiles and segments
+// per bra pair of the Fock lists: runs of FP64 / FP32 tiles
 __global__ void list_runs_kernel(const ListEntry* __restrict__ E, int ne, const ListClass* __restrict__ LC,
                                  long long NB, const int4* __restrict__ items, const long long* __restrict__ off,
                                  long long N, const long long* __restrict__ cls_item, const long long* __restrict__ roff,
@@ -211,8 +201,6 @@ __global__ void list_runs_kernel(const ListEntry* __restrict__ E, int ne, const 
             auto none = [](long long, long long) {};
             rcnt[0 * (NB + 1) + b] = bra_runs(E[e], items, i, false, C.chunk, C.cap64, none);
             rcnt[1 * (NB + 1) + b] = bra_runs(E[e], items, i, true, C.chunk, C.cap32, none);
-            rcnt[2 * (NB + 1) + b] = C.segs ? bra_runs(E[e], items, i, false, C.cap64, C.cap64, none) : 0;
-            rcnt[3 * (NB + 1) + b] = C.segs ? bra_runs(E[e], items, i, true, C.cap32, C.cap32, none) : 0;
             continue;
         }
         // writing pass: pieces numbered from the bra's first item's list offsets
@@ -220,14 +208,11 @@ __global__ void list_runs_kernel(const ListEntry* __restrict__ E, int ne, const 
         const ListDst D = dst[k];
         const long long c0 = cls_item[k], b0 = cls_bra[k];
         for (int a = 0; a < kRunCounts; ++a) {
-            if (a >= 2 && !C.segs) break;
             const long long base = off[a * (N + 1) + it0] - off[a * (N + 1) + c0];
             long long j = roff[a * (NB + 1) + b] - roff[a * (NB + 1) + b0];
-            int2* out = a == 0 ? D.r64 : a == 1 ? D.r32 : a == 2 ? D.sr64 : D.sr32;
+            int2* out = a == 0 ? D.r64 : D.r32;
             auto put = [&](long long f, long long en) { out[j++] = make_int2((int)(base + f), (int)(base + en)); };
-            const bool fp32 = a & 1;
-            const int piece = a < 2 ? C.chunk : (fp32 ? C.cap32 : C.cap64);
-            bra_runs(E[e], items, i, fp32, piece, fp32 ? C.cap32 : C.cap64, put);
+            bra_runs(E[e], items, i, a == 1, C.chunk, a == 1 ? C.cap32 : C.cap64, put);
         }
     }
 }
