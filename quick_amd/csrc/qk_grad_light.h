@@ -141,8 +141,13 @@ __global__ void __launch_bounds__(256, (GradFold<LA, LB, LC, LD, R>::type::kWave
     // tiles' places, each a bra pair and up to 64 surviving kets in w.list;
     // otherwise tiles of a bra pair and consecutive kets
     const bool compact = w.steps != nullptr;
-    for (long long t = wave0; t < w.ntiles; t += nwaves) {
-        const Tile tl = compact ? w.steps[t] : w.tiles[t];
+    // 2^w.lsplit wavefronts share a tile where tiles are few, each taking a part of
+    // its primitive quartets: the derivatives are linear in them (one water: 2.28 ->
+    // 0.76 ms)
+    const int lsplit = w.lsplit;
+    for (long long t = wave0; t < w.ntiles << lsplit; t += nwaves) {
+        const Tile tl = compact ? w.steps[t >> lsplit] : w.tiles[t >> lsplit];
+        const int share = int(t) & ((1 << lsplit) - 1);
         if (tl.len == 0) continue;   // wavefront-uniform: no survivor in this slot
         const int p = __builtin_amdgcn_readfirstlane(tl.p);
         const bool inrange = lane < tl.len;
@@ -161,7 +166,11 @@ __global__ void __launch_bounds__(256, (GradFold<LA, LB, LC, LD, R>::type::kWave
         const int pb0 = a.pr.prim0[p], pbs = a.pr.pstride[p], nbp = a.pr.nprim[p];
         stage_bra_grad<R>(a, pb0, pbs, nbp, lane, bra);
         if (!active) continue;
-        ++nsurv;
+        nsurv += share == 0;
+        // the bra's primitives are split first, then the ket's
+        int lsi = 0;
+        while (lsi < lsplit && (1 << lsi) < nbp) ++lsi;
+        const int si = share & ((1 << lsi) - 1), sj = share >> lsi, SI = 1 << lsi, SJ = 1 << (lsplit - lsi);
         const int Mb = a.q.qfinal[qa] + a.q.qfinal[qb] + a.q.qfinal[qc] + a.q.qfinal[qd] + 2;
         const R Ax = R(a.xyz[3 * atA]), Ay = R(a.xyz[3 * atA + 1]), Az = R(a.xyz[3 * atA + 2]);
         const R Cx = R(a.xyz[3 * atC]), Cy = R(a.xyz[3 * atC + 1]), Cz = R(a.xyz[3 * atC + 2]);
@@ -214,7 +223,7 @@ __global__ void __launch_bounds__(256, (GradFold<LA, LB, LC, LD, R>::type::kWave
                 Fd::template fold<K, R>(Dab, Dcd, Dac, Dbd, Dad, Dbc, ABx, ABy, ABz, CDx, CDy, CDz, W);
             });
             const int ni = nbp;   // <= 64 primitive pairs per Qshell pair (checked on the host)
-            for (int j = 0; j < nkp; ++j) {
+            for (int j = sj; j < nkp; j += SJ) {
                 const int kj = pk0 + j * pks;
                 const R zcd = PP.zeta[kj], oo2e = PP.oo2z[kj];
                 const R Qx = PP.Px[kj], Qy = PP.Py[kj], Qz = PP.Pz[kj];
@@ -223,7 +232,7 @@ __global__ void __launch_bounds__(256, (GradFold<LA, LB, LC, LD, R>::type::kWave
                 const R ge = R(2) * ec * oo2e;                       // gamma / eta
                 const R d2 = R(-2) * (zcd - ec);                     // -2 delta
                 const R d2x = d2 * CDx, d2y = d2 * CDy, d2z = d2 * CDz;
-                for (int i = 0; i < ni; ++i) {
+                for (int i = si; i < ni; i += SI) {
                     if (!((rdn * bra[6 * 64 + i]) * ccd > rcut)) continue;
                     if (K == 0) ++nprimq;
                     const R zab = bra[i], oo2z = bra[64 + i];

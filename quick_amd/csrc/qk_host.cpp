@@ -277,6 +277,7 @@ struct qk_ctx {
     DBuf<Tile> d_gsteps[2][kNumQuartetClasses];
     DBuf<int> d_gslot0[2][kNumQuartetClasses];
     DBuf<int> d_glist[2][kNumQuartetClasses];
+    int glsplit[2][kNumQuartetClasses] = {};   // wavefronts per tile, log2 (share_tiles)
     double grad_prep_cutoff = -1, grad_prep_thr = -1;
     int grad_prep_precision = -1;
     bool grad_prepared = false;
@@ -636,7 +637,7 @@ using ListSumsFn = std::function<int(const std::vector<long long>&, std::vector<
 // one after another (up to 1,296 of them, 0.4 us each in FP64), so where a class
 // has too few tiles to fill the GPU the longest chain is the kernel's time; there
 // each tile's primitives are split over wavefronts that would be idle (one water:
-// Fock build 2.39 -> 0.54 ms).  2,048 wavefronts (two
+// Fock build 2.39 -> 0.54 ms, gradient 2.28 -> 0.76 ms).  2,048 wavefronts (two
 // per SIMD) are taken as full: above that a share only repeats the quartet's
 // screening and digestion.
 constexpr long long kSplitTiles = 2048;
@@ -1604,6 +1605,7 @@ static int grad_prepare(qk_ctx* c, const qk_opts* o) {
         }
     }
     cls_item[kNumQuartetClasses] = nitem;
+    const std::vector<int> most = most_primitives(c);
     const ListSumsFn grad_dst = [&](const std::vector<long long>& sm, std::vector<ListDst>& dst) -> int {
         for (int k = 0; k < kNumQuartetClasses; ++k) {
             const long long* v = &sm[(size_t)k * kListCounts];
@@ -1615,6 +1617,7 @@ static int grad_prepare(qk_ctx* c, const qk_opts* o) {
             c->ngtiles32[k] = v[1];
             c->ngsegs[0][k] = v[2];
             c->ngsegs[1][k] = v[3];
+            for (int f = 0; f < 2; ++f) c->glsplit[f][k] = grad_class_is_light(k) ? share_tiles(v[f], most[k]) : 0;
         }
         // every class's lists in one allocation
         Arena& A = c->grad_arena;
@@ -1767,7 +1770,8 @@ static int grad_enqueue(qk_ctx* c, const double* dD, const double* dcutmat_or_nu
             a.counters = c->d_gcounters.p + 2 * (fp32 ? kNumQuartetClasses + k : k);
             const int slot = (fp32 ? 3 : 2) * kNumQuartetClasses + k;
             if (c->timing) HIPCHK(hipEventRecord(c->ev_t0[slot], ls));
-            if (grad_class_is_light(k) && grad_compacts(k, fp32, mixed)) {
+            w.lsplit = c->glsplit[fp32 ? 1 : 0][k];
+            if (grad_class_is_light(k) && w.lsplit == 0 && grad_compacts(k, fp32, mixed)) {
                 // density compaction, then the kernel over the queued steps
                 const int f = fp32 ? 1 : 0;
                 CompactArgs cq = ca;
@@ -1776,13 +1780,13 @@ static int grad_enqueue(qk_ctx* c, const double* dD, const double* dcutmat_or_nu
                 launch_compact(cq, c->d_gsegs[f][k].p, c->ngsegs[f][k], c->d_glist[f][k].p, ls);
                 w.list = c->d_glist[f][k].p;
                 w.steps = cq.steps;
-                const int grid = (int)std::min<long long>((nt + 3) / 4, 256LL * 8);
+                const int grid = (int)std::min<long long>(((nt << w.lsplit) + 3) / 4, 256LL * 8);
                 if (launch_grad_light(k, a, w, grid, fp32, ls)) {
                     set_err("gradient kernel launch failed for class %d", k);
                     return -1;
                 }
             } else if (grad_class_is_light(k)) {
-                const int grid = (int)std::min<long long>((nt + 3) / 4, 256LL * 8);
+                const int grid = (int)std::min<long long>(((nt << w.lsplit) + 3) / 4, 256LL * 8);
                 if (launch_grad_light(k, a, w, grid, fp32, ls)) {
                     set_err("gradient kernel launch failed for class %d", k);
                     return -1;
