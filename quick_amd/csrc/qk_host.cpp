@@ -43,10 +43,8 @@ void launch_density_cutoff(const double* D, const int* sh_f0, const int* sh_nf, 
                            hipStream_t s);
 void launch_fill_u64(unsigned long long* p, long long count, hipStream_t s);
 void launch_compact(const CompactArgs& a, const int4* segs, long long nsegs, int* list, hipStream_t s);
-void launch_oneint(const OneFuncs& f, const OneSys& sys, const int2* const* pairs, const long long* npairs, double* S,
-                   double* H, hipStream_t s);
-void launch_oneint_grad(const OneFuncs& f, const OneSys& sys, const int2* const* pairs, const long long* npairs,
-                        const double* D, const double* W,
+void launch_oneint(const OneFuncs& f, const OneSys& sys, const OnePairs* w, double* S, double* H, hipStream_t s);
+void launch_oneint_grad(const OneFuncs& f, const OneSys& sys, const OnePairs* w, const double* D, const double* W,
                         unsigned long long* G, hipStream_t s);
 void launch_jpair_scatter(const unsigned long long* J, const int* jofs, const int* pstride, const int* qa,
                           const int* qb, const DevQshells& q, int npair, unsigned long long* X, int n,
@@ -315,10 +313,11 @@ struct qk_ctx {
     // one-electron integrals: per basis function its atom, (l, m, n), primitive
     // count, shell Qfinal, exponents and coefficients (10 per function), and
     // the nuclear charges (qk_set_charges)
-    DBuf<int> d1_atom, d1_lmn, d1_np, d1_qf;
+    DBuf<int> d1_atom, d1_fn, d1_np, d1_qf;
     // function pairs mu <= nu by total angular momentum l(mu) + l(nu) (0..4)
-    DBuf<int2> d1_pairs[5];
-    long long n1_pairs[5] = {};
+    DBuf<int2> d1_pairs[kNumPairClasses];
+    OnePairs n1_pairs[kNumPairClasses] = {};
+    bool n1_whole = false, n1_cover = false;   // shells hold each component once; every function in a shell
     DBuf<double> d1_a, d1_c, d_chg;
     std::vector<double> chg;
     DBuf<unsigned long long> d1_acc;
@@ -566,7 +565,8 @@ extern "C" int qk_set_system(qk_ctx* c, int natom, const double* xyz, int nshell
         // per basis function, for the one-electron integrals: the shell's
         // exponents and the coefficients QUICK's attrashell applies,
         // gccoeff(k, ksumtype + L) cons(f) (nuclear.f90:196-221)
-        std::vector<int> fat(nbasis), flmn(nbasis), fnp(nbasis), fqf(nbasis);
+        std::vector<int> fat(nbasis), ffn(nbasis, -1), fnp(nbasis), fqf(nbasis);
+        c->n1_whole = true;
         std::vector<double> fa(10 * (size_t)nbasis, 0.0), fc(10 * (size_t)nbasis, 0.0);
         for (size_t q = 0; q < c->q_L.size(); ++q) {
             const int sh = c->q_shell[q], L = c->q_L[q];
@@ -574,7 +574,13 @@ extern "C" int qk_set_system(qk_ctx* c, int natom, const double* xyz, int nshell
             for (int i = 0; i < ncart_of(L); ++i) {
                 const int fn = c->q_f0[q] + i;
                 fat[fn] = katom[sh] - 1;
-                flmn[fn] = KLMN[3 * fn] | (KLMN[3 * fn + 1] << 4) | (KLMN[3 * fn + 2] << 8);
+                // its component: x powers falling, then y powers falling
+                const int x = KLMN[3 * fn], y = KLMN[3 * fn + 1], z = KLMN[3 * fn + 2];
+                if (x + y + z > 2) { set_err("one-electron integrals: functions above d"); return -1; }
+                const bool ok = x >= 0 && y >= 0 && z >= 0 && x + y + z == L;
+                int* slot = ok ? &ffn[c->q_f0[q] + (L - x) * (L - x + 1) / 2 + z] : nullptr;
+                if (slot && *slot < 0) *slot = fn;
+                else c->n1_whole = false;
                 fnp[fn] = kprim[sh];
                 fqf[fn] = Qfinal[sh];
                 for (int u = 0; u < kprim[sh]; ++u) {
@@ -583,21 +589,26 @@ extern "C" int qk_set_system(qk_ctx* c, int natom, const double* xyz, int nshell
                 }
             }
         }
-        if (c->d1_atom.upload(fat) || c->d1_lmn.upload(flmn) || c->d1_np.upload(fnp) || c->d1_qf.upload(fqf) ||
+        if (c->d1_atom.upload(fat) || c->d1_fn.upload(ffn) || c->d1_np.upload(fnp) || c->d1_qf.upload(fqf) ||
             c->d1_a.upload(fa) || c->d1_c.upload(fc))
             return -1;
-        std::vector<int> fl(nbasis);
-        for (int fn = 0; fn < nbasis; ++fn) fl[fn] = KLMN[3 * fn] + KLMN[3 * fn + 1] + KLMN[3 * fn + 2];
-        std::vector<int2> pl[5];
-        for (int nu = 0; nu < nbasis; ++nu)
-            for (int mu = 0; mu <= nu; ++mu) {
-                const int L = fl[mu] + fl[nu];
-                if (L > 4) { set_err("one-electron integrals: functions above d"); return -1; }
-                pl[L].push_back(make_int2(mu, nu));
+        c->n1_cover = std::find(ffn.begin(), ffn.end(), -1) == ffn.end();
+        std::vector<int2> pl[kNumPairClasses][kOneBuckets];
+        const int nq = (int)c->q_L.size();
+        for (int i = 0; i < nq; ++i)
+            for (int j = i; j < nq; ++j) {
+                const int a = c->q_L[i] >= c->q_L[j] ? i : j, b = i + j - a;
+                const int npp = kprim[c->q_shell[a]] * kprim[c->q_shell[b]];
+                pl[pair_class_of(c->q_L[a], c->q_L[b])][one_bucket(npp)].push_back(make_int2(c->q_f0[a], c->q_f0[b]));
             }
-        for (int L = 0; L < 5; ++L) {
-            if (c->d1_pairs[L].upload(pl[L])) return -1;
-            c->n1_pairs[L] = (long long)pl[L].size();
+        for (int k = 0; k < kNumPairClasses; ++k) {
+            std::vector<int2> all;
+            for (int b = 0; b < kOneBuckets; ++b) {
+                all.insert(all.end(), pl[k][b].begin(), pl[k][b].end());
+                c->n1_pairs[k].n[b] = (long long)pl[k][b].size();
+            }
+            if (c->d1_pairs[k].upload(all)) return -1;
+            c->n1_pairs[k].pairs = c->d1_pairs[k].p;
         }
         c->chg.clear();
     }
@@ -1852,19 +1863,22 @@ extern "C" int qk_set_charges(qk_ctx* c, const double* charges) {
 static int oneint_ready(qk_ctx* c, const char* what) {
     if (!c || !c->have_system) { set_err("%s: no system", what); return -1; }
     if ((int)c->chg.size() != c->natom) { set_err("%s: nuclear charges not set (qk_set_charges)", what); return -1; }
+    if (!c->n1_whole) { set_err("%s: a shell does not hold each of its components once (KLMN)", what); return -1; }
     (void)hipSetDevice(c->device);
     return 0;
 }
 
 static OneFuncs one_funcs(const qk_ctx* c) {
-    return OneFuncs{c->d1_atom.p, c->d1_lmn.p, c->d1_np.p, c->d1_qf.p, c->d1_a.p, c->d1_c.p};
+    return OneFuncs{c->d1_atom.p, c->d1_fn.p, c->d1_np.p, c->d1_qf.p, c->d1_a.p, c->d1_c.p};
 }
 
 extern "C" int qk_oneint_device(qk_ctx* c, double* dS, double* dH, void* stream) {
     if (oneint_ready(c, "qk_oneint_device")) return -1;
     const OneSys sys{c->d_xyz.p, c->d_chg.p, c->natom, c->nbasis};
-    const int2* pl[5] = {c->d1_pairs[0].p, c->d1_pairs[1].p, c->d1_pairs[2].p, c->d1_pairs[3].p, c->d1_pairs[4].p};
-    launch_oneint(one_funcs(c), sys, pl, c->n1_pairs, dS, dH, (hipStream_t)stream);
+    if (!c->n1_cover)   // functions outside every shell
+        for (double* p : {dS, dH})
+            if (p) launch_fill_u64((unsigned long long*)p, (long long)c->nbasis * c->nbasis, (hipStream_t)stream);
+    launch_oneint(one_funcs(c), sys, c->n1_pairs, dS, dH, (hipStream_t)stream);
     HIPCHK(hipGetLastError());
     return 0;
 }
@@ -1893,8 +1907,7 @@ extern "C" int qk_oneint_grad_device(qk_ctx* c, const double* dD, const double* 
     if (c->d1_acc.alloc(m + 1)) return -1;
     launch_fill_u64(c->d1_acc.p, m + 1, s);
     const OneSys sys{c->d_xyz.p, c->d_chg.p, c->natom, c->nbasis};
-    const int2* pl[5] = {c->d1_pairs[0].p, c->d1_pairs[1].p, c->d1_pairs[2].p, c->d1_pairs[3].p, c->d1_pairs[4].p};
-    launch_oneint_grad(one_funcs(c), sys, pl, c->n1_pairs, dD, dW, c->d1_acc.p, s);
+    launch_oneint_grad(one_funcs(c), sys, c->n1_pairs, dD, dW, c->d1_acc.p, s);
     launch_grad_finalize(c->d1_acc.p, dgrad, m, c->d1_acc.p + m, s);
     HIPCHK(hipGetLastError());
     return 0;

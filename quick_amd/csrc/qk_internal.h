@@ -279,11 +279,22 @@ struct GradArgs {
 constexpr int k1eMaxPrim = 10;   // QUICK's MAXPRIM
 struct OneFuncs {
     const int* atom;     // 0-based
-    const int* lmn;      // l | m << 4 | n << 8
+    const int* fn;       // per shell (its first function's place onward): the function of each component
     const int* np;       // primitives
     const int* qf;       // Qfinal of the function's shell (Boys order)
     const double* a;     // k1eMaxPrim exponents per function
     const double* c;     // k1eMaxPrim coefficients per function: gccoeff(k, ksumtype + L) cons(f)
+};
+// The shell pairs of one class: (first functions of A and B, l(A) >= l(B)), in
+// buckets of 2^kOneLog lanes per pair: above 16 primitive pairs, 3 to 16, fewer
+constexpr int kOneBuckets = 3;
+constexpr int kOneLog[kOneBuckets] = {4, 2, 0};
+__host__ __device__ constexpr int one_bucket(int primitive_pairs) {
+    return primitive_pairs > 16 ? 0 : (primitive_pairs > 2 ? 1 : 2);
+}
+struct OnePairs {
+    const int2* pairs;
+    long long n[kOneBuckets];
 };
 struct OneSys {
     const double* xyz;   // 3 x natom
