@@ -47,6 +47,7 @@ constexpr int kXcMaxPrim = 10;     // QUICK's MAXPRIM
 constexpr int kXcBatch = 256;      // grid points per batch
 constexpr int kXcTile = 64;        // GEMM tile (rows and columns)
 constexpr int kXcShellThreads = 320;
+constexpr int kXcds = 8;             // accelerator dies, each with its own L2
 constexpr double kXcFix = 0x1p48;  // V accumulator units
 
 typedef double v4d __attribute__((ext_vector_type(4)));
@@ -281,9 +282,12 @@ __global__ void __launch_bounds__(256) xc_batch_lists(const double* __restrict__
 // ---------------------------------------------------------------------------
 // per density
 
+// flag of a function with the centre, exponents and coefficients of the one before
+constexpr int kXcSameRadial = 1 << 16;
+
 struct XcFuncs {
     const int* atom;     // 0-based
-    const int* lmn;      // l | m << 4 | n << 8
+    const int* lmn;      // l | m << 4 | n << 8, kXcSameRadial
     const int* np;
     const double* c;     // kXcMaxPrim per function
     const double* a;
@@ -304,52 +308,86 @@ struct XcBatch {
     int batch;    // global batch index (its function list)
 };
 
-// Phi and its gradient for kXcBatch points x kXcTile functions of a batch.
-__global__ void __launch_bounds__(256) xc_values(const XcBatch* __restrict__ bt, const double* __restrict__ pts,
-                                                 const int* __restrict__ sig, int nbasis, const XcFuncs fn,
-                                                 double* __restrict__ ws) {
-    const XcBatch B = bt[blockIdx.y];
-    const int f0 = blockIdx.x * kXcTile;
-    if (f0 >= B.w) return;
+// Phi and its gradient for one rho GEMM tile, kXcTile points x kXcTile functions.
+// A lane is a point and a wavefront takes one function at a time, so the
+// contraction length, the powers and the coefficients are scalars and the
+// exponentials are evaluated as often as the function needs (with a lane per
+// function every function of the 64 cost as much as the longest contraction among
+// them), once for components that share them.  Sixteen functions at a time go
+// through LDS to be written as rows of 128 bytes.  Bound by its
+// stores: (H2O)64 on SG-1 (11,361 batches, 18 GB) 6.5 -> 3.6 ms, 5.0 TB/s.
+constexpr int kXcValCols = 16, kXcValRow = kXcValCols + 2;   // functions per step; LDS row (16-byte aligned)
+__global__ void __launch_bounds__(256) xc_values(const int4* __restrict__ tasks, const XcBatch* __restrict__ bt,
+                                                 const double* __restrict__ pts, const int* __restrict__ sig,
+                                                 int nbasis, const XcFuncs fn, double* __restrict__ ws) {
+    const int4 tk = tasks[blockIdx.x];
+    if (tk.x < 0) return;
+    const XcBatch B = bt[tk.x];
     const int* sl = sig + (long long)B.batch * nbasis;
-    double* P0 = ws + B.ws;
     const long long plane = (long long)kXcBatch * B.w;
-    for (int q = 0; q < kXcBatch * kXcTile / 256; ++q) {
-        const int e = threadIdx.x + 256 * q;
-        const int p = e / kXcTile, k = f0 + (e % kXcTile);
-        double v = 0.0, gx = 0.0, gy = 0.0, gz = 0.0;
-        if (p < B.cnt && k < B.m) {
-            const int mu = sl[k];
-            const int at = fn.atom[mu];
-            const double* P = pts + 4 * (B.p0 + p);
-            const double x = P[0] - fn.xyz[3 * at], y = P[1] - fn.xyz[3 * at + 1], z = P[2] - fn.xyz[3 * at + 2];
-            const double r2 = x * x + y * y + z * z;
-            if (r2 <= fn.r2[mu]) {
-                double rad = 0.0, drad = 0.0;   // sum c e^{-a r^2}, sum -2 a c e^{-a r^2}
-                const int np = fn.np[mu];
-                for (int c = 0; c < np; ++c) {
-                    const double al = fn.a[kXcMaxPrim * mu + c];
-                    const double t = fn.c[kXcMaxPrim * mu + c] * exp(-al * r2);
-                    rad += t;
-                    drad -= 2.0 * al * t;
+    double* const out = ws + B.ws + (long long)tk.y * kXcTile * B.w + tk.z * kXcTile;
+    __shared__ __align__(16) double s_v[4][kXcTile][kXcValRow];
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int p = tk.y * kXcTile + lane;
+    const bool in = p < B.cnt;
+    const double* P = pts + 4 * (B.p0 + (in ? p : 0));
+    const double px = P[0], py = P[1], pz = P[2];
+    constexpr int kPer = kXcValCols / 4;   // functions per wavefront and step
+    for (int c0 = 0; c0 < kXcTile; c0 += kXcValCols) {
+        double rad = 0.0, drad = 0.0;   // sum c e^{-a r^2}, sum -2 a c e^{-a r^2}
+        int last = -2;                  // the function they belong to
+        for (int c = kPer * wv; c < kPer * (wv + 1); ++c) {
+            const int k = tk.z * kXcTile + c0 + c;
+            double v = 0.0, gx = 0.0, gy = 0.0, gz = 0.0;
+            if (k < B.m) {
+                const int mu = __builtin_amdgcn_readfirstlane(sl[k]);
+                const int at = fn.atom[mu];
+                const double x = px - fn.xyz[3 * at], y = py - fn.xyz[3 * at + 1], z = pz - fn.xyz[3 * at + 2];
+                const double r2 = x * x + y * y + z * z;
+                const bool on = in && r2 <= fn.r2[mu];
+                if (__any(on)) {
+                    const int code = fn.lmn[mu];
+                    if (!(mu == last + 1 && (code & kXcSameRadial))) {
+                        rad = drad = 0.0;
+                        const int np = fn.np[mu];
+                        for (int u = 0; u < np; ++u) {
+                            const double al = fn.a[kXcMaxPrim * mu + u];
+                            const double t = fn.c[kXcMaxPrim * mu + u] * exp(-al * r2);
+                            rad += t;
+                            drad -= 2.0 * al * t;
+                        }
+                    }
+                    last = mu;
+                    const int l = code & 15, m = (code >> 4) & 15, n = (code >> 8) & 15;
+                    auto ipow = [](double b, int k) { return k == 0 ? 1.0 : (k == 1 ? b : (k == 2 ? b * b : b * b * b)); };
+                    const double xl = ipow(x, l), ym = ipow(y, m), zn = ipow(z, n);
+                    const double xl1 = l ? ipow(x, l - 1) : 0.0, ym1 = m ? ipow(y, m - 1) : 0.0,
+                                 zn1 = n ? ipow(z, n - 1) : 0.0;
+                    if (on) {
+                        v = rad * xl * ym * zn;
+                        gx = (drad * xl * x + l * rad * xl1) * ym * zn;
+                        gy = (drad * ym * y + m * rad * ym1) * xl * zn;
+                        gz = (drad * zn * z + n * rad * zn1) * xl * ym;
+                    }
                 }
-                const int code = fn.lmn[mu];
-                const int l = code & 15, m = (code >> 4) & 15, n = (code >> 8) & 15;
-                auto ipow = [](double b, int k) { return k == 0 ? 1.0 : (k == 1 ? b : (k == 2 ? b * b : b * b * b)); };
-                const double xl = ipow(x, l), ym = ipow(y, m), zn = ipow(z, n);
-                const double xl1 = l ? ipow(x, l - 1) : 0.0, ym1 = m ? ipow(y, m - 1) : 0.0,
-                             zn1 = n ? ipow(z, n - 1) : 0.0;
-                v = rad * xl * ym * zn;
-                gx = (drad * xl * x + l * rad * xl1) * ym * zn;
-                gy = (drad * ym * y + m * rad * ym1) * xl * zn;
-                gz = (drad * zn * z + n * rad * zn1) * xl * ym;
             }
+            s_v[0][lane][c] = v;
+            s_v[1][lane][c] = gx;
+            s_v[2][lane][c] = gy;
+            s_v[3][lane][c] = gz;
         }
-        const long long o = (long long)p * B.w + k;
-        P0[o] = v;
-        P0[plane + o] = gx;
-        P0[2 * plane + o] = gy;
-        P0[3 * plane + o] = gz;
+        __syncthreads();
+        // eight lanes a row of sixteen, two values each
+        const int col = 2 * (threadIdx.x & 7);
+#pragma unroll
+        for (int d = 0; d < 4; ++d)
+#pragma unroll
+            for (int h = 0; h < kXcTile; h += 32) {
+                const int row = h + (threadIdx.x >> 3);
+                *reinterpret_cast<double2*>(out + d * plane + (long long)row * B.w + c0 + col) =
+                    *reinterpret_cast<const double2*>(&s_v[d][row][col]);
+            }
+        __syncthreads();
     }
 }
 
@@ -378,12 +416,17 @@ __device__ __forceinline__ void mfma_slab(v4d acc[2][2], const double* As, const
 // rho GEMM task: (chunk batch, row tile of points, column tile of functions)
 // T = Phi D_sub over all of the batch's functions; the epilogue forms the row
 // dots of the tile with Phi and grad Phi and writes them as partials
-// part[(col tile) x kXcBatch + row][4] (fixed order, no atomics).
-__global__ void __launch_bounds__(256) xc_rho_gemm(const int4* __restrict__ tasks, const XcBatch* __restrict__ bt,
+// part[(col tile) x kXcBatch + row][4] (fixed order, no atomics).  Compiled for
+// four blocks per CU, as many as its LDS allows: it waits on D and, in the
+// epilogue, on the four planes (18 GB on (H2O)64), and at two blocks the
+// accumulators went through AGPRs; with the columns' D pointers fixed per thread,
+// 9.65 -> 7.9 ms (26 -> 32 TFLOP/s), xc_v_gemm 6.4 -> 5.7 ms (58 TFLOP/s).
+__global__ void __launch_bounds__(256, 4) xc_rho_gemm(const int4* __restrict__ tasks, const XcBatch* __restrict__ bt,
                                                    const int* __restrict__ sig, int nbasis,
                                                    const double* __restrict__ D, double* __restrict__ ws,
                                                    double* __restrict__ part) {
     const int4 tk = tasks[blockIdx.x];
+    if (tk.x < 0) return;
     const XcBatch B = bt[tk.x];
     const int pr0 = tk.y * kXcTile, jc0 = tk.z * kXcTile;
     const int* sl = sig + (long long)B.batch * nbasis;
@@ -391,14 +434,15 @@ __global__ void __launch_bounds__(256) xc_rho_gemm(const int4* __restrict__ task
     const long long plane = (long long)kXcBatch * B.w;
     // two LDS slabs: the MFMAs read one while the next is stored into the other
     __shared__ double As[2][16 * kXcTile], Bs[2][16 * kXcTile];
-    __shared__ int s_sj[kXcTile];
     __shared__ double s_red[2][kXcTile][4];
     const int t = threadIdx.x;
-    if (t < kXcTile) s_sj[t] = jc0 + t < B.m ? sl[jc0 + t] : -1;
+    // a thread loads the B values of one column; their rows are the wavefront's
+    const int gj = jc0 + (t & 63) < B.m ? sl[jc0 + (t & 63)] : -1;
+    const int kw = __builtin_amdgcn_readfirstlane(t >> 6);
+    const double* const Dj = D + max(gj, 0);
     v4d acc[2][2];
     for (int i = 0; i < 2; ++i)
         for (int j = 0; j < 2; ++j) acc[i][j] = v4d{0.0, 0.0, 0.0, 0.0};
-    __syncthreads();
     // the slab at k0 into registers: A = Phi rows (points) x k, k contiguous in
     // memory; B = D[sig k][sig j]
     double ra[4], rb[4];
@@ -408,9 +452,8 @@ __global__ void __launch_bounds__(256) xc_rho_gemm(const int4* __restrict__ task
             const int e = t + 256 * q;
             const int ia = e >> 4, ka = e & 15;
             ra[q] = P0[(long long)(pr0 + ia) * B.w + k0 + ka];
-            const int kb = e >> 6, jb = e & 63;
-            const int gk = k0 + kb < B.m ? sl[k0 + kb] : -1, gj = s_sj[jb];
-            rb[q] = (gk >= 0 && gj >= 0) ? D[(long long)gk * nbasis + gj] : 0.0;
+            const int kb = k0 + kw + 4 * q;
+            rb[q] = kb < B.m && gj >= 0 ? Dj[(long long)sl[kb] * nbasis] : 0.0;
         }
     };
     auto store = [&](int buf) {
@@ -418,7 +461,7 @@ __global__ void __launch_bounds__(256) xc_rho_gemm(const int4* __restrict__ task
         for (int q = 0; q < 4; ++q) {
             const int e = t + 256 * q;
             As[buf][(e & 15) * kXcTile + (e >> 4)] = ra[q];
-            Bs[buf][(e >> 6) * kXcTile + (e & 63)] = rb[q];
+            Bs[buf][e] = rb[q];
         }
     };
     load(0);
@@ -532,10 +575,11 @@ __global__ void __launch_bounds__(256) xc_point(const XcBatch* __restrict__ bt, 
 // V_sub = Phi^T Z + Z^T Phi over the batch's points, added to the fixed-point
 // accumulator (packed lower triangle over basis functions); in a diagonal tile
 // only the elements on or below its diagonal.
-__global__ void __launch_bounds__(256) xc_v_gemm(const int4* __restrict__ tasks, const XcBatch* __restrict__ bt,
+__global__ void __launch_bounds__(256, 4) xc_v_gemm(const int4* __restrict__ tasks, const XcBatch* __restrict__ bt,
                                                  const int* __restrict__ sig, int nbasis,
                                                  const double* __restrict__ ws, unsigned long long* __restrict__ V) {
     const int4 tk = tasks[blockIdx.x];
+    if (tk.x < 0) return;
     const XcBatch B = bt[tk.x];
     const int I0 = tk.y * kXcTile, J0 = tk.z * kXcTile;
     const int* sl = sig + (long long)B.batch * nbasis;
@@ -879,6 +923,10 @@ int qk_xc_set_system(qk_xc* x, int natom, const double* xyz, const int* Z, int n
             fa[(size_t)kXcMaxPrim * f + c] = aexp[(size_t)maxcontract * f + c];
             amin = std::min(amin, aexp[(size_t)maxcontract * f + c]);
         }
+        if (f > 0 && fatom[f - 1] == a && fnp[f - 1] == fnp[f] &&
+            std::equal(&fc[(size_t)kXcMaxPrim * f], &fc[(size_t)kXcMaxPrim * f] + fnp[f], &fc[(size_t)kXcMaxPrim * (f - 1)]) &&
+            std::equal(&fa[(size_t)kXcMaxPrim * f], &fa[(size_t)kXcMaxPrim * f] + fnp[f], &fa[(size_t)kXcMaxPrim * (f - 1)]))
+            flmn[f] |= kXcSameRadial;
         x->sig2[f] = sigrad2_or_null ? sigrad2_or_null[f] : sigrad2_of(amin, l + m + n, basis_cut);
         x->reach2[a] = std::max(x->reach2[a], x->sig2[f]);
     }
@@ -951,6 +999,25 @@ static int xc_finish_grid(qk_xc* x, XBuf<double>& pts_in, XBuf<int>& atom_in, lo
     x->chunks.clear();
     qk_xc::Chunk ch;
     long long ws = 0, part = 0, maxws = 0, maxpart = 0;
+    // A chunk's tasks are dealt to the eight XCDs by batch (block b of a launch
+    // runs on XCD b % 8), each batch to the one with the fewest tasks so far: the
+    // tiles of a batch that several tasks read then come from one L2.  Tasks of
+    // batch -1 fill the shorter queues.  (Measured on (H2O)64: xc_rho_gemm 9.9 -> 9.65 ms.)
+    std::vector<int4> rho_q[kXcds], v_q[kXcds];
+    auto deal = [](std::vector<int4>* q, std::vector<int4>& out) {
+        size_t len = 0;
+        for (int x = 0; x < kXcds; ++x) len = std::max(len, q[x].size());
+        for (size_t i = 0; i < len; ++i)
+            for (int x = 0; x < kXcds; ++x) out.push_back(i < q[x].size() ? q[x][i] : int4{-1, 0, 0, 0});
+        for (int x = 0; x < kXcds; ++x) q[x].clear();
+    };
+    auto end_chunk = [&] {
+        deal(rho_q, rho_t);
+        deal(v_q, v_t);
+        ch.nrho = (long long)rho_t.size() - ch.rho0;
+        ch.nv = (long long)v_t.size() - ch.v0;
+        x->chunks.push_back(ch);
+    };
     const long long kXcWorkspaceBytes = xc_workspace_bytes();
     x->flops = 0.0;
     for (int b = 0; b < x->nbatch; ++b) {
@@ -958,7 +1025,7 @@ static int xc_finish_grid(qk_xc* x, XBuf<double>& pts_in, XBuf<int>& atom_in, lo
         const int w = std::max(kXcTile, (m + kXcTile - 1) / kXcTile * kXcTile);
         const long long need = 5LL * kXcBatch * w;
         if (ch.nb > 0 && (ws + need) * 8 > kXcWorkspaceBytes) {
-            x->chunks.push_back(ch);
+            end_chunk();
             ch = qk_xc::Chunk();
             ch.b0 = b;
             ch.rho0 = (long long)rho_t.size();
@@ -982,15 +1049,16 @@ static int xc_finish_grid(qk_xc* x, XBuf<double>& pts_in, XBuf<int>& atom_in, lo
         ch.nb += 1;
         if (m == 0) continue;
         const int T = w / kXcTile;
+        int xcd = 0;
+        for (int k = 1; k < kXcds; ++k)
+            if (v_q[k].size() < v_q[xcd].size()) xcd = k;
         for (int r = 0; r < kXcBatch / kXcTile; ++r)
-            for (int c = 0; c < T; ++c) rho_t.push_back(int4{local, r, c, 0});
+            for (int c = 0; c < T; ++c) rho_q[xcd].push_back(int4{local, r, c, 0});
         for (int I = 0; I < T; ++I)
-            for (int J = 0; J <= I; ++J) v_t.push_back(int4{local, I, J, 0});
-        ch.nrho = (long long)rho_t.size() - ch.rho0;
-        ch.nv = (long long)v_t.size() - ch.v0;
+            for (int J = 0; J <= I; ++J) v_q[xcd].push_back(int4{local, I, J, 0});
         x->flops += 2.0 * kXcBatch * (double)w * w + 2.0 * 2.0 * kXcBatch * kXcTile * kXcTile * (T * (T + 1) / 2);
     }
-    if (ch.nb > 0) x->chunks.push_back(ch);
+    if (ch.nb > 0) end_chunk();
     // batch descriptors are per chunk: local index within the chunk
     if (x->d_bt.upload(bts) || x->d_rho_tasks.upload(rho_t) || x->d_v_tasks.upload(v_t)) return -1;
     if (x->d_ws.alloc(std::max(1LL, maxws)) || x->d_part.alloc(std::max(1LL, maxpart)) || x->d_ept.alloc(n) ||
@@ -1123,11 +1191,9 @@ int qk_xc_device(qk_xc* x, const double* dD, double* dV, double* Exc, double* ne
     XcFuncs fn{x->d_fatom.p, x->d_flmn.p, x->d_fnp.p, x->d_fc.p, x->d_fa.p, x->d_fr2.p, x->d_xyz.p};
     for (const auto& ch : x->chunks) {
         const XcBatch* bt = x->d_bt.p + ch.b0;
-        int wmax = 0;
-        for (int b = ch.b0; b < ch.b0 + ch.nb; ++b)
-            wmax = std::max(wmax, std::max(kXcTile, (x->h_nsig[b] + kXcTile - 1) / kXcTile * kXcTile));
-        hipLaunchKernelGGL(xc_values, dim3(wmax / kXcTile, ch.nb), dim3(256), 0, s, bt, x->d_pts.p, x->d_sig.p, n, fn,
-                           x->d_ws.p);
+        if (ch.nrho > 0)
+            hipLaunchKernelGGL(xc_values, dim3((unsigned)ch.nrho), dim3(256), 0, s, x->d_rho_tasks.p + ch.rho0, bt,
+                               x->d_pts.p, x->d_sig.p, n, fn, x->d_ws.p);
         if (ch.nrho > 0)
             hipLaunchKernelGGL(xc_rho_gemm, dim3((unsigned)ch.nrho), dim3(256), 0, s, x->d_rho_tasks.p + ch.rho0, bt,
                                x->d_sig.p, n, dD, x->d_ws.p, x->d_part.p);
