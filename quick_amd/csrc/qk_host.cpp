@@ -1147,16 +1147,18 @@ static int fock_enqueue(qk_ctx* c, const double* dD, const double* dcutmat_or_nu
     std::iota(order.begin(), order.end(), 0);
     std::sort(order.begin(), order.end(), [&](int x, int y) { return c->classes[x].total > c->classes[y].total; });
     if (mixed && !c->d_boys_tab.p) { set_err("mixed precision: Boys table missing"); return -1; }
-    // Two streams, forked from the caller's and joined with events.  In a mixed
-    // build the FP64 lists hold the few strongest pairs (long ket ranges on few
-    // bras): those kernels run on the second stream beside the FP32 lists.  In
-    // an FP64 build the classes alternate between the streams in this order, so
-    // that one class's tail overlaps the next class (measured: (H2O)32 36.0 ->
-    // 34.2 ms, n-icosane 20.3 -> 17.3 ms).
+    // Four streams (one per hardware queue), three of them forked from the caller's
+    // and joined with events, so that one class's tail overlaps the next classes.
+    // An FP64 build deals the classes to all four in this order; in a mixed build
+    // the FP64 lists, which hold the few strongest pairs (long ket ranges on few
+    // bras), go to two of them and the FP32 lists to the others.  Measured against
+    // one such pair of streams: one water 545 -> 426 us, n-nonane 4.95 -> 4.34 ms,
+    // (H2O)32 27.2 -> 26.5 ms, mixed at 1e-3 18.5 -> 17.5 ms.
     const hipStream_t s64 = c->streams[0];
     HIPCHK(hipEventRecord(c->ev_start, s));
-    HIPCHK(hipStreamWaitEvent(s64, c->ev_start, 0));
-    // The classes of one stream run one after another, so at most two kernels
+    const hipStream_t q4[4] = {s64, s, c->streams[1], c->streams[2]};
+    for (int k = 0; k < 3; ++k) HIPCHK(hipStreamWaitEvent(c->streams[k], c->ev_start, 0));
+    // The classes of one stream run one after another, so at most four kernels
     // are in flight.  Kernels that spill get a grid small enough
     // that their private-segment backing stays under kScratchBudget
     // (scratch_grid_cap); the grid-stride loop over tiles covers the rest.
@@ -1177,7 +1179,7 @@ static int fock_enqueue(qk_ctx* c, const double* dD, const double* dcutmat_or_nu
         ClassHost& CH = c->classes[k];
         if (CH.ntiles == 0 && CH.ntiles32 == 0) continue;
         // the stream of this class's FP64 list
-        const hipStream_t l64 = !mixed && (pos & 1) ? s : s64;
+        const hipStream_t l64 = mixed ? (pos & 1 ? c->streams[1] : s64) : q4[pos & 3];
         // one bra pair per block with its exchange rows in LDS, when they fit
         const int nrow = bra_rows(k);
         const size_t rows_lds = sizeof(unsigned long long) * (size_t)nrow * n;
@@ -1239,7 +1241,7 @@ static int fock_enqueue(qk_ctx* c, const double* dD, const double* dcutmat_or_nu
             c->cls_timed[k] = c->timing;
         }
         if (mixed && CH.ntiles32) {
-            const hipStream_t ls = light64 && (k == 19 || k == 20) ? s64 : s;
+            const hipStream_t ls = light64 && (k == 19 || k == 20) ? s64 : (pos & 1 ? c->streams[2] : s);
             a.counters = fb->counters + 2 * kNumQuartetClasses + 2 * k;
                     const int slot = kNumQuartetClasses + k;
             if (c->timing) HIPCHK(hipEventRecord(c->ev_t0[slot], ls));
@@ -1271,8 +1273,10 @@ static int fock_enqueue(qk_ctx* c, const double* dD, const double* dcutmat_or_nu
             c->cls_timed[slot] = c->timing;
         }
     }
-    HIPCHK(hipEventRecord(c->ev_cls[0], s64));
-    HIPCHK(hipStreamWaitEvent(s, c->ev_cls[0], 0));
+    for (int k = 0; k < 3; ++k) {
+        HIPCHK(hipEventRecord(c->ev_cls[k], c->streams[k]));
+        HIPCHK(hipStreamWaitEvent(s, c->ev_cls[k], 0));
+    }
     launch_jpair_scatter(fb->J, c->dp_jofs.p, c->dp_pstride.p, c->dp_qa.p, c->dp_qb.p, a.q, c->nclass_pairs, fb->X,
                          n, s);
     launch_fock_finalize(fb->X, fb->xcopies, c->d_cons.p, dG, n, fb->counters + kRangeFlag, s);
@@ -1746,16 +1750,17 @@ static int grad_enqueue(qk_ctx* c, const double* dD, const double* dcutmat_or_nu
     ca.steps = nullptr;
     ca.slot0 = nullptr;
     ca.chunk = 64;
-    // Two streams, forked from the caller's and joined with events.  A mixed
-    // gradient's FP64 list holds the few strongest pairs: its kernels have
-    // little parallelism and long per-quartet chains, so they run on the second
-    // stream beside the FP32 list.  In an FP64 gradient the classes alternate
-    // between the streams (measured: (H2O)32 188.8 -> 172 ms, n-icosane 113.9
-    // -> 102.5 ms).  One kernel per stream is in flight, each within its grid's
-    // scratch bound, so at most two bounded backings are live.
+    // Four streams as in the Fock build.  A mixed gradient's FP64 list holds the
+    // few strongest pairs: its kernels have little parallelism and long
+    // per-quartet chains, so they run on two of the streams beside the FP32 list.
+    // In an FP64 gradient the classes go round the four.  Measured against two
+    // streams: one water 764 -> 490 us, n-icosane 23.6 -> 22.3 ms, mixed (H2O)32
+    // 22.6 -> 21.7 ms.  One kernel per stream is in flight, each within its
+    // grid's scratch bound, so at most four bounded backings are live.
     const hipStream_t s64 = c->streams[0];
     HIPCHK(hipEventRecord(c->ev_start, s));
-    HIPCHK(hipStreamWaitEvent(s64, c->ev_start, 0));
+    const hipStream_t q4[4] = {s64, s, c->streams[1], c->streams[2]};
+    for (int k = 0; k < 3; ++k) HIPCHK(hipStreamWaitEvent(c->streams[k], c->ev_start, 0));
     // When the FP64 lists are light (under 7.5% of the candidate tiles), the
     // FP32 lists of (dp|ds) and of the table-driven d-d bra classes ((dd|ps),
     // (dd|pp), (dd|ds), (dd|dp), (dd|dd)) follow them on the second stream.
@@ -1775,7 +1780,7 @@ static int grad_enqueue(qk_ctx* c, const double* dD, const double* dcutmat_or_nu
     for (int pass = 0; pass < (mixed ? 2 : 1); ++pass) {
         const bool fp32 = pass == 1;
         for (int k = 0; k < kNumQuartetClasses; ++k) {
-            const hipStream_t ls = fp32 ? (((on_second >> k) & 1u) ? s64 : s) : (!mixed && (k & 1) ? s : s64);
+            const hipStream_t ls = fp32 ? (((on_second >> k) & 1u) ? s64 : (k & 1 ? c->streams[2] : s)) : (mixed ? (k & 1 ? c->streams[1] : s64) : q4[k & 3]);
             const long long nt = fp32 ? c->ngtiles32[k] : c->ngtiles[k];
             if (nt == 0) continue;
             ClassWork w{(fp32 ? c->d_gtiles32[k] : c->d_gtiles[k]).p, nt};
@@ -1815,8 +1820,10 @@ static int grad_enqueue(qk_ctx* c, const double* dD, const double* dcutmat_or_nu
             c->cls_timed[slot] = c->timing;
         }
     }
-    HIPCHK(hipEventRecord(c->ev_cls[0], s64));
-    HIPCHK(hipStreamWaitEvent(s, c->ev_cls[0], 0));
+    for (int k = 0; k < 3; ++k) {
+        HIPCHK(hipEventRecord(c->ev_cls[k], c->streams[k]));
+        HIPCHK(hipStreamWaitEvent(s, c->ev_cls[k], 0));
+    }
     launch_grad_finalize(c->d_gacc.p, dgrad, 3 * c->natom, c->d_gcounters.p + kGradRangeFlag, s);
     HIPCHK(hipGetLastError());
     return 0;
