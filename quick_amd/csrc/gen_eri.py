@@ -157,7 +157,7 @@ def gen_vrr(cls):
     return f"{sig}\n{{\n{body}\n}}\n", ne * nf, nflop, len(order)
 
 
-def gen_hrr(cls):
+def gen_hrr(cls, ia=None):
     """acc[e][f] -> out[a][b][c][d] in QUICK's component order."""
     la, lb, lc, ld = cls
     E, F = la + lb, lc + ld
@@ -203,6 +203,8 @@ def gen_hrr(cls):
     nonlocal_flops = [0]
     A_list, B_list = QUICK_ORDER[la], QUICK_ORDER[lb]
     C_list, D_list = QUICK_ORDER[lc], QUICK_ORDER[ld]
+    if ia is not None:   # the outputs of one component of A
+        A_list = A_list[ia:ia + 1]
     # (ab|f0) for the needed f: all f in flist
     for a in A_list:
         for b in B_list:
@@ -241,9 +243,15 @@ def gen_hrr(cls):
                 for d in D_list:
                     outs.append(f"    out[{k}] = {ket_expr((a, b), c, d)};")
                     k += 1
+    if ia is not None:
+        return "\n".join(lines + outs), nonlocal_flops[0], k
     sig = (f"template <typename R>\n__device__ __forceinline__ void hrr_{tag(cls)}(const R* __restrict__ acc, "
            "R ABx, R ABy, R ABz, R CDx, R CDy, R CDz, R* __restrict__ out)")
     return f"{sig}\n{{\n" + "\n".join(lines + outs) + "\n}\n", nonlocal_flops[0], k
+
+
+# Classes whose outputs (162) do not fit in the registers at once
+SLICED_CLASSES = [(2, 1, 1, 1)]
 
 
 def write_units(outdir):
@@ -295,12 +303,22 @@ def write_units(outdir):
 def main(path):
     out = ["// Generated by quick_amd/csrc/gen_eri.py -- do not edit.",
            "// Per-class VRR/HRR for (la lb|lc ld), la>=lb, lc>=ld, bra pair class >= ket pair class.",
-           "#pragma once", ""]
+           "#pragma once", "",
+           "// the HRR of one component of A (see fock_quartets), for the classes that take it in slices",
+           "template <int LA, int LB, int LC, int LD>\nstruct HrrSlices {\n    static constexpr bool on = false;\n};", ""]
     table = []
     for cls in quartet_classes():
         v, nacc, vflop, nterms = gen_vrr(cls)
         h, hflop, nout = gen_hrr(cls)
         out += [v, h]
+        if cls in SLICED_CLASSES:
+            out += [f"template <>\nstruct HrrSlices<{', '.join(map(str, cls))}> {{", "    static constexpr bool on = true;",
+                    "    template <int IA, typename R>",
+                    "    static __device__ __forceinline__ void hrr(const R* __restrict__ acc, R ABx, R ABy, R ABz, R CDx, "
+                    "R CDy, R CDz, R* __restrict__ out)", "    {"]
+            for ia in range(len(QUICK_ORDER[cls[0]])):
+                out += [f"    if constexpr (IA == {ia}) {{", gen_hrr(cls, ia)[0], "    }"]
+            out += ["    }", "};"]
         table.append((cls, nacc, vflop, hflop, nout))
     hdr = ["// Generated by quick_amd/csrc/gen_eri.py -- do not edit.",
            "// Arithmetic operations of the generated code, per class (FMA = 2):",

@@ -1,5 +1,6 @@
 // qk_kernels.h -- device code shared by the per-class translation units.
 #pragma once
+#include <utility>
 #include "qk_internal.h"
 #include "eri_generated.inc"
 
@@ -286,6 +287,12 @@ __device__ __forceinline__ long long wave_sum_i64(long long v) {
 // The thread-per-quartet Fock kernels: one body, in FP64 (fock_kernel) and in
 // FP32 with FP64-grade accumulation (fock_kernel_f32).
 
+// f(0), ..., f(N - 1) with compile-time arguments
+template <class F, int... I>
+__device__ __forceinline__ void for_each_int(std::integer_sequence<int, I...>, F&& f) {
+    (f(std::integral_constant<int, I>{}), ...);
+}
+
 // pieces that differ with the arithmetic type
 template <typename R>
 struct FockType;
@@ -339,8 +346,8 @@ __device__ __forceinline__ void fock_quartets(const FockArgs& a, const ClassWork
     constexpr int NE = nrange(LA, LA + LB), NF = nrange(LC, LC + LD);
     constexpr int NACC = NE * NF;
     constexpr int NA = ncart(LA), NB = ncart(LB), NC = ncart(LC), ND = ncart(LD);
-    constexpr int NOUT = NA * NB * NC * ND;
     constexpr int LT = LA + LB + LC + LD;
+    constexpr bool kSliced = HrrSlices<LA, LB, LC, LD>::on;
     constexpr bool RUNS = MODE != kNoRuns, STAGE = MODE == kStaged;
     constexpr bool kKeepJ = RUNS && NA * NB <= 9;   // the run's Coulomb block in registers
     constexpr bool kCentreC = LC + LD > 0;
@@ -508,18 +515,6 @@ __device__ __forceinline__ void fock_quartets(const FockArgs& a, const ClassWork
         const KetGather<R> g1 = gather(T1, r1, RUNS ? rb.sh : a.rec[T1.p].sh, share_j(t + tstep));
         if (active) {
             const int atA = rb.at & 0xffff, atB = rb.at >> 16, atD = r0.at >> 16;
-            R out[NOUT];
-            {
-                const R Ax = R(a.xyz[3 * atA]), Ay = R(a.xyz[3 * atA + 1]), Az = R(a.xyz[3 * atA + 2]);
-                const R Bx = R(a.xyz[3 * atB]), By = R(a.xyz[3 * atB + 1]), Bz = R(a.xyz[3 * atB + 2]);
-                R CDx = R(0), CDy = R(0), CDz = R(0);
-                if constexpr (kCentreC) {
-                    CDx = R(g0.Cx) - R(a.xyz[3 * atD]);
-                    CDy = R(g0.Cy) - R(a.xyz[3 * atD + 1]);
-                    CDz = R(g0.Cz) - R(a.xyz[3 * atD + 2]);
-                }
-                ClassOps<LA, LB, LC, LD>::template hrr<R>(acc, Ax - Bx, Ay - By, Az - Bz, CDx, CDy, CDz, out);
-            }
             // digestion: G = (X + X^T)/2 with X accumulating
             //   X[a][b] += 4w D[c][d] I,  X[c][d] += 4w D[a][b] I,
             //   X[a][c] -= h w D[b][d] I, X[a][d] -= h w D[b][c] I,
@@ -532,70 +527,105 @@ __device__ __forceinline__ void fock_quartets(const FockArgs& a, const ClassWork
             if (r0.misc & 16u) wgt *= R(0.5);
             if (p == q0) wgt *= R(0.5);
             const R jw = R(4) * wgt, kw = -R(a.hybrid) * wgt;
-            // element (row, col) of the density; n <= 65535, so the index fits 32 bits
-            auto DG = [&](int row, int col) { return Dp[unsigned(row) * unsigned(n) + unsigned(col)]; };
-#define OUT(ia, ib, ic, id) out[(((ia)*NB + (ib)) * NC + (ic)) * ND + (id)]
-            if (a.hybrid != 0.0) {
-                // exchange: the bra rows of D from LDS (staged per run) or from memory,
-                // the sums into the block's LDS rows or straight into X.  No branch
-                // between them: the density reads of all of them go out together (a
-                // test for zero at each one made every sum wait for its own reads)
+            // exchange: the bra rows of D from LDS (staged per run) or from memory,
+            // the sums into the block's LDS rows or straight into X.  No branch
+            // between them: the density reads of all of them go out together (a
+            // test for zero at each one made every sum wait for its own reads)
+            auto put = [&](int r, int grow, int col, R s) {
+                const long long iv = Ft::fixed(kw * s);
+                if constexpr (RUNS) atomicAdd(s_xrows + r * n + col, (unsigned long long)iv);
+                else if (iv != 0) atomicAdd(Xc + (long long)grow * n + col, (unsigned long long)iv);
+            };
+            R sbc[NB * NC], sbd[NB * ND], scd[NC * ND];
+#pragma unroll
+            for (int k = 0; k < NB * NC; ++k) sbc[k] = R(0);
+#pragma unroll
+            for (int k = 0; k < NB * ND; ++k) sbd[k] = R(0);
+#pragma unroll
+            for (int k = 0; k < NC * ND; ++k) scd[k] = R(0);
+            // components [i0, i0 + NS) of A: all at once, or one after another in
+            // (dp|pp), whose 162 integrals do not fit in the registers together
+            // (private memory 2,128 -> 924 bytes per lane; (H2O)32 3.92 -> 3.27 ms,
+            // and with four times the blocks under the scratch bound n-nonane's build
+            // 4.34 -> 3.65 ms; (dd|ps) and (dp|ds), 108 integrals, gained nothing or
+            // lost: 0.82 -> 1.02 ms)
+            auto slice = [&](auto i0_) {
+                constexpr int i0 = decltype(i0_)::value, NS = kSliced ? 1 : NA;
+                const R* Ds = Dp;
+                if constexpr (kSliced) asm volatile("" : "+s"(Ds));   // the reads are not kept from slice to slice
+                // element (row, col) of the density; n <= 65535, so the index fits 32 bits
+                auto DG = [&](int row, int col) { return Ds[unsigned(row) * unsigned(n) + unsigned(col)]; };
                 auto B = [&](int r, int grow, int col) {
                     if constexpr (STAGE) return sD[r * n + col];
                     else return DG(grow, col);
                 };
-                auto put = [&](int r, int grow, int col, R s) {
-                    const long long iv = Ft::fixed(kw * s);
-                    if constexpr (RUNS) atomicAdd(s_xrows + r * n + col, (unsigned long long)iv);
-                    else if (iv != 0) atomicAdd(Xc + (long long)grow * n + col, (unsigned long long)iv);
-                };
-                for (int ia = 0; ia < NA; ++ia)
-                    for (int ic = 0; ic < NC; ++ic) {
-                        R s = R(0);
-                        for (int ib = 0; ib < NB; ++ib)
-                            for (int id = 0; id < ND; ++id) s += B(NA + ib, fb + ib, fd + id) * OUT(ia, ib, ic, id);
-                        put(ia, fa + ia, fc + ic, s);
+                R out[NS * NB * NC * ND];
+                {
+                    const R Ax = R(a.xyz[3 * atA]), Ay = R(a.xyz[3 * atA + 1]), Az = R(a.xyz[3 * atA + 2]);
+                    const R Bx = R(a.xyz[3 * atB]), By = R(a.xyz[3 * atB + 1]), Bz = R(a.xyz[3 * atB + 2]);
+                    R CDx = R(0), CDy = R(0), CDz = R(0);
+                    if constexpr (kCentreC) {
+                        CDx = R(g0.Cx) - R(a.xyz[3 * atD]);
+                        CDy = R(g0.Cy) - R(a.xyz[3 * atD + 1]);
+                        CDz = R(g0.Cz) - R(a.xyz[3 * atD + 2]);
                     }
-                for (int ia = 0; ia < NA; ++ia)
-                    for (int id = 0; id < ND; ++id) {
-                        R s = R(0);
-                        for (int ib = 0; ib < NB; ++ib)
-                            for (int ic = 0; ic < NC; ++ic) s += B(NA + ib, fb + ib, fc + ic) * OUT(ia, ib, ic, id);
-                        put(ia, fa + ia, fd + id, s);
-                    }
-                for (int ib = 0; ib < NB; ++ib)
-                    for (int ic = 0; ic < NC; ++ic) {
-                        R s = R(0);
-                        for (int ia = 0; ia < NA; ++ia)
-                            for (int id = 0; id < ND; ++id) s += B(ia, fa + ia, fd + id) * OUT(ia, ib, ic, id);
-                        put(NA + ib, fb + ib, fc + ic, s);
-                    }
-                for (int ib = 0; ib < NB; ++ib)
-                    for (int id = 0; id < ND; ++id) {
-                        R s = R(0);
-                        for (int ia = 0; ia < NA; ++ia)
-                            for (int ic = 0; ic < NC; ++ic) s += B(ia, fa + ia, fc + ic) * OUT(ia, ib, ic, id);
-                        put(NA + ib, fb + ib, fd + id, s);
-                    }
-            }
-            for (int ia = 0; ia < NA; ++ia)
-                for (int ib = 0; ib < NB; ++ib) {
-                    R s = R(0);
-                    for (int ic = 0; ic < NC; ++ic)
-                        for (int id = 0; id < ND; ++id) s += DG(fc + ic, fd + id) * OUT(ia, ib, ic, id);
-                    jac[ia * NB + ib] += Ft::fixed(jw * s);
+                    if constexpr (kSliced)
+                        HrrSlices<LA, LB, LC, LD>::template hrr<i0, R>(acc, Ax - Bx, Ay - By, Az - Bz, CDx, CDy, CDz, out);
+                    else
+                        ClassOps<LA, LB, LC, LD>::template hrr<R>(acc, Ax - Bx, Ay - By, Az - Bz, CDx, CDy, CDz, out);
                 }
-            long long vj[NC * ND];
-            for (int ic = 0; ic < NC; ++ic)
-                for (int id = 0; id < ND; ++id) {
-                    R s = R(0);
-                    for (int ia = 0; ia < NA; ++ia)
-                        for (int ib = 0; ib < NB; ++ib) s += DG(fa + ia, fb + ib) * OUT(ia, ib, ic, id);
-                    vj[ic * ND + id] = Ft::fixed(jw * s);
+#define OUT(is, ib, ic, id) out[(((is)*NB + (ib)) * NC + (ic)) * ND + (id)]
+                if (a.hybrid != 0.0) {
+                    for (int is = 0; is < NS; ++is)
+                        for (int ic = 0; ic < NC; ++ic) {
+                            R s = R(0);
+                            for (int ib = 0; ib < NB; ++ib)
+                                for (int id = 0; id < ND; ++id) s += B(NA + ib, fb + ib, fd + id) * OUT(is, ib, ic, id);
+                            put(i0 + is, fa + i0 + is, fc + ic, s);
+                        }
+                    for (int is = 0; is < NS; ++is)
+                        for (int id = 0; id < ND; ++id) {
+                            R s = R(0);
+                            for (int ib = 0; ib < NB; ++ib)
+                                for (int ic = 0; ic < NC; ++ic) s += B(NA + ib, fb + ib, fc + ic) * OUT(is, ib, ic, id);
+                            put(i0 + is, fa + i0 + is, fd + id, s);
+                        }
+                    for (int ib = 0; ib < NB; ++ib)
+                        for (int ic = 0; ic < NC; ++ic)
+                            for (int is = 0; is < NS; ++is)
+                                for (int id = 0; id < ND; ++id)
+                                    sbc[ib * NC + ic] += B(i0 + is, fa + i0 + is, fd + id) * OUT(is, ib, ic, id);
+                    for (int ib = 0; ib < NB; ++ib)
+                        for (int id = 0; id < ND; ++id)
+                            for (int is = 0; is < NS; ++is)
+                                for (int ic = 0; ic < NC; ++ic)
+                                    sbd[ib * ND + id] += B(i0 + is, fa + i0 + is, fc + ic) * OUT(is, ib, ic, id);
                 }
-            for (int k = 0; k < NC * ND; ++k)
-                if (vj[k] != 0) atomicAdd(a.J + r0.jofs + (long long)k * pks, (unsigned long long)vj[k]);
+                for (int is = 0; is < NS; ++is)
+                    for (int ib = 0; ib < NB; ++ib) {
+                        R s = R(0);
+                        for (int ic = 0; ic < NC; ++ic)
+                            for (int id = 0; id < ND; ++id) s += DG(fc + ic, fd + id) * OUT(is, ib, ic, id);
+                        jac[(i0 + is) * NB + ib] += Ft::fixed(jw * s);
+                    }
+                for (int ic = 0; ic < NC; ++ic)
+                    for (int id = 0; id < ND; ++id)
+                        for (int is = 0; is < NS; ++is)
+                            for (int ib = 0; ib < NB; ++ib)
+                                scd[ic * ND + id] += DG(fa + i0 + is, fb + ib) * OUT(is, ib, ic, id);
 #undef OUT
+            };
+            for_each_int(std::make_integer_sequence<int, kSliced ? NA : 1>{}, slice);
+            if (a.hybrid != 0.0) {
+                for (int ib = 0; ib < NB; ++ib)
+                    for (int ic = 0; ic < NC; ++ic) put(NA + ib, fb + ib, fc + ic, sbc[ib * NC + ic]);
+                for (int ib = 0; ib < NB; ++ib)
+                    for (int id = 0; id < ND; ++id) put(NA + ib, fb + ib, fd + id, sbd[ib * ND + id]);
+            }
+            for (int k = 0; k < NC * ND; ++k) {
+                const long long vj = Ft::fixed(jw * scd[k]);
+                if (vj != 0) atomicAdd(a.J + r0.jofs + (long long)k * pks, (unsigned long long)vj);
+            }
         }
         if constexpr (!kKeepJ) flush_j(rb, p);
         T0 = T1; T1 = T2; T2 = T3;
@@ -742,9 +772,10 @@ struct OccupancyF {
     // six or more exchange rows already hold a run-mode block to three per CU
     // at 800 functions (more functions: fewer): asking for four wavefronts per
     // SIMD only made such kernels spill (measured: ppps 1.34 -> 1.27 ms, dsds
-    // 0.44 -> 0.42 ms with three)
+    // 0.44 -> 0.42 ms with three); (dp|pp), with 144 accumulators, spills at two
+    // (1.10 -> 0.97 ms with one)
     static constexpr int rows = ncart(LA) + ncart(LB);
-    static constexpr int value = nacc <= 36 ? (rows >= 6 ? 3 : 4) : 2;
+    static constexpr int value = nacc <= 36 ? (rows >= 6 ? 3 : 4) : (nacc < 144 ? 2 : 1);
 };
 
 // the tabulated expansion (kStride: the LDS slice or the table in memory)
