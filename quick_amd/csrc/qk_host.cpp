@@ -649,10 +649,13 @@ using ListSumsFn = std::function<int(const std::vector<long long>&, std::vector<
 // one after another (up to 1,296 of them, 0.4 us each in FP64), so where a class
 // has too few tiles to fill the GPU the longest chain is the kernel's time; there
 // each tile's primitives are split over wavefronts that would be idle (one water:
-// Fock build 2.39 -> 0.54 ms, gradient 2.28 -> 0.76 ms).  2,048 wavefronts (two
+// Fock build 2.39 -> 0.54 ms, gradient 2.28 -> 0.76 ms).  1,024 wavefronts (one
 // per SIMD) are taken as full: above that a share only repeats the quartet's
-// screening and digestion.
-constexpr long long kSplitTiles = 2048;
+// screening and digestion.  Measured with 256 / 512 / 1,024 / 2,048 / 8,192: one
+// water 504 / 391 / 394 / 410 / 433 us, n-nonane 3.26 / 3.31 / 3.42 / 3.62 / 6.1 ms,
+// SCF of (H2O)4 52.8 / 52.6 / 50.6 / 53.7 / 71 ms, gradient of n-icosane 23.4 /
+// 23.4 / 23.8 / 24.1 / 25.9 ms.
+constexpr long long kSplitTiles = 1024;
 static int share_tiles(long long tiles, int prims) {
     int l = 0;
     while (l < 6 && tiles > 0 && (tiles << l) < kSplitTiles && (2 << l) <= prims) ++l;
