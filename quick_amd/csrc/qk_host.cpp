@@ -322,6 +322,7 @@ struct qk_ctx {
     DBuf<double> d1_a, d1_c, d_chg;
     std::vector<double> chg;
     DBuf<unsigned long long> d1_acc;
+    DBuf<double> d1_m[2], d1_grad;   // the host entry points' matrices and gradient (kept: allocating them cost 0.4 ms)
     // pair-indexed Coulomb buffer of the prepared pair list (FockArgs::J)
     DBuf<int> dp_jofs;
     DBuf<unsigned long long> d_J;
@@ -1953,7 +1954,7 @@ extern "C" int qk_oneint_grad_device(qk_ctx* c, const double* dD, const double* 
 extern "C" int qk_oneint_host(qk_ctx* c, double* S, double* H) {
     if (oneint_ready(c, "qk_oneint_host")) return -1;
     const size_t nn = (size_t)c->nbasis * c->nbasis;
-    DBuf<double> dS, dH;
+    DBuf<double>&dS = c->d1_m[0], &dH = c->d1_m[1];
     if (dS.alloc(nn) || dH.alloc(nn)) return -1;
     if (qk_oneint_device(c, dS.p, dH.p, nullptr)) return -1;
     if (S) HIPCHK(hipMemcpy(S, dS.p, nn * sizeof(double), hipMemcpyDeviceToHost));
@@ -1964,7 +1965,7 @@ extern "C" int qk_oneint_host(qk_ctx* c, double* S, double* H) {
 extern "C" int qk_oneint_grad_host(qk_ctx* c, const double* D, const double* W, double* grad) {
     if (oneint_ready(c, "qk_oneint_grad_host")) return -1;
     const size_t nn = (size_t)c->nbasis * c->nbasis, m = 3 * (size_t)c->natom;
-    DBuf<double> dD, dW, dg;
+    DBuf<double>&dD = c->d1_m[0], &dW = c->d1_m[1], &dg = c->d1_grad;
     if (dD.alloc(nn) || dW.alloc(nn) || dg.alloc(m)) return -1;
     HIPCHK(hipMemcpy(dD.p, D, nn * sizeof(double), hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(dW.p, W, nn * sizeof(double), hipMemcpyHostToDevice));
