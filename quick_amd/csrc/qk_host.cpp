@@ -578,7 +578,6 @@ extern "C" int qk_set_system(qk_ctx* c, int natom, const double* xyz, int nshell
                 fat[fn] = katom[sh] - 1;
                 // its component: x powers falling, then y powers falling
                 const int x = KLMN[3 * fn], y = KLMN[3 * fn + 1], z = KLMN[3 * fn + 2];
-                if (x + y + z > 2) { set_err("one-electron integrals: functions above d"); return -1; }
                 const bool ok = x >= 0 && y >= 0 && z >= 0 && x + y + z == L;
                 int* slot = ok ? &ffn[c->q_f0[q] + (L - x) * (L - x + 1) / 2 + z] : nullptr;
                 if (slot && *slot < 0) *slot = fn;
@@ -594,6 +593,11 @@ extern "C" int qk_set_system(qk_ctx* c, int natom, const double* xyz, int nshell
         if (c->d1_atom.upload(fat) || c->d1_fn.upload(ffn) || c->d1_np.upload(fnp) || c->d1_qf.upload(fqf) ||
             c->d1_a.upload(fa) || c->d1_c.upload(fc))
             return -1;
+        for (int fn = 0; fn < nbasis; ++fn)   // those outside every shell too
+            if (KLMN[3 * fn] + KLMN[3 * fn + 1] + KLMN[3 * fn + 2] > 2) {
+                set_err("one-electron integrals: functions above d");
+                return -1;
+            }
         c->n1_cover = std::find(ffn.begin(), ffn.end(), -1) == ffn.end();
         std::vector<int2> pl[kNumPairClasses][kOneBuckets];
         const int nq = (int)c->q_L.size();
@@ -1913,8 +1917,10 @@ extern "C" int qk_oneint_device(qk_ctx* c, double* dS, double* dH, void* stream)
     hipStream_t of[kNumPairClasses];
     if (one_fork(c, (hipStream_t)stream, of)) return -1;
     launch_oneint(one_funcs(c), sys, c->n1_pairs, dS, dH, of);
-    HIPCHK(hipGetLastError());
-    return one_join(c, (hipStream_t)stream);
+    const hipError_t launched = hipGetLastError();   // joined also where a launch failed
+    if (one_join(c, (hipStream_t)stream)) return -1;
+    HIPCHK(launched);
+    return 0;
 }
 
 extern "C" int qk_nuclear_repulsion(qk_ctx* c, double* E) {
@@ -1944,8 +1950,9 @@ extern "C" int qk_oneint_grad_device(qk_ctx* c, const double* dD, const double* 
     hipStream_t of[kNumPairClasses];
     if (one_fork(c, s, of)) return -1;
     launch_oneint_grad(one_funcs(c), sys, c->n1_pairs, dD, dW, c->d1_acc.p, of);
-    HIPCHK(hipGetLastError());
+    const hipError_t launched = hipGetLastError();
     if (one_join(c, s)) return -1;
+    HIPCHK(launched);
     launch_grad_finalize(c->d1_acc.p, dgrad, m, c->d1_acc.p + m, s);
     HIPCHK(hipGetLastError());
     return 0;
