@@ -739,13 +739,17 @@ static std::vector<int> most_primitives(const qk_ctx* c) {
 // classes up to a d-p bra (ppps 16.5 -> 10.7 ms, dpps 17.4 -> 9.5 ms, FP64
 // build 235 -> 202 ms) and for the FP32 classes with a p or p-p ket (ppps
 // 10.3 -> 7.6 ms), and costs the FP32 classes with an s-s ket (dsss 6.6 ->
-// 9.1 ms) and every d-d bra (on (H2O)32, ddps 1.04 -> 1.77 ms)
+// 9.1 ms) and every d-d bra (FP32, on (H2O)32: ddps 1.04 -> 1.77 ms).  In FP64 a
+// d-d bra keeps its rows while two blocks fit a CU, as many as its registers allow
+// ((H2O)32 build 25.96 -> 25.25 ms); one block per CU loses ((H2O)64 mixed 107.5
+// -> 108.2 ms)
 constexpr size_t kRowsLdsMax = 152 * 1024, kRowsLdsSmall = 64 * 1024;
+constexpr size_t kRowsLdsTwo = 160 * 1024 / 2 - 7 * 64 * sizeof(double) - 1024;   // beside the bra slab and the static LDS
 static int bra_rows(int k) { return ncart_of(kClassL[k][0]) + ncart_of(kClassL[k][1]); }
 // whether class k takes one bra pair per block with its exchange rows in LDS
 static bool fock_uses_runs(int k, int n, bool fp32) {
     const size_t rows = sizeof(unsigned long long) * (size_t)bra_rows(k) * n;
-    const bool big_ok = bra_rows(k) <= 9 && rows <= kRowsLdsMax;
+    const bool big_ok = (bra_rows(k) <= 9 && rows <= kRowsLdsMax) || (!fp32 && rows <= kRowsLdsTwo);
     const int nket = ncart_of(kClassL[k][2]) * ncart_of(kClassL[k][3]);
     return !fock_class_is_team(k) && (rows <= kRowsLdsSmall || (big_ok && (!fp32 || nket >= 3)));
 }
