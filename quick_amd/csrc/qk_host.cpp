@@ -1774,7 +1774,7 @@ static int grad_enqueue(qk_ctx* c, const double* dD, const double* dcutmat_or_nu
     const hipStream_t q4[4] = {s64, s, c->streams[1], c->streams[2]};
     for (int k = 0; k < 3; ++k) HIPCHK(hipStreamWaitEvent(c->streams[k], c->ev_start, 0));
     // When the FP64 lists are light (under 7.5% of the candidate tiles), the
-    // FP32 lists of (dp|ds) and of the table-driven d-d bra classes ((dd|ps),
+    // FP32 lists of (dp|ds) and of the longer d-d bra classes ((dd|ps),
     // (dd|pp), (dd|ds), (dd|dp), (dd|dd)) follow them on the second stream.
     // Measured on mixed gradients at 1e-2: (H2O)32, FP64 lists 4.0% of the
     // tiles, 82.3 -> 76.2 ms (the second stream had stood idle for half the
