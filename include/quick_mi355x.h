@@ -137,7 +137,7 @@ int qk_prepare(qk_ctx* c, const qk_opts* o);
 /* Forward: dG <- G(dD), the two-electron operator (full symmetric n x n) for
  * the density dD; both device pointers, n x n doubles.  Runs on `stream`
  * (a hipStream_t, NULL = default) and returns after enqueueing; part of the
- * work also runs on three streams of the context, forked from `stream` and joined
+ * work runs on three streams of the context, forked from `stream` and joined
  * back to it with events. */
 int qk_fock_device(qk_ctx* c, const double* dD, double* dG, const qk_opts* o, void* stream);
 /* No counterpart in the reference.  For callers that cannot allocate device
