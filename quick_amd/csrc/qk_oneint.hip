@@ -166,7 +166,9 @@ constexpr double kPi = 3.14159265358979323846;
 // less than 1e-24 to any element and are skipped
 constexpr double k1eKabCut = 1e-24;
 
-// A lane's pair of shells and its walk over their primitive pairs
+// A lane's pair of shells and its walk over their primitive pairs.  A lane beyond
+// the batch's pairs walks none, but it runs the same code up to the wavefront's
+// sums: it holds the batch's first pair, so that what it reads belongs to that pair.
 struct OnePair {
     bool have;        // whether the lane has a pair
     int fA, fB;       // first functions
@@ -177,7 +179,7 @@ struct OnePair {
     __device__ __forceinline__ void load(const OneFuncs& f, const OneSys& sys, const int2* pairs, long long k, bool in,
                                          int first) {
         have = in;
-        const int2 pr = in ? pairs[k] : make_int2(0, 0);
+        const int2 pr = pairs[in ? k : 0];
         fA = pr.x; fB = pr.y;
         nB = f.np[fB];
         npp = in ? f.np[fA] * nB : 0;
@@ -238,7 +240,7 @@ struct OnePrim {
 // The pair list of a class holds first the pairs of many primitives, 2^kOneLog[0]
 // lanes each, then those of fewer: a lane walks at most about four primitive
 // pairs.  Calls use(first pair, pairs, lanes per pair log2) for the wavefront's
-// batch.
+// batch, which has at least one pair.
 template <class F>
 __device__ __forceinline__ void one_batches(const OnePairs& w, F&& use) {
     const long long wave0 = __builtin_amdgcn_readfirstlane(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6));
