@@ -311,14 +311,13 @@ struct qk_ctx {
     DBuf<int> d_sh_f0, d_sh_nf;
     DBuf<double> d_Dp, d_cm, d_D, d_G;
     DBuf<unsigned long long> d_X, d_counters;
-    // one-electron integrals: per basis function its atom, (l, m, n), primitive
-    // count, shell Qfinal, exponents and coefficients (10 per function), and
-    // the nuclear charges (qk_set_charges)
-    DBuf<int> d1_atom, d1_fn, d1_np, d1_qf;
-    // function pairs mu <= nu by total angular momentum l(mu) + l(nu) (0..4)
+    // one-electron integrals: the shells' components (OneFuncs), and the nuclear
+    // charges (qk_set_charges)
+    DBuf<int> d1_atom, d1_fn, d1_out, d1_np, d1_qf;
+    // their shell pairs by class
     DBuf<int2> d1_pairs[kNumPairClasses];
     OnePairs n1_pairs[kNumPairClasses] = {};
-    bool n1_whole = false, n1_cover = false;   // shells hold each component once; every function in a shell
+    bool n1_powers = false, n1_cover = false;   // no negative power in a shell; every function in a shell
     DBuf<double> d1_a, d1_c, d_chg;
     std::vector<double> chg;
     DBuf<unsigned long long> d1_acc;
@@ -564,48 +563,73 @@ extern "C" int qk_set_system(qk_ctx* c, int natom, const double* xyz, int nshell
         std::vector<int> qnc(c->q_L.size());
         for (size_t k = 0; k < qnc.size(); ++k) qnc[k] = ncart_of(c->q_L[k]);
         if (c->dq_nc.upload(qnc)) return -1;
-        // per basis function, for the one-electron integrals: the shell's
+        // the one-electron integrals' shells and slots (OneFuncs), with the shell's
         // exponents and the coefficients QUICK's attrashell applies,
-        // gccoeff(k, ksumtype + L) cons(f) (nuclear.f90:196-221)
-        std::vector<int> fat(nbasis), ffn(nbasis, -1), fnp(nbasis), fqf(nbasis);
-        c->n1_whole = true;
-        std::vector<double> fa(10 * (size_t)nbasis, 0.0), fc(10 * (size_t)nbasis, 0.0);
-        for (size_t q = 0; q < c->q_L.size(); ++q) {
-            const int sh = c->q_shell[q], L = c->q_L[q];
-            const int col = ksumtype[sh] - 1 + L;
-            for (int i = 0; i < ncart_of(L); ++i) {
-                const int fn = c->q_f0[q] + i;
-                fat[fn] = katom[sh] - 1;
-                // its component: x powers falling, then y powers falling
-                const int x = KLMN[3 * fn], y = KLMN[3 * fn + 1], z = KLMN[3 * fn + 2];
-                const bool ok = x >= 0 && y >= 0 && z >= 0 && x + y + z == L;
-                int* slot = ok ? &ffn[c->q_f0[q] + (L - x) * (L - x + 1) / 2 + z] : nullptr;
-                if (slot && *slot < 0) *slot = fn;
-                else c->n1_whole = false;
-                fnp[fn] = kprim[sh];
-                fqf[fn] = Qfinal[sh];
-                for (int u = 0; u < kprim[sh]; ++u) {
-                    fa[10 * (size_t)fn + u] = gcexpo[u + 10 * (size_t)col];
-                    fc[10 * (size_t)fn + u] = gccoeff[u + 10 * (size_t)col] * cons[fn];
-                }
+        // gccoeff(k, ksumtype + L) cons(f) (nuclear.f90:196-221).  A function that
+        // several Qshells claim belongs to the last of them.
+        const int nq = (int)c->q_L.size();
+        std::vector<int> owner(nbasis, -1);
+        for (int q = 0; q < nq; ++q)
+            for (int i = 0; i < ncart_of(c->q_L[q]); ++i) owner[c->q_f0[q] + i] = q;
+        std::vector<int> sat, sfn, sout, snp, sqf;
+        std::vector<double> sa, sc;
+        struct OneShell { int slot, L, q; };
+        std::vector<OneShell> shells;
+        c->n1_powers = true;
+        // function f (-1: none) as the next slot of Qshell q; an empty one stands for f0
+        auto slot = [&](int q, int f, int f0) {
+            const int sh = c->q_shell[q], col = ksumtype[sh] - 1 + c->q_L[q];
+            sat.push_back(katom[sh] - 1);
+            sfn.push_back(f < 0 ? f0 : f);
+            sout.push_back(f);
+            snp.push_back(kprim[sh]);
+            sqf.push_back(Qfinal[sh]);
+            for (int u = 0; u < k1eMaxPrim; ++u) {
+                const bool in = u < kprim[sh];
+                sa.push_back(in ? gcexpo[u + 10 * (size_t)col] : 0.0);
+                sc.push_back(in && f >= 0 ? gccoeff[u + 10 * (size_t)col] * cons[f] : 0.0);
+            }
+        };
+        // place of a function in its shell: x powers falling, then y powers falling
+        auto place = [&](int f, int L) { return (L - KLMN[3 * f]) * (L - KLMN[3 * f] + 1) / 2 + KLMN[3 * f + 2]; };
+        for (int q = 0; q < nq; ++q) {
+            const int L = c->q_L[q], n = ncart_of(L), f0 = c->q_f0[q];
+            int at[6] = {-1, -1, -1, -1, -1, -1};
+            bool whole = true;
+            for (int f = f0; f < f0 + n; ++f) {
+                const int* l = KLMN + 3 * (size_t)f;
+                if (l[0] < 0 || l[1] < 0 || l[2] < 0) c->n1_powers = whole = false;
+                else if (l[0] + l[1] + l[2] != L || owner[f] != q || at[place(f, L)] >= 0) whole = false;
+                else at[place(f, L)] = f;
+            }
+            if (whole) {
+                shells.push_back({(int)sfn.size(), L, q});
+                for (int k = 0; k < n; ++k) slot(q, at[k], f0);
+                continue;
+            }
+            for (int f = f0; f < f0 + n; ++f) {   // function by function
+                const int* l = KLMN + 3 * (size_t)f;
+                const int Lf = l[0] + l[1] + l[2];
+                if (owner[f] != q || l[0] < 0 || l[1] < 0 || l[2] < 0 || Lf > 2) continue;
+                shells.push_back({(int)sfn.size(), Lf, q});
+                for (int k = 0; k < ncart_of(Lf); ++k) slot(q, k == place(f, Lf) ? f : -1, f);
             }
         }
-        if (c->d1_atom.upload(fat) || c->d1_fn.upload(ffn) || c->d1_np.upload(fnp) || c->d1_qf.upload(fqf) ||
-            c->d1_a.upload(fa) || c->d1_c.upload(fc))
+        if (c->d1_atom.upload(sat) || c->d1_fn.upload(sfn) || c->d1_out.upload(sout) || c->d1_np.upload(snp) ||
+            c->d1_qf.upload(sqf) || c->d1_a.upload(sa) || c->d1_c.upload(sc))
             return -1;
         for (int fn = 0; fn < nbasis; ++fn)   // those outside every shell too
             if (KLMN[3 * fn] + KLMN[3 * fn + 1] + KLMN[3 * fn + 2] > 2) {
                 set_err("one-electron integrals: functions above d");
                 return -1;
             }
-        c->n1_cover = std::find(ffn.begin(), ffn.end(), -1) == ffn.end();
+        c->n1_cover = std::find(owner.begin(), owner.end(), -1) == owner.end();
         std::vector<int2> pl[kNumPairClasses][kOneBuckets];
-        const int nq = (int)c->q_L.size();
-        for (int i = 0; i < nq; ++i)
-            for (int j = i; j < nq; ++j) {
-                const int a = c->q_L[i] >= c->q_L[j] ? i : j, b = i + j - a;
-                const int npp = kprim[c->q_shell[a]] * kprim[c->q_shell[b]];
-                pl[pair_class_of(c->q_L[a], c->q_L[b])][one_bucket(npp)].push_back(make_int2(c->q_f0[a], c->q_f0[b]));
+        for (size_t i = 0; i < shells.size(); ++i)
+            for (size_t j = i; j < shells.size(); ++j) {
+                const OneShell &a = shells[shells[i].L >= shells[j].L ? i : j], &b = shells[shells[i].L >= shells[j].L ? j : i];
+                const int npp = kprim[c->q_shell[a.q]] * kprim[c->q_shell[b.q]];
+                pl[pair_class_of(a.L, b.L)][one_bucket(npp)].push_back(make_int2(a.slot, b.slot));
             }
         for (int k = 0; k < kNumPairClasses; ++k) {
             std::vector<int2> all;
@@ -1883,13 +1907,13 @@ extern "C" int qk_set_charges(qk_ctx* c, const double* charges) {
 static int oneint_ready(qk_ctx* c, const char* what) {
     if (!c || !c->have_system) { set_err("%s: no system", what); return -1; }
     if ((int)c->chg.size() != c->natom) { set_err("%s: nuclear charges not set (qk_set_charges)", what); return -1; }
-    if (!c->n1_whole) { set_err("%s: a shell does not hold each of its components once (KLMN)", what); return -1; }
+    if (!c->n1_powers) { set_err("%s: a function with a negative power (KLMN)", what); return -1; }
     (void)hipSetDevice(c->device);
     return 0;
 }
 
 static OneFuncs one_funcs(const qk_ctx* c) {
-    return OneFuncs{c->d1_atom.p, c->d1_fn.p, c->d1_np.p, c->d1_qf.p, c->d1_a.p, c->d1_c.p};
+    return OneFuncs{c->d1_atom.p, c->d1_fn.p, c->d1_out.p, c->d1_np.p, c->d1_qf.p, c->d1_a.p, c->d1_c.p};
 }
 
 // The one-electron kernels' streams: the classes are independent and few of them

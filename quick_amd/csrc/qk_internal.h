@@ -275,17 +275,22 @@ struct GradArgs {
     const float* boys_tab;   // kBoysTabRows x kBoysTabM
 };
 
-// One-electron integrals (qk_oneint.hip): per basis function its data, and the nuclei.
+// One-electron integrals (qk_oneint.hip): their shells' components, one slot
+// each.  A Qshell whose KLMN holds each component of its angular momentum once has
+// its slots in component order; any other is taken apart into shells of the
+// angular momentum that each function's KLMN gives, whose other components are
+// empty (coefficients 0).
 constexpr int k1eMaxPrim = 10;   // QUICK's MAXPRIM
 struct OneFuncs {
     const int* atom;     // 0-based
-    const int* fn;       // per shell (its first function's place onward): the function of each component
+    const int* fn;       // its function; of an empty component the function its shell holds
+    const int* out;      // its function; -1 for an empty component
     const int* np;       // primitives
     const int* qf;       // Qfinal of the function's shell (Boys order)
-    const double* a;     // k1eMaxPrim exponents per function
-    const double* c;     // k1eMaxPrim coefficients per function: gccoeff(k, ksumtype + L) cons(f)
+    const double* a;     // k1eMaxPrim exponents
+    const double* c;     // k1eMaxPrim coefficients: gccoeff(k, ksumtype + L) cons(f)
 };
-// The shell pairs of one class: (first functions of A and B, l(A) >= l(B)), in
+// The shell pairs of one class: (first slots of A and B, l(A) >= l(B)), in
 // buckets of 2^kOneLog lanes per pair: above 16 primitive pairs, 3 to 16, fewer
 constexpr int kOneBuckets = 3;
 constexpr int kOneLog[kOneBuckets] = {4, 2, 0};

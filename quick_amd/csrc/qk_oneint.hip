@@ -45,7 +45,7 @@ __device__ __forceinline__ void sfor(F&& f) {
 }
 
 // power of direction d in component k of a shell of angular momentum l: x powers
-// falling, then y powers falling (OneFuncs::fn holds the function of each)
+// falling, then y powers falling (the order of a shell's slots)
 __host__ __device__ constexpr int cart(int l, int k, int d) {
     for (int x = l; x >= 0; --x)
         for (int y = l - x; y >= 0; --y, --k)
@@ -171,7 +171,7 @@ constexpr double k1eKabCut = 1e-24;
 // sums: it holds the batch's first pair, so that what it reads belongs to that pair.
 struct OnePair {
     bool have;        // whether the lane has a pair
-    int fA, fB;       // first functions
+    int fA, fB;       // first slots
     int nB, npp;      // primitives of B, primitive pairs
     int atA, atB;
     double A[3], B[3], AB2;
@@ -232,8 +232,9 @@ struct OnePrim {
 #pragma unroll
         for (int d = 0; d < 3; ++d) asm volatile("" : "+v"(PA[d]), "+v"(PB[d]));
     }
-    __device__ __forceinline__ double coef(const OneFuncs& f, int I, int J) const {
-        return f.c[k1eMaxPrim * I + ci] * f.c[k1eMaxPrim * J + cj];
+    // of two slots
+    __device__ __forceinline__ double coef(const OneFuncs& f, int sA, int sB) const {
+        return f.c[k1eMaxPrim * sA + ci] * f.c[k1eMaxPrim * sB + cj];
     }
 };
 
@@ -308,7 +309,7 @@ __global__ void __launch_bounds__(256, LA + LB >= 2 && LA * LB > 0 ? 1 : 2)
                     constexpr int ib = decltype(ib_)::value;
                     constexpr int ax = cart(LA, ia, 0), ay = cart(LA, ia, 1), az = cart(LA, ia, 2);
                     constexpr int bx = cart(LB, ib, 0), by = cart(LB, ib, 1), bz = cart(LB, ib, 2);
-                    const double cc = o.coef(f, f.fn[q.fA + ia], f.fn[q.fB + ib]);
+                    const double cc = o.coef(f, q.fA + ia, q.fB + ib);
                     const double sx = t[0].s[ax][bx], sy = t[1].s[ay][by], sz = t[2].s[az][bz];
                     const double kx = t[0].template kin<ax, bx>(o.b), ky = t[1].template kin<ay, by>(o.b),
                                  kz = t[2].template kin<az, bz>(o.b);
@@ -342,7 +343,8 @@ __global__ void __launch_bounds__(256, LA + LB >= 2 && LA * LB > 0 ? 1 : 2)
 #pragma unroll
             for (int k = 0; k < NA * NB; ++k) {
                 if (q.fA == q.fB && k % NB < k / NB) continue;   // one shell: its lower half by symmetry
-                const int I = f.fn[q.fA + k / NB], J = f.fn[q.fB + k % NB];
+                const int I = f.out[q.fA + k / NB], J = f.out[q.fB + k % NB];
+                if (I < 0 || J < 0) continue;   // an empty component
                 const long long o1 = (long long)I * sys.n + J, o2 = (long long)J * sys.n + I;
                 if (S) S[o1] = S[o2] = so[k];
                 if (H) H[o1] = H[o2] = ho[k];
@@ -419,7 +421,7 @@ __global__ void __launch_bounds__(256, LA + LB >= 2 ? 1 : 2)
                     constexpr int ax = cart(LA, ia, 0), ay = cart(LA, ia, 1), az = cart(LA, ia, 2);
                     constexpr int bx = cart(LB, ib, 0), by = cart(LB, ib, 1), bz = cart(LB, ib, 2);
                     const int I = f.fn[q.fA + ia], J = f.fn[q.fB + ib];
-                    const double c = o.coef(f, I, J) * v0 * elem(Dm, I, J);
+                    const double c = o.coef(f, q.fA + ia, q.fB + ib) * v0 * elem(Dm, I, J);
                     sfor<ax + bx + 1>([&](auto t_) {
                         constexpr int tt = decltype(t_)::value;
                         const double ct = c * E[0].e[ax][bx][tt];
@@ -485,7 +487,7 @@ __global__ void __launch_bounds__(256, LA + LB >= 2 ? 1 : 2)
                     constexpr int la[3] = {cart(LA, ia, 0), cart(LA, ia, 1), cart(LA, ia, 2)};
                     constexpr int lb[3] = {cart(LB, ib, 0), cart(LB, ib, 1), cart(LB, ib, 2)};
                     const int I = f.fn[q.fA + ia], J = f.fn[q.fB + ib];
-                    const double cc = o.coef(f, I, J);
+                    const double cc = o.coef(f, q.fA + ia, q.fB + ib);
                     const double d = cc * elem(Dm, I, J), wv = cc * elem(Wm, I, J);
                     double sd[3], kd[3], dsd[3], dkd[3];
                     sfor<3>([&](auto d_) {

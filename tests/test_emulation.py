@@ -58,6 +58,70 @@ def test_functions_outside_every_shell(lib, k, low):
     assert dS <= 1e-12 and dH <= 1e-10 and free == 0.0 and dg <= 1e-10
 
 
+def odd_shells(kind):
+    """(tables for the library, basis for the oracle) of two waters with shells that do not hold each Cartesian
+    component of their angular momentum once"""
+    s, x = water_cluster(2, 1, 1, seed=5)
+    b = build_basis(s, np.asarray(x, float))
+    b.KLMN = b.KLMN.copy()
+    f0 = lambda sh, L: int(b.ksumtype[sh]) - 1 + int(b.Qsbasis[sh, L])
+    sp = next(i for i in range(b.nshell) if b.Qfinal[i] == 1)
+    d = next(i for i in range(b.nshell) if b.Qfinal[i] == 2)
+    if kind == "twice":        # p functions x, x, z
+        b.KLMN[:, f0(sp, 1) + 1] = b.KLMN[:, f0(sp, 1)]
+    elif kind == "other-l":    # a p function among the d, an s among the p, a p in an s shell
+        b.KLMN[:, f0(d, 2) + 3] = (0, 1, 0)
+        b.KLMN[:, f0(sp, 1) + 2] = 0
+    elif kind == "order":      # a permuted d shell stays whole
+        n = np.arange(f0(d, 2), f0(d, 2) + 6)
+        b.KLMN[:, n] = b.KLMN[:, n[[3, 5, 0, 4, 1, 2]]]
+    if kind != "shared":
+        return b, b
+    # a hydrogen's second s shell (one primitive) claims the function of its first (three)
+    h = next(i for i in range(b.nshell) if b.kprim[i] == 3 and b.Qfinal[i] == 0)
+    f = f0(h, 0)
+    c, o = copy.copy(b), copy.copy(b)
+    c.ksumtype = np.array(b.ksumtype)
+    c.ksumtype[h + 1] = c.ksumtype[h]
+    o.ncontract, o.dcoeff, o.aexp = b.ncontract.copy(), b.dcoeff.copy(), b.aexp.copy()
+    o.ncontract[f] = 1
+    o.dcoeff[:, f] = b.gccoeff[:, f] * b.cons[f]
+    o.aexp[:, f] = b.gcexpo[:, f]
+    o.ncontract[f + 1] = 0     # held by no shell now
+    return c, o
+
+
+def odd_shell_errors(kind):
+    """one-electron integrals and gradient of such a basis against the oracle's, which go function by function"""
+    from oracle import oracle as O
+    from quick_amd.fock import FockEngine
+    lib, ref = odd_shells(kind)
+    e = FockEngine(lib)
+    e.set_charges(ref.Z.astype(float))
+    S, H = e.oneint()
+    So, Ho = O.hcore(ref)
+    D, W = (synthetic_density(ref.xyz, ref.katom, ref.ksumtype, ref.nbasis, q) for q in (3, 4))
+    return np.abs(S - So).max(), np.abs(H - Ho).max(), np.abs(e.oneint_grad(D, W) - O.oneint_grad(ref, D, W)).max()
+
+
+ODD = ["twice", "other-l", "order", "shared"]
+
+
+@pytest.mark.parametrize("kind", ODD)
+def test_shells_without_each_component_once(lib, kind):
+    out = emulation.run(lib, f"from tests.test_emulation import *\nprint(*odd_shell_errors({kind!r}))")
+    dS, dH, dg = map(float, out.split())
+    assert dS <= 1e-12 and dH <= 1e-10 and dg <= 1e-10
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ODD)
+def test_shells_without_each_component_once_on_the_device(kind):
+    print(f"[gpu-test] odd shells: {kind}", flush=True)
+    dS, dH, dg = odd_shell_errors(kind)
+    assert dS <= 1e-12 and dH <= 1e-10 and dg <= 1e-10
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("k", [1, 6])
 def test_functions_outside_every_shell_on_the_device(k):
