@@ -1153,6 +1153,38 @@ static int fold_timing(qk_ctx* c) {
     return 0;
 }
 
+// The context's streams that a call works on beside the caller's.  They are
+// forked from it and joined back with events; a call that has forked joins on
+// every path, also after an error (later work on the caller's stream, or a
+// capture of it, has to be ordered after whatever the call put on them).
+constexpr int kForks = 3;
+static int join_streams(qk_ctx* c, hipStream_t s) {
+    hipError_t bad = hipSuccess;
+    for (int k = 0; k < kForks; ++k) {
+        hipError_t e = hipEventRecord(c->ev_cls[k], c->streams[k]);
+        if (e == hipSuccess) e = hipStreamWaitEvent(s, c->ev_cls[k], 0);
+        if (e != hipSuccess) bad = e;
+    }
+    if (bad != hipSuccess) { set_err("joining a stream failed: %s", hipGetErrorString(bad)); return -1; }
+    return 0;
+}
+// runs work() (0 or an error code) between fork and join
+template <class Work>
+static int with_streams(qk_ctx* c, hipStream_t s, Work&& work) {
+    HIPCHK(hipEventRecord(c->ev_start, s));
+    int rc = 0;
+    for (int k = 0; k < kForks && rc == 0; ++k) {
+        const hipError_t e = hipStreamWaitEvent(c->streams[k], c->ev_start, 0);
+        if (e != hipSuccess) { set_err("forking a stream failed: %s", hipGetErrorString(e)); rc = -1; }
+    }
+    if (rc == 0) rc = work();
+    if (rc == 0) return join_streams(c, s);
+    const std::string first = g_err;   // the work's error is the one to report
+    (void)join_streams(c, s);
+    g_err = first;
+    return rc;
+}
+
 // enqueue the whole build on `s` (classes fan out to the context's streams and join back)
 // (fb: the scratch to use; NULL = the context's own, preparing the work lists
 // for these options first)
@@ -1191,9 +1223,7 @@ static int fock_enqueue(qk_ctx* c, const double* dD, const double* dcutmat_or_nu
     // one such pair of streams: one water 545 -> 426 us, n-nonane 4.95 -> 4.34 ms,
     // (H2O)32 27.2 -> 26.5 ms, mixed at 1e-3 18.5 -> 17.5 ms.
     const hipStream_t s64 = c->streams[0];
-    HIPCHK(hipEventRecord(c->ev_start, s));
     const hipStream_t q4[4] = {s64, s, c->streams[1], c->streams[2]};
-    for (int k = 0; k < 3; ++k) HIPCHK(hipStreamWaitEvent(c->streams[k], c->ev_start, 0));
     // The classes of one stream run one after another, so at most four kernels
     // are in flight.  Kernels that spill get a grid small enough
     // that their private-segment backing stays under kScratchBudget
@@ -1210,109 +1240,109 @@ static int fock_enqueue(qk_ctx* c, const double* dD, const double* dcutmat_or_nu
         tiles32 += c->classes[k].ntiles32;
     }
     const bool light64 = mixed && tiles64 * 10 < tiles64 + tiles32;
-    for (size_t pos = 0; pos < order.size(); ++pos) {
-        const int k = order[pos];
-        ClassHost& CH = c->classes[k];
-        if (CH.ntiles == 0 && CH.ntiles32 == 0) continue;
-        // the stream of this class's FP64 list
-        const hipStream_t l64 = mixed ? (pos & 1 ? c->streams[1] : s64) : q4[pos & 3];
-        // one bra pair per block with its exchange rows in LDS, when they fit
-        const int nrow = bra_rows(k);
-        const size_t rows_lds = sizeof(unsigned long long) * (size_t)nrow * n;
-        const bool use_runs = fock_uses_runs(k, n, false), use_runs32 = fock_uses_runs(k, n, true);
-        // dynamic LDS of the thread-per-quartet kernels: the exchange rows and
-        // one bra slab (run mode), or four bra slabs (7 x 64 values each)
-        const size_t slab64 = 7 * 64 * sizeof(double), slab32 = 7 * 64 * sizeof(float);
-        // FP64 run mode: the bra rows of D in LDS too, where they fit kStageLds
-        // and leave the kernel as many resident blocks per CU as without them
-        // (measured on (H2O)32: FP64 build 38.4 -> 37.5 ms, psps 3.14 -> 2.73 ms;
-        // on (H2O)64 (ss|ss) staged fell from five blocks per CU to two, 16.6 ->
-        // 21.6 ms; in the FP32 kernels the second code path cost more than it saved)
-        const size_t drows64 = sizeof(double) * (size_t)nrow * n;
-        if (c->stage_n != n) {
-            for (int j = 0; j < kNumQuartetClasses; ++j) c->stage_ok[j] = -1;
-            c->stage_n = n;
-        }
-        if (use_runs && c->stage_ok[k] < 0) {
-            const size_t plain = rows_lds + slab64, staged = plain + drows64;
-            c->stage_ok[k] = staged <= kStageLds && fock_class_blocks(k, false, kStaged, staged) >=
-                                                        fock_class_blocks(k, false, kRuns, plain)
-                                 ? 1
-                                 : 0;
-        }
-        const bool stage64 = use_runs && c->stage_ok[k] == 1;
-        const size_t lds64 = use_runs ? rows_lds + slab64 + (stage64 ? drows64 : 0) : 4 * slab64;
-        const size_t lds32 = use_runs32 ? rows_lds + slab32 : 4 * slab32;
-        if (CH.ntiles) {
-            if (c->timing) HIPCHK(hipEventRecord(c->ev_t0[k], l64));
-            a.counters = fb->counters + 2 * k;
-            if (fock_class_is_team(k)) {
-                ClassWork w{CH.d_tiles.p, CH.ntiles, nullptr, 0};
-                // one 64-lane block per tile; up to 16 resident per CU
-                const int grid = (int)std::min<long long>(CH.ntiles, 256LL * 16);
-                launch_team_class(k, a, w, grid, l64);
-            } else {
-                const int mode = !use_runs ? kNoRuns : (stage64 ? kStaged : kRuns);
-                const long long cap = std::min(256LL * 16, scratch_grid_cap(fock_class_scratch(k, false, mode), 4));
-                ClassWork w{CH.d_tiles.p, CH.ntiles};
-                long long grid = (CH.ntiles + 3) / 4;   // 4 wavefronts per block
-                if (use_runs) {
-                    w.runs = CH.d_runs.p;
-                    w.nruns = CH.nruns;
-                    grid = share_runs(w, CH.lsplit);
-                    if (CH.compact && fb->compact) {
-                        // density screen first: every lane of the class kernel then has a quartet
-                        CompactArgs cq = ca;
-                        cq.steps = CH.d_steps.p;
-                        cq.slot0 = CH.d_slot0.p;
-                        launch_compact(cq, CH.d_segs.p, CH.nsegs, CH.d_list.p, l64);
-                        w.list = CH.d_list.p;
-                        w.steps = CH.d_steps.p;
-                    }
-                }
-                launch_fock_class(k, false, mode, a, w, (int)std::min(grid, cap), lds64, l64);
+    const auto classes = [&]() -> int {
+        for (size_t pos = 0; pos < order.size(); ++pos) {
+            const int k = order[pos];
+            ClassHost& CH = c->classes[k];
+            if (CH.ntiles == 0 && CH.ntiles32 == 0) continue;
+            // the stream of this class's FP64 list
+            const hipStream_t l64 = mixed ? (pos & 1 ? c->streams[1] : s64) : q4[pos & 3];
+            // one bra pair per block with its exchange rows in LDS, when they fit
+            const int nrow = bra_rows(k);
+            const size_t rows_lds = sizeof(unsigned long long) * (size_t)nrow * n;
+            const bool use_runs = fock_uses_runs(k, n, false), use_runs32 = fock_uses_runs(k, n, true);
+            // dynamic LDS of the thread-per-quartet kernels: the exchange rows and
+            // one bra slab (run mode), or four bra slabs (7 x 64 values each)
+            const size_t slab64 = 7 * 64 * sizeof(double), slab32 = 7 * 64 * sizeof(float);
+            // FP64 run mode: the bra rows of D in LDS too, where they fit kStageLds
+            // and leave the kernel as many resident blocks per CU as without them
+            // (measured on (H2O)32: FP64 build 38.4 -> 37.5 ms, psps 3.14 -> 2.73 ms;
+            // on (H2O)64 (ss|ss) staged fell from five blocks per CU to two, 16.6 ->
+            // 21.6 ms; in the FP32 kernels the second code path cost more than it saved)
+            const size_t drows64 = sizeof(double) * (size_t)nrow * n;
+            if (c->stage_n != n) {
+                for (int j = 0; j < kNumQuartetClasses; ++j) c->stage_ok[j] = -1;
+                c->stage_n = n;
             }
-            HIPCHK(hipGetLastError());
-            if (c->timing) HIPCHK(hipEventRecord(c->ev_t1[k], l64));
-            c->cls_timed[k] = c->timing;
-        }
-        if (mixed && CH.ntiles32) {
-            const hipStream_t ls = light64 && (k == 19 || k == 20) ? s64 : (pos & 1 ? c->streams[2] : s);
-            a.counters = fb->counters + 2 * kNumQuartetClasses + 2 * k;
-                    const int slot = kNumQuartetClasses + k;
-            if (c->timing) HIPCHK(hipEventRecord(c->ev_t0[slot], ls));
-            ClassWork w{CH.d_tiles32.p, CH.ntiles32};
-            if (fock_class_is_team(k)) {
-                // one 64-lane block per tile; up to 20 resident per CU (five wavefronts per SIMD)
-                launch_team_f32_class(k, a, w, (int)std::min<long long>(CH.ntiles32, 256LL * 20), ls);
-            } else {
-                const int mode = use_runs32 ? kRuns : kNoRuns;
-                const long long cap = std::min(256LL * 16, scratch_grid_cap(fock_class_scratch(k, true, mode), 4));
-                long long grid = (CH.ntiles32 + 3) / 4;
-                if (use_runs32) {
-                    w.runs = CH.d_runs32.p;
-                    w.nruns = CH.nruns32;
-                    grid = share_runs(w, CH.lsplit32);
-                    if (CH.compact32 && fb->compact) {
-                        CompactArgs cq = ca;
-                        cq.steps = CH.d_steps32.p;
-                        cq.slot0 = CH.d_slot032.p;
-                        launch_compact(cq, CH.d_segs32.p, CH.nsegs32, CH.d_list32.p, ls);
-                        w.list = CH.d_list32.p;
-                        w.steps = CH.d_steps32.p;
-                    }
-                }
-                launch_fock_class(k, true, mode, a, w, (int)std::min(grid, cap), lds32, ls);
+            if (use_runs && c->stage_ok[k] < 0) {
+                const size_t plain = rows_lds + slab64, staged = plain + drows64;
+                c->stage_ok[k] = staged <= kStageLds && fock_class_blocks(k, false, kStaged, staged) >=
+                                                            fock_class_blocks(k, false, kRuns, plain)
+                                     ? 1
+                                     : 0;
             }
-            HIPCHK(hipGetLastError());
-            if (c->timing) HIPCHK(hipEventRecord(c->ev_t1[slot], ls));
-            c->cls_timed[slot] = c->timing;
+            const bool stage64 = use_runs && c->stage_ok[k] == 1;
+            const size_t lds64 = use_runs ? rows_lds + slab64 + (stage64 ? drows64 : 0) : 4 * slab64;
+            const size_t lds32 = use_runs32 ? rows_lds + slab32 : 4 * slab32;
+            if (CH.ntiles) {
+                if (c->timing) HIPCHK(hipEventRecord(c->ev_t0[k], l64));
+                a.counters = fb->counters + 2 * k;
+                if (fock_class_is_team(k)) {
+                    ClassWork w{CH.d_tiles.p, CH.ntiles, nullptr, 0};
+                    // one 64-lane block per tile; up to 16 resident per CU
+                    const int grid = (int)std::min<long long>(CH.ntiles, 256LL * 16);
+                    launch_team_class(k, a, w, grid, l64);
+                } else {
+                    const int mode = !use_runs ? kNoRuns : (stage64 ? kStaged : kRuns);
+                    const long long cap = std::min(256LL * 16, scratch_grid_cap(fock_class_scratch(k, false, mode), 4));
+                    ClassWork w{CH.d_tiles.p, CH.ntiles};
+                    long long grid = (CH.ntiles + 3) / 4;   // 4 wavefronts per block
+                    if (use_runs) {
+                        w.runs = CH.d_runs.p;
+                        w.nruns = CH.nruns;
+                        grid = share_runs(w, CH.lsplit);
+                        if (CH.compact && fb->compact) {
+                            // density screen first: every lane of the class kernel then has a quartet
+                            CompactArgs cq = ca;
+                            cq.steps = CH.d_steps.p;
+                            cq.slot0 = CH.d_slot0.p;
+                            launch_compact(cq, CH.d_segs.p, CH.nsegs, CH.d_list.p, l64);
+                            w.list = CH.d_list.p;
+                            w.steps = CH.d_steps.p;
+                        }
+                    }
+                    launch_fock_class(k, false, mode, a, w, (int)std::min(grid, cap), lds64, l64);
+                }
+                HIPCHK(hipGetLastError());
+                if (c->timing) HIPCHK(hipEventRecord(c->ev_t1[k], l64));
+                c->cls_timed[k] = c->timing;
+            }
+            if (mixed && CH.ntiles32) {
+                const hipStream_t ls = light64 && (k == 19 || k == 20) ? s64 : (pos & 1 ? c->streams[2] : s);
+                a.counters = fb->counters + 2 * kNumQuartetClasses + 2 * k;
+                const int slot = kNumQuartetClasses + k;
+                if (c->timing) HIPCHK(hipEventRecord(c->ev_t0[slot], ls));
+                ClassWork w{CH.d_tiles32.p, CH.ntiles32};
+                if (fock_class_is_team(k)) {
+                    // one 64-lane block per tile; up to 20 resident per CU (five wavefronts per SIMD)
+                    launch_team_f32_class(k, a, w, (int)std::min<long long>(CH.ntiles32, 256LL * 20), ls);
+                } else {
+                    const int mode = use_runs32 ? kRuns : kNoRuns;
+                    const long long cap = std::min(256LL * 16, scratch_grid_cap(fock_class_scratch(k, true, mode), 4));
+                    long long grid = (CH.ntiles32 + 3) / 4;
+                    if (use_runs32) {
+                        w.runs = CH.d_runs32.p;
+                        w.nruns = CH.nruns32;
+                        grid = share_runs(w, CH.lsplit32);
+                        if (CH.compact32 && fb->compact) {
+                            CompactArgs cq = ca;
+                            cq.steps = CH.d_steps32.p;
+                            cq.slot0 = CH.d_slot032.p;
+                            launch_compact(cq, CH.d_segs32.p, CH.nsegs32, CH.d_list32.p, ls);
+                            w.list = CH.d_list32.p;
+                            w.steps = CH.d_steps32.p;
+                        }
+                    }
+                    launch_fock_class(k, true, mode, a, w, (int)std::min(grid, cap), lds32, ls);
+                }
+                HIPCHK(hipGetLastError());
+                if (c->timing) HIPCHK(hipEventRecord(c->ev_t1[slot], ls));
+                c->cls_timed[slot] = c->timing;
+            }
         }
-    }
-    for (int k = 0; k < 3; ++k) {
-        HIPCHK(hipEventRecord(c->ev_cls[k], c->streams[k]));
-        HIPCHK(hipStreamWaitEvent(s, c->ev_cls[k], 0));
-    }
+        return 0;
+    };
+    if (with_streams(c, s, classes)) return -1;
     launch_jpair_scatter(fb->J, c->dp_jofs.p, c->dp_pstride.p, c->dp_qa.p, c->dp_qb.p, a.q, c->nclass_pairs, fb->X,
                          n, s);
     launch_fock_finalize(fb->X, fb->xcopies, c->d_cons.p, dG, n, fb->counters + kRangeFlag, s);
@@ -1794,9 +1824,7 @@ static int grad_enqueue(qk_ctx* c, const double* dD, const double* dcutmat_or_nu
     // 22.6 -> 21.7 ms.  One kernel per stream is in flight, each within its
     // grid's scratch bound, so at most four bounded backings are live.
     const hipStream_t s64 = c->streams[0];
-    HIPCHK(hipEventRecord(c->ev_start, s));
     const hipStream_t q4[4] = {s64, s, c->streams[1], c->streams[2]};
-    for (int k = 0; k < 3; ++k) HIPCHK(hipStreamWaitEvent(c->streams[k], c->ev_start, 0));
     // When the FP64 lists are light (under 7.5% of the candidate tiles), the
     // FP32 lists of (dp|ds) and of the longer d-d bra classes ((dd|ps),
     // (dd|pp), (dd|ds), (dd|dp), (dd|dd)) follow them on the second stream.
@@ -1813,53 +1841,53 @@ static int grad_enqueue(qk_ctx* c, const double* dD, const double* dcutmat_or_nu
         tiles32 += c->ngtiles32[k];
     }
     const unsigned on_second = mixed && tiles64 * 40 < (tiles64 + tiles32) * 3 ? kFp32OnSecond : 0u;
-    for (int pass = 0; pass < (mixed ? 2 : 1); ++pass) {
-        const bool fp32 = pass == 1;
-        for (int k = 0; k < kNumQuartetClasses; ++k) {
-            const hipStream_t ls = fp32 ? (((on_second >> k) & 1u) ? s64 : (k & 1 ? c->streams[2] : s)) : (mixed ? (k & 1 ? c->streams[1] : s64) : q4[k & 3]);
-            const long long nt = fp32 ? c->ngtiles32[k] : c->ngtiles[k];
-            if (nt == 0) continue;
-            ClassWork w{(fp32 ? c->d_gtiles32[k] : c->d_gtiles[k]).p, nt};
-            a.counters = c->d_gcounters.p + 2 * (fp32 ? kNumQuartetClasses + k : k);
-            const int slot = (fp32 ? 3 : 2) * kNumQuartetClasses + k;
-            if (c->timing) HIPCHK(hipEventRecord(c->ev_t0[slot], ls));
-            w.lsplit = c->glsplit[fp32 ? 1 : 0][k];
-            if (grad_class_is_light(k) && w.lsplit == 0 && grad_compacts(k, fp32, mixed)) {
-                // density compaction, then the kernel over the queued steps
-                const int f = fp32 ? 1 : 0;
-                CompactArgs cq = ca;
-                cq.steps = c->d_gsteps[f][k].p;
-                cq.slot0 = c->d_gslot0[f][k].p;
-                launch_compact(cq, c->d_gsegs[f][k].p, c->ngsegs[f][k], c->d_glist[f][k].p, ls);
-                w.list = c->d_glist[f][k].p;
-                w.steps = cq.steps;
-                const int grid = (int)std::min<long long>(((nt << w.lsplit) + 3) / 4, 256LL * 8);
-                if (launch_grad_light(k, a, w, grid, fp32, ls)) {
-                    set_err("gradient kernel launch failed for class %d", k);
-                    return -1;
+    const auto classes = [&]() -> int {
+        for (int pass = 0; pass < (mixed ? 2 : 1); ++pass) {
+            const bool fp32 = pass == 1;
+            for (int k = 0; k < kNumQuartetClasses; ++k) {
+                const hipStream_t ls = fp32 ? (((on_second >> k) & 1u) ? s64 : (k & 1 ? c->streams[2] : s)) : (mixed ? (k & 1 ? c->streams[1] : s64) : q4[k & 3]);
+                const long long nt = fp32 ? c->ngtiles32[k] : c->ngtiles[k];
+                if (nt == 0) continue;
+                ClassWork w{(fp32 ? c->d_gtiles32[k] : c->d_gtiles[k]).p, nt};
+                a.counters = c->d_gcounters.p + 2 * (fp32 ? kNumQuartetClasses + k : k);
+                const int slot = (fp32 ? 3 : 2) * kNumQuartetClasses + k;
+                if (c->timing) HIPCHK(hipEventRecord(c->ev_t0[slot], ls));
+                w.lsplit = c->glsplit[fp32 ? 1 : 0][k];
+                if (grad_class_is_light(k) && w.lsplit == 0 && grad_compacts(k, fp32, mixed)) {
+                    // density compaction, then the kernel over the queued steps
+                    const int f = fp32 ? 1 : 0;
+                    CompactArgs cq = ca;
+                    cq.steps = c->d_gsteps[f][k].p;
+                    cq.slot0 = c->d_gslot0[f][k].p;
+                    launch_compact(cq, c->d_gsegs[f][k].p, c->ngsegs[f][k], c->d_glist[f][k].p, ls);
+                    w.list = c->d_glist[f][k].p;
+                    w.steps = cq.steps;
+                    const int grid = (int)std::min<long long>(((nt << w.lsplit) + 3) / 4, 256LL * 8);
+                    if (launch_grad_light(k, a, w, grid, fp32, ls)) {
+                        set_err("gradient kernel launch failed for class %d", k);
+                        return -1;
+                    }
+                } else if (grad_class_is_light(k)) {
+                    const int grid = (int)std::min<long long>(((nt << w.lsplit) + 3) / 4, 256LL * 8);
+                    if (launch_grad_light(k, a, w, grid, fp32, ls)) {
+                        set_err("gradient kernel launch failed for class %d", k);
+                        return -1;
+                    }
+                } else {
+                    const size_t lds = grad_lds_bytes(kGradBlobs[k], fp32);
+                    const int grid = (int)std::min<long long>(nt, 256LL * (fp32 ? 20 : 16));
+                    if (launch_grad_class(a, w, c->d_gtab[k].p, lds, grid, fp32, ls)) {
+                        set_err("gradient kernel launch failed for class %d (%zu bytes LDS)", k, lds);
+                        return -1;
+                    }
                 }
-            } else if (grad_class_is_light(k)) {
-                const int grid = (int)std::min<long long>(((nt << w.lsplit) + 3) / 4, 256LL * 8);
-                if (launch_grad_light(k, a, w, grid, fp32, ls)) {
-                    set_err("gradient kernel launch failed for class %d", k);
-                    return -1;
-                }
-            } else {
-                const size_t lds = grad_lds_bytes(kGradBlobs[k], fp32);
-                const int grid = (int)std::min<long long>(nt, 256LL * (fp32 ? 20 : 16));
-                if (launch_grad_class(a, w, c->d_gtab[k].p, lds, grid, fp32, ls)) {
-                    set_err("gradient kernel launch failed for class %d (%zu bytes LDS)", k, lds);
-                    return -1;
-                }
+                if (c->timing) HIPCHK(hipEventRecord(c->ev_t1[slot], ls));
+                c->cls_timed[slot] = c->timing;
             }
-            if (c->timing) HIPCHK(hipEventRecord(c->ev_t1[slot], ls));
-            c->cls_timed[slot] = c->timing;
         }
-    }
-    for (int k = 0; k < 3; ++k) {
-        HIPCHK(hipEventRecord(c->ev_cls[k], c->streams[k]));
-        HIPCHK(hipStreamWaitEvent(s, c->ev_cls[k], 0));
-    }
+        return 0;
+    };
+    if (with_streams(c, s, classes)) return -1;
     launch_grad_finalize(c->d_gacc.p, dgrad, 3 * c->natom, c->d_gcounters.p + kGradRangeFlag, s);
     HIPCHK(hipGetLastError());
     return 0;
@@ -1920,20 +1948,9 @@ static OneFuncs one_funcs(const qk_ctx* c) {
 // fill the GPU, so they go out on the caller's stream and three of the context's,
 // forked from it and joined after (measured with the gradient's rows of blocks:
 // integrals and gradient of (H2O)32 4.83 -> 3.31 ms)
-constexpr int kOneStreams = 3;
-static int one_fork(qk_ctx* c, hipStream_t s, hipStream_t* of) {
-    HIPCHK(hipEventRecord(c->ev_start, s));
-    for (int k = 0; k < kOneStreams; ++k) HIPCHK(hipStreamWaitEvent(c->streams[k], c->ev_start, 0));
+static void one_streams(const qk_ctx* c, hipStream_t s, hipStream_t* of) {
     static const int where[kNumPairClasses] = {-1, 0, 1, 1, 2, 2};
     for (int k = 0; k < kNumPairClasses; ++k) of[k] = where[k] < 0 ? s : c->streams[where[k]];
-    return 0;
-}
-static int one_join(qk_ctx* c, hipStream_t s) {
-    for (int k = 0; k < kOneStreams; ++k) {
-        HIPCHK(hipEventRecord(c->ev_cls[k], c->streams[k]));
-        HIPCHK(hipStreamWaitEvent(s, c->ev_cls[k], 0));
-    }
-    return 0;
 }
 
 extern "C" int qk_oneint_device(qk_ctx* c, double* dS, double* dH, void* stream) {
@@ -1943,12 +1960,12 @@ extern "C" int qk_oneint_device(qk_ctx* c, double* dS, double* dH, void* stream)
         for (double* p : {dS, dH})
             if (p) launch_fill_u64((unsigned long long*)p, (long long)c->nbasis * c->nbasis, (hipStream_t)stream);
     hipStream_t of[kNumPairClasses];
-    if (one_fork(c, (hipStream_t)stream, of)) return -1;
-    launch_oneint(one_funcs(c), sys, c->n1_pairs, dS, dH, of);
-    const hipError_t launched = hipGetLastError();   // joined also where a launch failed
-    if (one_join(c, (hipStream_t)stream)) return -1;
-    HIPCHK(launched);
-    return 0;
+    one_streams(c, (hipStream_t)stream, of);
+    return with_streams(c, (hipStream_t)stream, [&]() -> int {
+        launch_oneint(one_funcs(c), sys, c->n1_pairs, dS, dH, of);
+        HIPCHK(hipGetLastError());
+        return 0;
+    });
 }
 
 extern "C" int qk_nuclear_repulsion(qk_ctx* c, double* E) {
@@ -1976,11 +1993,13 @@ extern "C" int qk_oneint_grad_device(qk_ctx* c, const double* dD, const double* 
     launch_fill_u64(c->d1_acc.p, m + 1, s);
     const OneSys sys{c->d_xyz.p, c->d_chg.p, c->natom, c->nbasis};
     hipStream_t of[kNumPairClasses];
-    if (one_fork(c, s, of)) return -1;
-    launch_oneint_grad(one_funcs(c), sys, c->n1_pairs, dD, dW, c->d1_acc.p, of);
-    const hipError_t launched = hipGetLastError();
-    if (one_join(c, s)) return -1;
-    HIPCHK(launched);
+    one_streams(c, s, of);
+    const auto classes = [&]() -> int {
+        launch_oneint_grad(one_funcs(c), sys, c->n1_pairs, dD, dW, c->d1_acc.p, of);
+        HIPCHK(hipGetLastError());
+        return 0;
+    };
+    if (with_streams(c, s, classes)) return -1;
     launch_grad_finalize(c->d1_acc.p, dgrad, m, c->d1_acc.p + m, s);
     HIPCHK(hipGetLastError());
     return 0;

@@ -128,3 +128,48 @@ def test_functions_outside_every_shell_on_the_device(k):
     print(f"[gpu-test] {k} functions outside every shell", flush=True)
     dS, dH, free, dg = free_function_errors(k)
     assert dS <= 1e-12 and dH <= 1e-10 and free == 0.0 and dg <= 1e-10
+
+
+JOIN = """
+from tests.emulation import without_d
+from quick_amd.basis import build_basis
+from quick_amd.geometry import synthetic_density
+b = without_d(build_basis(["H", "H"], np.array([[0.0, 0.0, 0.0], [0.3, 0.5, 0.7]])))
+D = synthetic_density(b.xyz, b.katom, b.ksumtype, b.nbasis, 3).ravel(order="F").copy()
+W = D.copy()
+e = FockEngine(b)
+e.compute_schwarz()
+e.set_charges([1.0, 1.0])
+emu.emu_fail_in.argtypes = [C.c_longlong]
+o = make_opts(**KW)
+e.prepare(o)
+p = lambda a: C.c_void_p(a.ctypes.data)
+calls = {"fock": lambda x: lib().qk_fock_device(e.h, p(D), p(x), C.byref(o), None),
+         "grad": lambda x: lib().qk_grad_device(e.h, p(D), p(x), C.byref(o), None),
+         "oneint": lambda x: lib().qk_oneint_device(e.h, p(x), None, None),
+         "oneint_grad": lambda x: lib().qk_oneint_grad_device(e.h, p(D), p(W), p(x), None)}
+for name, call in calls.items():
+    new = lambda: np.zeros(3 * b.natom if "grad" in name else b.nbasis ** 2)
+    good = new()
+    assert call(good) == 0 and emu.emu_unjoined() == 0, name
+    failed = 0
+    for n in range(1000):
+        emu.emu_fail_in(n)
+        rc = call(new())
+        emu.emu_fail_in(-1)
+        assert emu.emu_unjoined() == 0, f"{name}: error {n} leaves {emu.emu_unjoined()} streams forked"
+        if rc == 0:
+            break
+        failed += 1
+        again = new()
+        assert call(again) == 0 and np.array_equal(again, good), f"{name} after error {n}"
+    print(name, failed)
+"""
+
+
+@pytest.mark.parametrize("kw", ["dict()", "dict(precision=QK_MIXED, fp32_threshold=1e-1)"], ids=["fp64", "mixed"])
+def test_streams_are_joined_after_any_error(lib, kw):
+    """every launch check of a call fails once: the call reports it, the streams it forked are ordered before what
+    follows on the caller's, and the next call gives the same result as before"""
+    out = dict(line.split() for line in emulation.run(lib, JOIN.replace("KW", kw)).splitlines())
+    assert int(out["fock"]) >= 8 and int(out["grad"]) >= 8 and int(out["oneint"]) and int(out["oneint_grad"]), out
