@@ -587,9 +587,7 @@ __global__ void nuclear_grad_kernel(const OneSys sys, unsigned long long* __rest
     }
 }
 
-// one launch per class of shell pairs (lists built on the host once per system);
-// the (d|d) gradient is the one kernel here that spills (its grid of one block per
-// CU bounds the scratch backing)
+// one launch per class of shell pairs (lists built on the host once per system)
 static int one_grid(const OnePairs& w, long long per_cu = 8) {
     long long waves = 0;
     for (int b = 0; b < kOneBuckets; ++b) waves += (w.n[b] + (64 >> kOneLog[b]) - 1) / (64 >> kOneLog[b]);
@@ -614,13 +612,20 @@ void launch_oneint(const OneFuncs& f, const OneSys& sys, const OnePairs* w, doub
 // pair).  Measured on (H2O)32: (d|d) 277 -> 87 us, (d|s) 228 -> 93 us.
 static int one_rows(int grid, int natom) { return std::max(1, std::min({8, 512 / grid, natom / 8})); }
 
+// (d|d) is the one class here that spills; it takes one block per CU, and its grid,
+// rows and all, keeps its scratch backing under the bound
 void launch_oneint_grad(const OneFuncs& f, const OneSys& sys, const OnePairs* w, const double* D, const double* W,
                         unsigned long long* G, const hipStream_t* s) {
     const size_t lds = sizeof(unsigned long long) * 3 * (size_t)sys.natom;
 #define QK_1E(k, la, lb)                                                                                      \
-    if (const int grid = one_grid(w[k], la + lb == 4 ? 1 : 8))                                               \
-        hipLaunchKernelGGL((oneint_grad_kernel<la, lb>), dim3(grid, one_rows(grid, sys.natom)), dim3(256), lds, \
-                           s[k], f, sys, w[k], D, W, G);
+    if (int grid = one_grid(w[k], la + lb == 4 ? 1 : 8)) {                                                    \
+        static const long long cap =                                                                          \
+            scratch_grid_cap(kernel_scratch(reinterpret_cast<const void*>(&oneint_grad_kernel<la, lb>)), 4);  \
+        grid = (int)std::min<long long>(grid, cap);                                                           \
+        const int rows = (int)std::min<long long>(one_rows(grid, sys.natom), cap / grid);                     \
+        hipLaunchKernelGGL((oneint_grad_kernel<la, lb>), dim3(grid, rows), dim3(256), lds, s[k], f, sys, w[k], D, W, \
+                           G);                                                                                \
+    }
     QK_1E_CLASSES(QK_1E)
 #undef QK_1E
     hipLaunchKernelGGL(nuclear_grad_kernel, dim3((sys.natom + 255) / 256), dim3(256), 0, s[0], sys, G);

@@ -75,6 +75,12 @@ def build(out: Path, jobs: int = 8) -> Path:
     return lib
 
 
+def symbols(lib: Path) -> list[str]:
+    """the functions the library exports"""
+    txt = subprocess.run(["nm", "-D", "--defined-only", str(lib)], check=True, capture_output=True, text=True).stdout
+    return [line.split()[-1] for line in txt.splitlines() if line.split()[-2] in "TWtwVu"]
+
+
 def run(lib: Path, code: str, low: bool = False, timeout: int = 600) -> str:
     """runs `code` in a child process whose quick_amd loads the emulated library"""
     env = {**os.environ, "QUICK_MI355X_LIB": str(lib), "OMP_NUM_THREADS": "1"}

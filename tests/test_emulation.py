@@ -173,3 +173,43 @@ def test_streams_are_joined_after_any_error(lib, kw):
     follows on the caller's, and the next call gives the same result as before"""
     out = dict(line.split() for line in emulation.run(lib, JOIN.replace("KW", kw)).splitlines())
     assert int(out["fock"]) >= 8 and int(out["grad"]) >= 8 and int(out["oneint"]) and int(out["oneint_grad"]), out
+
+
+SCRATCH = """
+from tests.emulation import without_d
+from quick_amd.basis import build_basis
+from quick_amd.geometry import synthetic_density, water_cluster
+emu.emu_set_scratch.argtypes = [C.c_char_p, C.c_longlong]
+for name in NAMES:
+    emu.emu_set_scratch(name.encode(), 1 << 20)
+def both(b):
+    D = synthetic_density(b.xyz, b.katom, b.ksumtype, b.nbasis, 3)
+    e = FockEngine(b)
+    e.set_charges(b.Z.astype(float))
+    return e, D
+s, x = water_cluster(3, 2, 1, seed=2)
+e, D = both(build_basis(s, np.asarray(x, float)))
+e.oneint_grad(D, D)
+e, D = both(without_d(build_basis(["H"] * 3, np.array([[0.0, 0.0, 0.0], [0.3, 0.5, 0.7], [1.1, 0.2, 0.4]]))))
+e.compute_schwarz()
+for o in (make_opts(), make_opts(precision=QK_MIXED, fp32_threshold=1e-1)):
+    e.fock(D, o), e.grad(D, o)
+print(emu.emu_record().decode())
+"""
+
+
+def test_grids_of_spilling_kernels(lib):
+    """the grids that the launchers really use, were every kernel that can spill to take 1 MiB per lane (the budget
+    then holds one block of 256 threads): no launch may back more than the budget"""
+    names = ["oneint_grad_kernel", "grad_light_kernel", "fock_kernel"]
+    nm = emulation.symbols(lib)
+    spill = [n for n in nm if any(k in n for k in names) and "launch" not in n]
+    assert len(spill) >= 6 + 12 + 12
+    seen = set()
+    for line in emulation.run(lib, SCRATCH.replace("NAMES", repr(spill))).split("\n"):
+        if line:
+            name, grid, block, _, _ = line.split()
+            if name in spill:
+                seen.add(name)
+                assert int(grid) == 1 and int(block) == 256, line
+    assert len(seen) >= 6 + 6 + 6
