@@ -122,7 +122,7 @@ __device__ __forceinline__ float rsqrt_nr(float x) { return __builtin_amdgcn_rsq
 // exp(-X), X >= 0: X = -k ln2 - r with |r| <= ln2 / 2 (ln2 in two parts, the
 // high one exact times k below 2^21), exp(r) by the degree-11 interpolant at the
 // Chebyshev nodes of the interval (largest relative error 1.7e-17), scaled by 2^k
-// (to zero beyond the range)
+// (to zero beyond the range; X up to 1e44, where r's error would overflow p)
 __device__ __forceinline__ double exp_neg(double X) {
     const double k = __builtin_rint(X * -1.4426950408889634);
     const double r = fma(k, -1.9082149292705877e-10, fma(k, -0.6931471803691238, -X));

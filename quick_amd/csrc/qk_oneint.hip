@@ -238,6 +238,15 @@ struct OnePrim {
     }
 };
 
+// QUICK's fit, with exp(-T) for any T: a nucleus may lie farther away than exp_neg
+// can carry (exp(-T) is zero from T = 746 on)
+template <int L>
+__device__ __forceinline__ void boys_one(double T, int M, const double* __restrict__ tab, double* F) {
+    const double E = exp_neg(fmin(T, 800.0));
+    boys_fit_main<L>(T, E, tab, F);
+    if (!boys_fit_up(T, M)) boys_fit_near0<L>(T, E, M, F);
+}
+
 // The pair list of a class holds first the pairs of many primitives, 2^kOneLog[0]
 // lanes each, then those of fewer: a lane walks at most about four primitive
 // pairs.  Calls use(first pair, pairs, lanes per pair log2) for the wavefront's
@@ -287,7 +296,7 @@ __global__ void __launch_bounds__(256, LA + LB >= 2 && LA * LB > 0 ? 1 : 2)
                     const double PC[3] = {o.P[0] - sys.xyz[3 * C], o.P[1] - sys.xyz[3 * C + 1],
                                           o.P[2] - sys.xyz[3 * C + 2]};
                     double F[L + 1], R0[NT];
-                    boys_fit<L>(o.p * (PC[0] * PC[0] + PC[1] * PC[1] + PC[2] * PC[2]), M, s_boys, F);
+                    boys_one<L>(o.p * (PC[0] * PC[0] + PC[1] * PC[1] + PC[2] * PC[2]), M, s_boys, F);
                     hermite_r_u<L>(o.p, PC, F, R0);
                     const double z = -sys.chg[C];
 #pragma unroll
@@ -440,7 +449,7 @@ __global__ void __launch_bounds__(256, LA + LB >= 2 ? 1 : 2)
             for (int C = C0; C < C1; ++C) {
                 const double PC[3] = {o.P[0] - sys.xyz[3 * C], o.P[1] - sys.xyz[3 * C + 1], o.P[2] - sys.xyz[3 * C + 2]};
                 double F[L + 2], R0[tet_size(L + 1)];
-                boys_fit<L + 1>(o.p * (PC[0] * PC[0] + PC[1] * PC[1] + PC[2] * PC[2]), M, s_boys, F);
+                boys_one<L + 1>(o.p * (PC[0] * PC[0] + PC[1] * PC[1] + PC[2] * PC[2]), M, s_boys, F);
                 hermite_r_u<L + 1>(o.p, PC, F, R0);
                 // one-centre terms add up to zero
                 const double z = q.atA == C && q.atB == C ? 0.0 : -sys.chg[C];

@@ -213,3 +213,28 @@ def test_grids_of_spilling_kernels(lib):
                 seen.add(name)
                 assert int(grid) == 1 and int(block) == 256, line
     assert len(seen) >= 6 + 6 + 6
+
+
+def far_charge_errors():
+    """a hydrogen molecule and a bare charge 1e25 bohr away, against the oracle: |dH|, |d one-electron grad|"""
+    from oracle import oracle as O
+    from quick_amd.fock import FockEngine
+    b = build_basis(["H", "H"], np.array([[0.0, 0.0, 0.0], [0.3, 0.5, 0.7]]))
+    b.xyz = np.asfortranarray(np.concatenate([b.xyz, [[1e25], [0.0], [0.0]]], axis=1))
+    b.Z = np.array([1, 1, 1])
+    D, W = (synthetic_density(b.xyz, b.katom, b.ksumtype, b.nbasis, q) for q in (3, 4))
+    e = FockEngine(b)
+    e.set_charges(b.Z.astype(float))
+    return np.abs(e.oneint()[1] - O.hcore(b)[1]).max(), np.abs(e.oneint_grad(D, W) - O.oneint_grad(b, D, W)).max()
+
+
+def test_charge_very_far_away(lib):
+    """Boys arguments of 1e50, beyond what exp's reduction can carry: finite, as the oracle has them"""
+    out = emulation.run(lib, "from tests.test_emulation import *\nprint(*far_charge_errors())")
+    assert all(float(v) <= 1e-10 for v in out.split()), out
+
+
+@pytest.mark.gpu
+def test_charge_very_far_away_on_the_device():
+    print("[gpu-test] a charge very far away", flush=True)
+    assert all(v <= 1e-10 for v in far_charge_errors())
