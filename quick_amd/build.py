@@ -38,7 +38,7 @@ def _compile(src: Path, verbose: bool) -> Path:
     obj = OBJ / (src.stem + ".o")
     deps = [src, CSRC / "qk_kernels.h", CSRC / "qk_internal.h", CSRC / "eri_generated.inc",
             CSRC / "qk_team.h", CSRC / "team_tables.inc", CSRC / "grad_tables.inc", CSRC / "grad_fold.inc",
-            CSRC / "qk_grad_light.h", CSRC / "xc_b3lyp.inc", CSRC / "lebedev.inc",
+            CSRC / "qk_grad_light.h", CSRC / "qk_xc_deal.h", CSRC / "xc_b3lyp.inc", CSRC / "lebedev.inc",
             HERE.parent / "include" / "quick_mi355x.h", Path(__file__)]
     if obj.exists() and all(obj.stat().st_mtime >= d.stat().st_mtime for d in deps if d.exists()):
         return obj

@@ -36,6 +36,7 @@
 
 #include "quick_mi355x.h"
 #include "qk_internal.h"
+#include "qk_xc_deal.h"
 
 #define QK_HD __host__ __device__
 #include "xc_b3lyp.inc"
@@ -47,7 +48,6 @@ constexpr int kXcMaxPrim = 10;     // QUICK's MAXPRIM
 constexpr int kXcBatch = 256;      // grid points per batch
 constexpr int kXcTile = 64;        // GEMM tile (rows and columns)
 constexpr int kXcShellThreads = 320;
-constexpr int kXcds = 8;             // accelerator dies, each with its own L2
 constexpr double kXcFix = 0x1p48;  // V accumulator units
 
 typedef double v4d __attribute__((ext_vector_type(4)));
@@ -999,21 +999,9 @@ static int xc_finish_grid(qk_xc* x, XBuf<double>& pts_in, XBuf<int>& atom_in, lo
     x->chunks.clear();
     qk_xc::Chunk ch;
     long long ws = 0, part = 0, maxws = 0, maxpart = 0;
-    // A chunk's tasks are dealt to the eight XCDs by batch (block b of a launch
-    // runs on XCD b % 8), each batch to the one with the fewest tasks so far: the
-    // tiles of a batch that several tasks read then come from one L2.  Tasks of
-    // batch -1 fill the shorter queues.  (Measured on (H2O)64: xc_rho_gemm 9.9 -> 9.65 ms.)
-    std::vector<int4> rho_q[kXcds], v_q[kXcds];
-    auto deal = [](std::vector<int4>* q, std::vector<int4>& out) {
-        size_t len = 0;
-        for (int x = 0; x < kXcds; ++x) len = std::max(len, q[x].size());
-        for (size_t i = 0; i < len; ++i)
-            for (int x = 0; x < kXcds; ++x) out.push_back(i < q[x].size() ? q[x][i] : int4{-1, 0, 0, 0});
-        for (int x = 0; x < kXcds; ++x) q[x].clear();
-    };
+    XcDeal<int4> deal;
     auto end_chunk = [&] {
-        deal(rho_q, rho_t);
-        deal(v_q, v_t);
+        deal.finish(rho_t, v_t);
         ch.nrho = (long long)rho_t.size() - ch.rho0;
         ch.nv = (long long)v_t.size() - ch.v0;
         x->chunks.push_back(ch);
@@ -1049,13 +1037,11 @@ static int xc_finish_grid(qk_xc* x, XBuf<double>& pts_in, XBuf<int>& atom_in, lo
         ch.nb += 1;
         if (m == 0) continue;
         const int T = w / kXcTile;
-        int xcd = 0;
-        for (int k = 1; k < kXcds; ++k)
-            if (v_q[k].size() < v_q[xcd].size()) xcd = k;
+        deal.begin_batch();
         for (int r = 0; r < kXcBatch / kXcTile; ++r)
-            for (int c = 0; c < T; ++c) rho_q[xcd].push_back(int4{local, r, c, 0});
+            for (int c = 0; c < T; ++c) deal.rho(int4{local, r, c, 0});
         for (int I = 0; I < T; ++I)
-            for (int J = 0; J <= I; ++J) v_q[xcd].push_back(int4{local, I, J, 0});
+            for (int J = 0; J <= I; ++J) deal.v(int4{local, I, J, 0});
         x->flops += 2.0 * kXcBatch * (double)w * w + 2.0 * 2.0 * kXcBatch * kXcTile * kXcTile * (T * (T + 1) / 2);
     }
     if (ch.nb > 0) end_chunk();
