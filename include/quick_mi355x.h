@@ -240,8 +240,10 @@ int qk_num_classes(void);
 int qk_class_info(qk_ctx* c, int k, int* lalblcld, long long* work);
 /* Fraction of wavefront lanes the work tiles of class k occupy (0..1). */
 double qk_class_lane_fill(qk_ctx* c, int k);
-/* Record HIP events around every class kernel of the following builds (on the
- * stream the kernels run on). */
+/* Record HIP events around every class kernel of the following builds and
+ * gradients.  While this is on the kernels run one after another on the caller's
+ * stream, so that each class's time is its own (its density compaction included);
+ * the calls then take longer than on their four streams. */
 int qk_set_timing(qk_ctx* c, int on);
 /* Figures of class k's FP64 kernel in the last build: surviving quartets,
  * primitive quartets, algorithmic flops; and the kernel's average time in ms

@@ -1221,7 +1221,8 @@ static int fock_enqueue(qk_ctx* c, const double* dD, const double* dcutmat_or_nu
     // the FP64 lists, which hold the few strongest pairs (long ket ranges on few
     // bras), go to two of them and the FP32 lists to the others.  Measured against
     // one such pair of streams: one water 545 -> 426 us, n-nonane 4.95 -> 4.34 ms,
-    // (H2O)32 27.2 -> 26.5 ms, mixed at 1e-3 18.5 -> 17.5 ms.
+    // (H2O)32 27.2 -> 26.5 ms, mixed at 1e-3 18.5 -> 17.5 ms.  With per-class timing
+    // on, all go to the caller's stream: each time is then one class's alone.
     const hipStream_t s64 = c->streams[0];
     const hipStream_t q4[4] = {s64, s, c->streams[1], c->streams[2]};
     // The classes of one stream run one after another, so at most four kernels
@@ -1246,7 +1247,7 @@ static int fock_enqueue(qk_ctx* c, const double* dD, const double* dcutmat_or_nu
             ClassHost& CH = c->classes[k];
             if (CH.ntiles == 0 && CH.ntiles32 == 0) continue;
             // the stream of this class's FP64 list
-            const hipStream_t l64 = mixed ? (pos & 1 ? c->streams[1] : s64) : q4[pos & 3];
+            const hipStream_t l64 = c->timing ? s : mixed ? (pos & 1 ? c->streams[1] : s64) : q4[pos & 3];
             // one bra pair per block with its exchange rows in LDS, when they fit
             const int nrow = bra_rows(k);
             const size_t rows_lds = sizeof(unsigned long long) * (size_t)nrow * n;
@@ -1308,7 +1309,7 @@ static int fock_enqueue(qk_ctx* c, const double* dD, const double* dcutmat_or_nu
                 c->cls_timed[k] = c->timing;
             }
             if (mixed && CH.ntiles32) {
-                const hipStream_t ls = light64 && (k == 19 || k == 20) ? s64 : (pos & 1 ? c->streams[2] : s);
+                const hipStream_t ls = c->timing ? s : light64 && (k == 19 || k == 20) ? s64 : (pos & 1 ? c->streams[2] : s);
                 a.counters = fb->counters + 2 * kNumQuartetClasses + 2 * k;
                 const int slot = kNumQuartetClasses + k;
                 if (c->timing) HIPCHK(hipEventRecord(c->ev_t0[slot], ls));
@@ -1845,7 +1846,10 @@ static int grad_enqueue(qk_ctx* c, const double* dD, const double* dcutmat_or_nu
         for (int pass = 0; pass < (mixed ? 2 : 1); ++pass) {
             const bool fp32 = pass == 1;
             for (int k = 0; k < kNumQuartetClasses; ++k) {
-                const hipStream_t ls = fp32 ? (((on_second >> k) & 1u) ? s64 : (k & 1 ? c->streams[2] : s)) : (mixed ? (k & 1 ? c->streams[1] : s64) : q4[k & 3]);
+                const hipStream_t ls =
+                    c->timing ? s
+                    : fp32    ? (((on_second >> k) & 1u) ? s64 : (k & 1 ? c->streams[2] : s))
+                              : (mixed ? (k & 1 ? c->streams[1] : s64) : q4[k & 3]);
                 const long long nt = fp32 ? c->ngtiles32[k] : c->ngtiles[k];
                 if (nt == 0) continue;
                 ClassWork w{(fp32 ? c->d_gtiles32[k] : c->d_gtiles[k]).p, nt};

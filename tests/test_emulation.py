@@ -238,3 +238,29 @@ def test_charge_very_far_away(lib):
 def test_charge_very_far_away_on_the_device():
     print("[gpu-test] a charge very far away", flush=True)
     assert all(v <= 1e-10 for v in far_charge_errors())
+
+
+TIMING = """
+from tests.emulation import without_d
+from quick_amd.basis import build_basis
+from quick_amd.geometry import synthetic_density
+b = without_d(build_basis(["H", "H"], np.array([[0.0, 0.0, 0.0], [0.3, 0.5, 0.7]])))
+D = synthetic_density(b.xyz, b.katom, b.ksumtype, b.nbasis, 3)
+e = FockEngine(b)
+e.compute_schwarz()
+for on in (False, True):
+    e.set_timing(on)
+    for o in (make_opts(), make_opts(precision=QK_MIXED, fp32_threshold=1e-1)):
+        for call in (e.fock, e.grad):
+            call(D, o)   # the lists
+            emu.emu_clear_record()
+            call(D, o)
+            print(on, *{line.split()[-1] for line in emu.emu_record().decode().splitlines()})
+"""
+
+
+def test_timed_classes_run_alone(lib):
+    """per-class times are those of one kernel at a time: with timing on, a call works on the caller's stream only"""
+    for line in emulation.run(lib, TIMING).splitlines():
+        on, *streams = line.split()
+        assert (streams == ["0"]) == (on == "True"), line
