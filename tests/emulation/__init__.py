@@ -5,7 +5,7 @@ emulator.cpp): the same kernels and the same host code, with every device
 allocation and a block's dynamic LDS lying against inaccessible pages.  Text
 that only the device compiler takes (inline asm that hides a value from the
 optimiser, the declaration of dynamic LDS, the launch by address) is replaced in
-copies.  Classes with a d shell are left out of the two-electron part, to keep
+copies, and the work lists, which share one allocation on the device, get one each.  Classes with a d shell are left out of the two-electron part, to keep
 the build short: their launchers stop the process.
 """
 from __future__ import annotations
@@ -32,6 +32,8 @@ def _host_text(text: str) -> str:
                   r"\1* const \2 = (\1*)emu::dynamic_lds();", text)
     text = text.replace("(void)hipLaunchKernel(f, dim3(grid), dim3(256), args, lds, s);",
                         "emu_launch_kernel((void (*)(FockArgs, ClassWork))f, dim3(grid), dim3(256), lds, s, aa, ww);")
+    # each work list in an allocation of its own instead of one for all
+    text = text.replace("b.view(reinterpret_cast<T*>(mem.p + off[slot]), count);", "b.release(); (void)b.alloc(count);")
     return "\n".join(line for line in text.split("\n") if not re.match(r"QK_GRAD_FOLD\(.*d", line))
 
 
