@@ -236,20 +236,27 @@ def class_blob(cls):
                              max_stage=max_stage, nout=nout)
 
 
+# the classes that run from their tables (the others run the code of gen_gradw.py)
+TABLE_CLASSES = [(2, 2, 2, 2)]
+
+
 def write(path):
     out = ["// Generated by quick_amd/csrc/gen_grad.py -- do not edit.",
            "// Per-class tables of the nuclear-gradient kernel (layout: GradHdr in qk_internal.h).",
            "#pragma once", "namespace qk {"]
     names = []
     for cls in quartet_classes():
+        if cls not in TABLE_CLASSES:
+            names.append(("nullptr", 0))
+            continue
         t = tag(cls)
         blob, info = class_blob(cls)
         out.append(f"static const int kGradBlob_{t}[{len(blob)}] = {{")
         for i in range(0, len(blob), 24):
             out.append("    " + ", ".join(str(v) for v in blob[i:i + 24]) + ",")
         out.append("};")
-        names.append((t, len(blob)))
-    out.append("static const int* const kGradBlobs[21] = {" + ", ".join(f"kGradBlob_{t}" for t, _ in names) + "};")
+        names.append((f"kGradBlob_{t}", len(blob)))
+    out.append("static const int* const kGradBlobs[21] = {" + ", ".join(t for t, _ in names) + "};")
     out.append("static const int kGradBlobLen[21] = {" + ", ".join(str(n) for _, n in names) + "};")
     out.append("}  // namespace qk")
     new = "\n".join(out) + "\n"

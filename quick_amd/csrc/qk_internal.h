@@ -322,11 +322,10 @@ struct FockArgs {
     unsigned long long* X;    // fixed-point accumulator: xcopies n x n copies
     unsigned long long* counters;  // [0] surviving quartets, [1] primitive quartets
     // Coulomb contributions per significant pair: element e of pair k's block
-    // (e over its NA x NB functions) at J[jofs[k] + e * pstride[k]], so that the
+    // (e over its NA x NB functions) at J[jofs + e * pstride[k]] (jofs: PairRec), so that the
     // lanes of a wavefront, which hold consecutive ket pairs of one group, add
     // to consecutive addresses; jpair_scatter adds J into X after the classes
     unsigned long long* J;
-    const int* jofs;
     int xcopies;              // copies of the accumulator (1 .. kXCopies)
     int n;
     int nshell;

@@ -97,21 +97,11 @@ __constant__ const double kBoysFit[kBoysFitRegions * kBoysFitTerms] = {
     0, 0, 0, 0, 0, 0, 0, 0, 0, 1.9623264149430e-01, -4.9695241464490e-01, -6.0156581186481e-05,
     0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
 
-// 1/x for the positive exponent sums of a primitive quartet: the hardware
-// reciprocal refined by two Newton-Raphson steps, r <- r + r (1 - x r), each of
-// which squares the relative error, so the result is within an ulp or two of
-// 1/x (the IEEE division sequence costs twice the instructions).  FP32: the
-// hardware reciprocal (the FP32 path's error budget is 1e-6).
-__device__ __forceinline__ double recip(double x) {
-    double r = __builtin_amdgcn_rcp(x);
-    r = fma(r, fma(-x, r, 1.0), r);
-    return fma(r, fma(-x, r, 1.0), r);
-}
-__device__ __forceinline__ float recip(float x) { return __builtin_amdgcn_rcpf(x); }
-
-// 1/sqrt(x) for the same sums: the hardware estimate refined by two Newton
-// steps, y <- y + y (1 - x y^2) / 2 (FP64); the hardware estimate (FP32).  A
-// primitive quartet takes 1/(zeta+eta) as its square (one rounding more).
+// 1/sqrt(x) for the positive exponent sums of a primitive quartet: the hardware
+// estimate refined by two Newton steps, y <- y + y (1 - x y^2) / 2, each of which
+// squares the relative error (FP64); the hardware estimate (FP32, whose error
+// budget is 1e-6).  A primitive quartet takes 1/(zeta+eta) as its square (one
+// rounding more).
 __device__ __forceinline__ double rsqrt_nr(double x) {
     double y = __builtin_amdgcn_rsq(x);
     y = fma(y * 0.5, fma(-x * y, y, 1.0), y);
@@ -748,8 +738,6 @@ template <typename R>
 __device__ __forceinline__ const R* grad_density(const GradArgs& a) {
     if constexpr (sizeof(R) == 8) return a.Dp; else return a.Dpf;
 }
-__device__ __forceinline__ double sqrt_r(double x) { return sqrt(x); }
-__device__ __forceinline__ float sqrt_r(float x) { return sqrtf(x); }
 
 // F_0..F_kMaxGradF(T) in FP32 for the gradient's table-driven kernel: the
 // expansion of boys_f32 at the highest order the table supports for it (read
@@ -759,11 +747,6 @@ constexpr int kMaxGradF = 10;
 static_assert(kMaxGradF + 4 < kBoysTabM, "Boys table too narrow for the gradient");
 __device__ __forceinline__ void boys_f32_all(float T, const float* tab, float* F) {
     boys_f32<kMaxGradF, kBoysTabM>(T, tab + kMaxGradF, F);
-}
-
-__device__ __forceinline__ void fx_add_f(unsigned long long* X, long long idx, float v) {
-    const long long iv = fx_round_f(v);
-    if (iv != 0) atomicAdd(X + idx, (unsigned long long)iv);
 }
 
 template <int LA, int LB, int LC, int LD>
