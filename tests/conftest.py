@@ -26,3 +26,11 @@ def golden():
         return cache[name]
 
     return get
+
+
+@pytest.fixture(scope="session")
+def emulated_lib(tmp_path_factory):
+    """the device code built for the CPU (tests/emulation)"""
+    from tests import emulation
+
+    return emulation.build(tmp_path_factory.mktemp("emulation"))

@@ -23,7 +23,6 @@ import numpy as np
 HERE = Path(__file__).resolve().parent
 ROOT = HERE.parents[1]
 CSRC = ROOT / "quick_amd" / "csrc"
-SP = ("ssss", "psss", "psps", "ppss", "ppps", "pppp")
 
 
 def _host_text(text: str) -> str:
@@ -34,7 +33,7 @@ def _host_text(text: str) -> str:
                         "emu_launch_kernel((void (*)(FockArgs, ClassWork))f, dim3(grid), dim3(256), lds, s, aa, ww);")
     # each work list in an allocation of its own instead of one for all
     text = text.replace("b.view(reinterpret_cast<T*>(mem.p + off[slot]), count);", "b.release(); (void)b.alloc(count);")
-    return "\n".join(line for line in text.split("\n") if not re.match(r"QK_GRAD_FOLD\(.*d", line))
+    return text
 
 
 def build(out: Path, jobs: int = 8) -> Path:
@@ -46,15 +45,15 @@ def build(out: Path, jobs: int = 8) -> Path:
     for f in list(CSRC.glob("*.hip")) + list(CSRC.glob("*.h")) + list(CSRC.glob("*.cpp")):
         (src / f.name).write_text(_host_text(f.read_text()))
     for code, args in (
-            ("import gen_eri, sys; gen_eri.main(sys.argv[1]); gen_eri.write_units(sys.argv[2])", ("eri_generated.inc", "gen")),
-            ("import gen_grad, sys; gen_grad.write(sys.argv[1])", ("grad_tables.inc",)),
-            ("import gen_gradw as g, sys; g.FOLD_CLASSES = {c: f for c, f in g.FOLD_CLASSES.items() if max(c) < 2}; "
-             "g.write(sys.argv[1]); g.write_units(sys.argv[2])", ("grad_fold.inc", "gen"))):
+            ("import gen_eri as g, sys; g.main(sys.argv[1]); g.write_units(sys.argv[2]); g.write_team(sys.argv[3])",
+             ("eri_generated.inc", "gen", "team_tables.inc")),
+            ("import gen_grad as g, sys; g.write(sys.argv[1])", ("grad_tables.inc",)),
+            ("import gen_gradw as g, sys; g.write(sys.argv[1]); g.write_units(sys.argv[2])", ("grad_fold.inc", "gen"))):
         subprocess.run([sys.executable, "-c", code, *(str(src / a) for a in args)], check=True,
                        env={**os.environ, "PYTHONPATH": str(CSRC)}, stdout=subprocess.DEVNULL)
     units = [src / n for n in ("qk_fock.hip", "qk_lists.hip", "qk_oneint.hip", "qk_grad.hip", "qk_host.cpp")]
-    units += [gen / f"{k}_{t}.hip" for k in ("fock", "grad") for t in SP]
-    units.append(HERE / "emulator.cpp")
+    units += [HERE / "emulator.cpp"] + list(gen.glob("*.hip"))
+    units.sort(key=lambda u: -u.stat().st_size)   # the longest compilations first
 
     def compile_(u: Path) -> Path:
         obj = out / (u.stem + ".o")
@@ -89,7 +88,7 @@ def run(lib: Path, code: str, low: bool = False, timeout: int = 600) -> str:
     pre = ("import faulthandler, sys; faulthandler.enable(); sys.modules['torch'] = None\n"
            "import ctypes as C, numpy as np\nfrom quick_amd.fock import *\nfrom quick_amd.fock import _ptr\n"
            f"emu = C.CDLL({str(lib)!r}); emu.emu_record.restype = C.c_char_p; emu.emu_alloc_low({int(low)})\n")
-    p = subprocess.run([sys.executable, "-c", pre + code], cwd=ROOT, env=env, capture_output=True, text=True,
+    p = subprocess.run([sys.executable, "-"], input=pre + code, cwd=ROOT, env=env, capture_output=True, text=True,
                        timeout=timeout)
     assert p.returncode == 0, f"exit {p.returncode}\n{p.stdout[-2000:]}\n{p.stderr[-4000:]}"
     return p.stdout

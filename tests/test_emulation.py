@@ -13,11 +13,6 @@ from quick_amd.geometry import synthetic_density, water_cluster
 ZOF = {"H": 1.0, "O": 8.0}
 
 
-@pytest.fixture(scope="session")
-def lib(tmp_path_factory):
-    return emulation.build(tmp_path_factory.mktemp("emulation"))
-
-
 def with_free_functions(b, k):
     """the basis with k functions in front that belong to no shell"""
     c = copy.copy(b)
@@ -51,9 +46,9 @@ def free_function_errors(k):
 
 @pytest.mark.parametrize("low", [False, True], ids=["high", "low"])
 @pytest.mark.parametrize("k", [1, 6])
-def test_functions_outside_every_shell(lib, k, low):
+def test_functions_outside_every_shell(emulated_lib, k, low):
     """lanes without a shell pair read nothing of the functions that no shell holds; tolerances as on the device"""
-    out = emulation.run(lib, f"from tests.test_emulation import *\nprint(*free_function_errors({k}))", low=low)
+    out = emulation.run(emulated_lib, f"from tests.test_emulation import *\nprint(*free_function_errors({k}))", low=low)
     dS, dH, free, dg = map(float, out.split())
     assert dS <= 1e-12 and dH <= 1e-10 and free == 0.0 and dg <= 1e-10
 
@@ -108,8 +103,8 @@ ODD = ["twice", "other-l", "order", "shared"]
 
 
 @pytest.mark.parametrize("kind", ODD)
-def test_shells_without_each_component_once(lib, kind):
-    out = emulation.run(lib, f"from tests.test_emulation import *\nprint(*odd_shell_errors({kind!r}))")
+def test_shells_without_each_component_once(emulated_lib, kind):
+    out = emulation.run(emulated_lib, f"from tests.test_emulation import *\nprint(*odd_shell_errors({kind!r}))")
     dS, dH, dg = map(float, out.split())
     assert dS <= 1e-12 and dH <= 1e-10 and dg <= 1e-10
 
@@ -168,10 +163,10 @@ for name, call in calls.items():
 
 
 @pytest.mark.parametrize("kw", ["dict()", "dict(precision=QK_MIXED, fp32_threshold=1e-1)"], ids=["fp64", "mixed"])
-def test_streams_are_joined_after_any_error(lib, kw):
+def test_streams_are_joined_after_any_error(emulated_lib, kw):
     """every launch check of a call fails once: the call reports it, the streams it forked are ordered before what
     follows on the caller's, and the next call gives the same result as before"""
-    out = dict(line.split() for line in emulation.run(lib, JOIN.replace("KW", kw)).splitlines())
+    out = dict(line.split() for line in emulation.run(emulated_lib, JOIN.replace("KW", kw)).splitlines())
     assert int(out["fock"]) >= 8 and int(out["grad"]) >= 8 and int(out["oneint"]) and int(out["oneint_grad"]), out
 
 
@@ -198,15 +193,15 @@ print(emu.emu_record().decode())
 """
 
 
-def test_grids_of_spilling_kernels(lib):
+def test_grids_of_spilling_kernels(emulated_lib):
     """the grids that the launchers really use, were every kernel that can spill to take 1 MiB per lane (the budget
     then holds one block of 256 threads): no launch may back more than the budget"""
     names = ["oneint_grad_kernel", "grad_light_kernel", "fock_kernel"]
-    nm = emulation.symbols(lib)
+    nm = emulation.symbols(emulated_lib)
     spill = [n for n in nm if any(k in n for k in names) and "launch" not in n]
     assert len(spill) >= 6 + 12 + 12
     seen = set()
-    for line in emulation.run(lib, SCRATCH.replace("NAMES", repr(spill))).split("\n"):
+    for line in emulation.run(emulated_lib, SCRATCH.replace("NAMES", repr(spill))).split("\n"):
         if line:
             name, grid, block, _, _ = line.split()
             if name in spill:
@@ -228,9 +223,9 @@ def far_charge_errors():
     return np.abs(e.oneint()[1] - O.hcore(b)[1]).max(), np.abs(e.oneint_grad(D, W) - O.oneint_grad(b, D, W)).max()
 
 
-def test_charge_very_far_away(lib):
+def test_charge_very_far_away(emulated_lib):
     """Boys arguments of 1e50, beyond what exp's reduction can carry: finite, as the oracle has them"""
-    out = emulation.run(lib, "from tests.test_emulation import *\nprint(*far_charge_errors())")
+    out = emulation.run(emulated_lib, "from tests.test_emulation import *\nprint(*far_charge_errors())")
     assert all(float(v) <= 1e-10 for v in out.split()), out
 
 
@@ -259,8 +254,8 @@ for on in (False, True):
 """
 
 
-def test_timed_classes_run_alone(lib):
+def test_timed_classes_run_alone(emulated_lib):
     """per-class times are those of one kernel at a time: with timing on, a call works on the caller's stream only"""
-    for line in emulation.run(lib, TIMING).splitlines():
+    for line in emulation.run(emulated_lib, TIMING).splitlines():
         on, *streams = line.split()
         assert (streams == ["0"]) == (on == "True"), line

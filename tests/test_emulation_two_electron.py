@@ -1,4 +1,4 @@
-"""The Fock and gradient kernels of the s and p classes on the CPU, where an access
+"""The Fock and gradient kernels on the CPU, where an access
 outside an allocation ends the process (tests/emulation): work lists, compacted
 steps, pair records, prefetched kets and primitives, shared tiles and runs.
 
@@ -6,12 +6,12 @@ The systems pass through every form: one tile with 64 wavefronts on it (one
 atom), several blocks per run, lists long enough to be compacted, with steps that
 hold nothing (a cluster with the density of one molecule), exchange rows beyond LDS
 (many functions), a gradient beyond LDS (many nuclei), pairs of 1 to 36
-primitives.  Results against the oracle as on the device: FP64 1e-10, mixed 1e-6.
+primitives; every class with d functions on one molecule, the others without.
+Results against the oracle as on the device: FP64 1e-10, mixed 1e-6.
 """
 import pytest
 
 from tests import emulation
-from tests.test_emulation import lib  # noqa: F401
 
 CODE = """
 import sys
@@ -27,7 +27,9 @@ if kind[0] == "H":
 else:
     sym, xyz = water_cluster(*kind[1], seed=5)
     xyz = np.asarray(xyz, float)
-b = without_d(build_basis(list(sym), xyz))
+b = build_basis(list(sym), xyz)
+if kind[0] != "d":
+    b = without_d(b)
 D = synthetic_density(b.xyz, b.katom, b.ksumtype, b.nbasis, 3)
 if kind[0] == "masked":   # the density of one molecule: most kets fail the screen
     D[b.nbasis // 6:] = D[:, b.nbasis // 6:] = 0.0
@@ -58,14 +60,14 @@ TAU = 1e-11
 CASES = {"1-atom": (("H", 1), TAU, 1.0), "2-atoms": (("H", 2), 1e-6, 0.0), "5-atoms": (("H", 5), TAU, 0.2),
          "water": (("water", (1, 1, 1)), TAU, 1.0), "3-waters": (("water", (3, 1, 1)), TAU, 1.0),
          "6-waters": (("water", (3, 2, 1)), TAU, 1.0), "masked": (("masked", (3, 2, 1)), TAU, 1.0),
-         "functions": (("free", (1, 1, 1), 3300), TAU, 1.0), "nuclei": (("nuclei", (1, 1, 1)), TAU, 1.0)}
+         "d": (("d", (1, 1, 1)), TAU, 1.0), "functions": (("free", (1, 1, 1), 3300), TAU, 1.0), "nuclei": (("nuclei", (1, 1, 1)), TAU, 1.0)}
 
 
 @pytest.mark.parametrize("name,low", [(n, low) for n in CASES for low in (False, True)
-                                      if not (low and n in ("6-waters", "functions", "nuclei"))],
+                                      if not (low and n in ("3-waters", "6-waters", "functions", "nuclei"))],
                          ids=lambda v: v if isinstance(v, str) else ("low" if v else "high"))
-def test_two_electron_kernels_stay_in_bounds(lib, name, low):  # noqa: F811
-    record = emulation.run(lib, CODE.replace("ARGS", repr(CASES[name])), low=low)
+def test_two_electron_kernels_stay_in_bounds(emulated_lib, name, low):
+    record = emulation.run(emulated_lib, CODE.replace("ARGS", repr(CASES[name])), low=low)
     launched = [line.split() for line in record.splitlines() if line]
     modes = {(n.split("ELi")[-1][0], "f32" in n) for n, *_ in launched if "fock_kernel" in n}
     compacted = any("compact_kernel" in n for n, *_ in launched)
