@@ -58,7 +58,7 @@ print(emu.emu_record().decode())
 
 TAU = 1e-11
 CASES = {"1-atom": (("H", 1), TAU, 1.0), "2-atoms": (("H", 2), 1e-6, 0.0), "5-atoms": (("H", 5), TAU, 0.2),
-         "water": (("water", (1, 1, 1)), TAU, 1.0), "3-waters": (("water", (3, 1, 1)), TAU, 1.0),
+         "3-waters": (("water", (3, 1, 1)), TAU, 1.0),
          "6-waters": (("water", (3, 2, 1)), TAU, 1.0), "masked": (("masked", (3, 2, 1)), TAU, 1.0),
          "d": (("d", (1, 1, 1)), TAU, 1.0), "functions": (("free", (1, 1, 1), 3300), TAU, 1.0), "nuclei": (("nuclei", (1, 1, 1)), TAU, 1.0)}
 
