@@ -164,8 +164,8 @@ int qk_fock_host(qk_ctx* c, const double* D, double* F, const qk_opts* o);
  * shell.f90:1863-2535, hrr.f90:862-1014).  opts->tau is the gradient cutoff
  * (quick_method%gradCutoff).  With opts->precision QK_MIXED, quartets whose
  * Schwarz bound Y_ij*Y_kl lies below opts->fp32_threshold are differentiated
- * in FP32 (accumulated in FP64 fixed point).  Runs on `stream`, with a second
- * stream of the context forked from it and joined back, as qk_fock_device. */
+ * in FP32 (accumulated in FP64 fixed point).  Runs on `stream` and on three
+ * streams of the context forked from it and joined back, as qk_fock_device. */
 int qk_grad_device(qk_ctx* c, const double* dD, double* dgrad, const qk_opts* o, void* stream);
 int qk_grad_host(qk_ctx* c, const double* D, double* grad, const qk_opts* o);
 
@@ -173,11 +173,15 @@ int qk_grad_host(qk_ctx* c, const double* D, double* grad, const qk_opts* o);
  * integral.f90:1633-1925; the one-electron part of hfgrad, gradient.f90:40-250).
  * qk_set_charges: the nuclear charges (natom, host), kept with the system.
  * qk_oneint_device: dS <- S, dH <- H_core = T + V (n x n device arrays; either
- *   may be NULL); asynchronous on `stream`.
+ *   may be NULL); asynchronous on `stream` and three streams of the context
+ *   forked from it and joined back.  A function that no shell holds has zero rows;
+ *   a shell whose KLMN does not name each Cartesian component of its angular
+ *   momentum once is evaluated function by function.
  * qk_nuclear_repulsion: E <- sum_{A<B} Z_A Z_B / R_AB (host).
  * qk_oneint_grad_device: dgrad (3 natom, device) += nuclear repulsion gradient
  *   + sum D dH/dR - sum W dS/dR for the density dD and the energy-weighted
- *   density dW = 2 sum_occ e_i c_i c_i^T (n x n device arrays); asynchronous.
+ *   density dW = 2 sum_occ e_i c_i c_i^T (n x n device arrays); asynchronous, on the
+ *   same streams.
  * qk_oneint_host / qk_oneint_grad_host: the same on host arrays, synchronous. */
 int qk_set_charges(qk_ctx* c, const double* charges);
 int qk_oneint_device(qk_ctx* c, double* dS, double* dH, void* stream);

@@ -682,7 +682,7 @@ using ListSumsFn = std::function<int(const std::vector<long long>&, std::vector<
 
 // Wavefronts per tile, log2, of a class with `tiles` tiles whose quartets hold at
 // most `prims` primitive quartets.  A lane works through its quartet's primitives
-// one after another (up to 1,296 of them, 0.4 us each in FP64), so where a class
+// one after another (up to 4,096 of them, 1,296 in 6-31G**; 0.4 us each in FP64), so where a class
 // has too few tiles to fill the GPU the longest chain is the kernel's time; there
 // each tile's primitives are split over wavefronts that would be idle (one water:
 // Fock build 2.39 -> 0.54 ms, gradient 2.28 -> 0.76 ms).  1,024 wavefronts (one

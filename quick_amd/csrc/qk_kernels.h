@@ -109,8 +109,8 @@ __device__ __forceinline__ double rsqrt_nr(double x) {
 }
 __device__ __forceinline__ float rsqrt_nr(float x) { return __builtin_amdgcn_rsqf(x); }
 
-// exp(-X), X >= 0: X = -k ln2 - r with |r| <= ln2 / 2 (ln2 in two parts, the
-// high one exact times k below 2^21), exp(r) by the degree-11 interpolant at the
+// exp(-X), X >= 0: X = -k ln2 - r with |r| <= ln2 / 2 (ln2 in the two parts of
+// fdlibm's e_exp.c, by Sun Microsystems: the high one exact times k below 2^21), exp(r) by the degree-11 interpolant at the
 // Chebyshev nodes of the interval (largest relative error 1.7e-17), scaled by 2^k
 // (to zero beyond the range; X up to 1e44, where r's error would overflow p)
 __device__ __forceinline__ double exp_neg(double X) {
@@ -756,7 +756,8 @@ struct OccupancyF {
     // at 800 functions (more functions: fewer): asking for four wavefronts per
     // SIMD only made such kernels spill (measured: ppps 1.34 -> 1.27 ms, dsds
     // 0.44 -> 0.42 ms with three); (dp|pp), with 144 accumulators, spills at two
-    // (1.10 -> 0.97 ms with one)
+    // (1.10 -> 0.97 ms with one).  The d-d bras leave run mode above 682 functions,
+    // where no rows bound them; (dd|ss) keeps three there and spills 47 registers
     static constexpr int rows = ncart(LA) + ncart(LB);
     static constexpr int value = nacc <= 36 ? (rows >= 6 ? 3 : 4) : (nacc < 144 ? 2 : 1);
 };

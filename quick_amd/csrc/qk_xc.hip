@@ -315,7 +315,8 @@ struct XcBatch {
 // function every function of the 64 cost as much as the longest contraction among
 // them), once for components that share them.  Sixteen functions at a time go
 // through LDS to be written as rows of 128 bytes.  Bound by its
-// stores: (H2O)64 on SG-1 (11,361 batches, 18 GB) 6.5 -> 3.6 ms, 5.0 TB/s.
+// stores: (H2O)64 on the 75 x 302 grid (11,361 batches, 18 GB) 6.5 -> 3.6 ms,
+// 5.0 TB/s.
 constexpr int kXcValCols = 16, kXcValRow = kXcValCols + 2;   // functions per step; LDS row (16-byte aligned)
 __global__ void __launch_bounds__(256) xc_values(const int4* __restrict__ tasks, const XcBatch* __restrict__ bt,
                                                  const double* __restrict__ pts, const int* __restrict__ sig,
