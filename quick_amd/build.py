@@ -34,13 +34,13 @@ HIP_FLAGS = [
 OBJ = HERE / "_build"
 
 
-def _compile(src: Path, verbose: bool) -> Path:
+def _compile(src: Path, verbose: bool, force: bool = False) -> Path:
     obj = OBJ / (src.stem + ".o")
     deps = [src, CSRC / "qk_kernels.h", CSRC / "qk_internal.h", CSRC / "eri_generated.inc",
             CSRC / "qk_team.h", CSRC / "team_tables.inc", CSRC / "grad_tables.inc", CSRC / "grad_fold.inc",
             CSRC / "qk_grad_light.h", CSRC / "qk_xc_deal.h", CSRC / "xc_b3lyp.inc", CSRC / "lebedev.inc",
             HERE.parent / "include" / "quick_mi355x.h", Path(__file__)]
-    if obj.exists() and all(obj.stat().st_mtime >= d.stat().st_mtime for d in deps if d.exists()):
+    if not force and obj.exists() and all(obj.stat().st_mtime >= d.stat().st_mtime for d in deps if d.exists()):
         return obj
     flags = [f for f in HIP_FLAGS if f != "-shared"]
     cmd = ["hipcc", *flags, "-I", str(HERE.parent / "include"), "-c", str(src), "-o", str(obj)]
@@ -50,7 +50,8 @@ def _compile(src: Path, verbose: bool) -> Path:
     return obj
 
 
-def build(verbose: bool = True, jobs: int = 8) -> Path:
+def build(verbose: bool = True, jobs: int = 8, force: bool = False) -> Path:
+    """force: compile every unit, also those whose object is newer than its sources"""
     from concurrent.futures import ThreadPoolExecutor
     OBJ.mkdir(exist_ok=True)
     subprocess.run([sys.executable, str(CSRC / "gen_eri.py"), str(CSRC / "eri_generated.inc"),
@@ -66,7 +67,7 @@ def build(verbose: bool = True, jobs: int = 8) -> Path:
     srcs += [CSRC / "qk_xc.hip", CSRC / "qk_oneint.hip", CSRC / "qk_scf.hip", CSRC / "qk_lists.hip", CSRC / "qk_fock.hip",
              CSRC / "qk_grad.hip", CSRC / "qk_host.cpp"]
     with ThreadPoolExecutor(jobs) as ex:
-        objs = list(ex.map(lambda s: _compile(s, verbose), srcs))
+        objs = list(ex.map(lambda s: _compile(s, verbose, force), srcs))
     tmp = LIB.with_suffix(".so.tmp")
     # rocBLAS and rocSOLVER serve the SCF step (qk_scf.hip)
     cmd = ["hipcc", f"--offload-arch={ARCH}", "-shared", "-fPIC", *map(str, objs), "-o", str(tmp),
